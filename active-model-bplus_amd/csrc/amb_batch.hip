@@ -28,15 +28,16 @@ namespace amb {
 template <typename T>
 struct BatchDesc {
     int64_t off;  // element offset of the realisation in the concatenated buffers
-    int ny, nx, nx4, ntx;
+    int ny, nx, ntx;
     uint32_t key0, key1;
     StepCoef<T> k;
 };
 
-// NOISE is kNoiseNone or kNoisePhilox: members with and without noise run in separate
+// NOISE is kNoiseNone, kNoisePhilox or kNoisePhiloxOdd: members without noise, and with it on
+// columns that do or do not split into fours, run in separate
 // launches, so each kernel holds only its own stage-B windows in registers.
 template <typename T, int TW, int TH, int NT, int NOISE>
-__global__ __launch_bounds__(NT, (min_waves_per_eu<T, TW, TH, NT>())) void batch_step_kernel(const BatchDesc<T>* __restrict__ desc,
+__global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) void batch_step_kernel(const BatchDesc<T>* __restrict__ desc,
                                                               const int2* __restrict__ tiles, const T* in, T* out,
                                                               const long long* step_base, int step_off, double* part)
 {
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(NT, (min_waves_per_eu<T, TW, TH, NT>())) void batch
     const BatchDesc<T>& d = desc[t.x];
     const int ty = t.y / d.ntx, tx = t.y - ty * d.ntx;
     const uint64_t step = (uint64_t)(*step_base) + (uint64_t)step_off;
-    step_tile<T, TW, TH, NT, NOISE>(reinterpret_cast<T*>(smem_raw), in + d.off, out + d.off, d.ny, d.nx, d.nx4,
+    step_tile<T, TW, TH, NT, NOISE>(reinterpret_cast<T*>(smem_raw), in + d.off, out + d.off, d.ny, d.nx,
                                     tx * TW, ty * TH, d.k, d.key0, d.key1, step, nullptr, red);
 }
 
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(NT) void resident_kernel(const BatchDesc<T>* __rest
     for (int k = 0; k < nsteps; ++k) {
         for (int t = 0; t < ntx * nty; ++t) {
             const int ty = t / ntx, tx = t - ty * ntx;
-            step_tile<T, TW, TH, NT, NOISE>(scratch, a, b, d.ny, d.nx, d.nx4, tx * TW, ty * TH, d.k, d.key0, d.key1,
+            step_tile<T, TW, TH, NT, NOISE>(scratch, a, b, d.ny, d.nx, tx * TW, ty * TH, d.k, d.key0, d.key1,
                                             step0 + (uint64_t)k, nullptr, nullptr);
             __syncthreads();  // the next tile's stage 0 overwrites what this one's stage B reads
         }
@@ -179,17 +180,16 @@ static hipError_t launch_resident(int precision, int noise, const void* desc, co
                                   int64_t max_n, const void* in, void* out, const long long* step, int nsteps,
                                   double* part, int64_t part_base, hipStream_t s)
 {
+#define AMB_RESIDENT(T, mode) \
+    launch_resident_t<T, mode>(desc, members, count, max_n, in, out, step, nsteps, part, part_base, s)
     if (precision == AMB_F32)
-        return noise == kNoisePhilox
-                   ? launch_resident_t<float, kNoisePhilox>(desc, members, count, max_n, in, out, step, nsteps, part,
-                                                            part_base, s)
-                   : launch_resident_t<float, kNoiseNone>(desc, members, count, max_n, in, out, step, nsteps, part,
-                                                          part_base, s);
-    return noise == kNoisePhilox
-               ? launch_resident_t<double, kNoisePhilox>(desc, members, count, max_n, in, out, step, nsteps, part,
-                                                         part_base, s)
-               : launch_resident_t<double, kNoiseNone>(desc, members, count, max_n, in, out, step, nsteps, part,
-                                                       part_base, s);
+        return noise == kNoiseNone     ? AMB_RESIDENT(float, kNoiseNone)
+               : noise == kNoisePhilox ? AMB_RESIDENT(float, kNoisePhilox)
+                                       : AMB_RESIDENT(float, kNoisePhiloxOdd);
+    return noise == kNoiseNone     ? AMB_RESIDENT(double, kNoiseNone)
+           : noise == kNoisePhilox ? AMB_RESIDENT(double, kNoisePhilox)
+                                   : AMB_RESIDENT(double, kNoisePhiloxOdd);
+#undef AMB_RESIDENT
 }
 
 template <typename T>
@@ -200,6 +200,9 @@ static hipError_t raise_resident_lds_t()
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, kNoisePhilox>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, kNoisePhiloxOdd>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
     return e;
 }
@@ -213,6 +216,9 @@ static hipError_t raise_batch_lds()
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void*)batch_step_kernel<T, TW, TH, NT, kNoisePhilox>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void*)batch_step_kernel<T, TW, TH, NT, kNoisePhiloxOdd>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
     return e;
 }
@@ -236,12 +242,13 @@ static hipError_t launch_batch_one(int noise, const void* desc, const int2* tile
 {
     using L = Lds<T, TW, TH, NT>;
     const auto* d = static_cast<const BatchDesc<T>*>(desc);
-    if (noise == kNoisePhilox)
-        hipLaunchKernelGGL((batch_step_kernel<T, TW, TH, NT, kNoisePhilox>), dim3(ntiles), dim3(NT), L::bytes, s, d,
-                           tiles, static_cast<const T*>(in), static_cast<T*>(out), step, step_off, part);
-    else
-        hipLaunchKernelGGL((batch_step_kernel<T, TW, TH, NT, kNoiseNone>), dim3(ntiles), dim3(NT), L::bytes, s, d,
-                           tiles, static_cast<const T*>(in), static_cast<T*>(out), step, step_off, part);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(ntiles), dim3(NT), L::bytes, s, d, tiles, static_cast<const T*>(in),
+                           static_cast<T*>(out), step, step_off, part);
+    };
+    if (noise == kNoisePhilox) launch(batch_step_kernel<T, TW, TH, NT, kNoisePhilox>);
+    else if (noise == kNoisePhiloxOdd) launch(batch_step_kernel<T, TW, TH, NT, kNoisePhiloxOdd>);
+    else launch(batch_step_kernel<T, TW, TH, NT, kNoiseNone>);
     return hipGetLastError();
 }
 
@@ -250,8 +257,7 @@ static hipError_t launch_batch_one(int noise, const void* desc, const int2* tile
 #define AMB_BCASE_F64(i, tw, th, nt) \
     case i: return launch_batch_one<double, tw, th, nt>(noise, desc, tiles, ntiles, in, out, step, step_off, part, s);
 
-// One step of the members listed in `tiles` (noise: kNoiseNone or kNoisePhilox, the same
-// for all of them).  part (nullable): the per-tile partials of the fused finite check,
+// One step of the members listed in `tiles` (noise: the same mode for all of them).  part (nullable): the per-tile partials of the fused finite check,
 // one entry per entry of `tiles` (padding entries write zeros).
 static hipError_t launch_batch(int precision, int tile, int noise, const void* desc, const int2* tiles, int ntiles,
                                const void* in, void* out, const long long* step, int step_off, double* part,
@@ -279,7 +285,7 @@ constexpr int kBatchGraphSteps = 32;
 
 struct Group {
     int tile = 0;
-    int noise = 0;  // kNoiseNone or kNoisePhilox
+    int noise = 0;  // kNoiseNone, kNoisePhilox or kNoisePhiloxOdd
     std::vector<int> members;
     int2* d_tiles = nullptr;
     int ntiles = 0;
@@ -310,8 +316,8 @@ struct amb_batch {
     int64_t last_bad = 0;
     // members kept in LDS by the resident kernel (when enabled and they fit)
     bool resident_on = true;
-    std::vector<int> resident;      // noiseless members first, then the noisy ones
-    int64_t resident_quiet = 0;     // how many of them are noiseless
+    std::vector<int> resident;         // grouped by noise mode:
+    int64_t resident_of[4] = {};       // how many of each (kNoiseNone, kNoisePhilox, -, kNoisePhiloxOdd)
     int* d_resident = nullptr;
     int64_t resident_max_n = 0;
     hipStream_t side = nullptr;     // capture branch of the resident launch, beside the tiled steps
@@ -393,21 +399,23 @@ int rebuild_groups(amb_batch* b)
     drop_graphs(b);
     free_groups(b);
     std::map<std::pair<int, int>, std::vector<int>> by_tile;  // (tile, noise mode) -> members
-    std::vector<int> quiet, noisy;
+    std::vector<int> kept[4];  // resident members per noise mode
     b->resident_max_n = 0;
     for (size_t r = 0; r < b->desc.size(); ++r) {
         const amb_realisation& m = b->desc[r];
-        const int noise = m.model.T > 0.0 ? kNoisePhilox : kNoiseNone;
+        const int noise = m.model.T > 0.0 ? philox_mode(m.nx) : kNoiseNone;
         if (b->resident_on && fits_resident(b->precision, m.ny, m.nx)) {
-            (noise == kNoisePhilox ? noisy : quiet).push_back((int)r);
+            kept[noise].push_back((int)r);
             b->resident_max_n = std::max(b->resident_max_n, m.ny * m.nx);
         } else {
             by_tile[{b->tile_of[r], noise}].push_back((int)r);
         }
     }
-    b->resident = quiet;
-    b->resident.insert(b->resident.end(), noisy.begin(), noisy.end());
-    b->resident_quiet = (int64_t)quiet.size();
+    b->resident.clear();
+    for (int m = 0; m < 4; ++m) {
+        b->resident.insert(b->resident.end(), kept[m].begin(), kept[m].end());
+        b->resident_of[m] = (int64_t)kept[m].size();
+    }
     if (b->d_resident) (void)hipFree(b->d_resident);
     b->d_resident = nullptr;
     if (!b->resident.empty()) {
@@ -455,7 +463,6 @@ std::vector<BatchDesc<T>> make_descs(const amb_batch* b)
         d[r].off = b->off[r];
         d[r].ny = (int)s.ny;
         d[r].nx = (int)s.nx;
-        d[r].nx4 = (s.nx % 4) == 0;
         d[r].ntx = 0;  // set per launch group below
         d[r].key0 = (uint32_t)s.seed;
         d[r].key1 = (uint32_t)(s.seed >> 32);
@@ -499,16 +506,15 @@ hipError_t launch_groups(amb_batch* b, int parity_in, const long long* step, int
 hipError_t launch_resident_members(amb_batch* b, int parity_in, int nsteps, hipStream_t s)
 {
     if (b->resident.empty() || nsteps <= 0) return hipSuccess;
-    const int64_t nq = b->resident_quiet, nn = (int64_t)b->resident.size() - nq;
     hipError_t e = hipSuccess;
-    if (nq > 0)
-        e = launch_resident(b->precision, kNoiseNone, b->d_desc, b->d_resident, (int)nq, b->resident_max_n,
-                            b->buf[parity_in & 1], b->buf[(parity_in + nsteps) & 1], b->d_step, nsteps,
-                            b->d_tile_part, b->ntiles_total, s);
-    if (e == hipSuccess && nn > 0)
-        e = launch_resident(b->precision, kNoisePhilox, b->d_desc, b->d_resident + nq, (int)nn, b->resident_max_n,
-                            b->buf[parity_in & 1], b->buf[(parity_in + nsteps) & 1], b->d_step, nsteps,
-                            b->d_tile_part, b->ntiles_total + nq, s);
+    int64_t first = 0;
+    for (int m = 0; m < 4 && e == hipSuccess; ++m) {
+        if (b->resident_of[m] > 0)
+            e = launch_resident(b->precision, m, b->d_desc, b->d_resident + first, (int)b->resident_of[m],
+                                b->resident_max_n, b->buf[parity_in & 1], b->buf[(parity_in + nsteps) & 1], b->d_step,
+                                nsteps, b->d_tile_part, b->ntiles_total + first, s);
+        first += b->resident_of[m];
+    }
     return e;
 }
 

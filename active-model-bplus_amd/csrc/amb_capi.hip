@@ -255,7 +255,6 @@ StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int nois
     a.out = static_cast<T*>(h->buf[(parity_in + 1) & 1]);
     a.ny = (int)h->ny;
     a.nx = (int)h->nx;
-    a.nx4 = (h->nx % 4) == 0;
     a.ntx = grid_tiles(h->nx, ts.tw);
     a.nty = grid_tiles(h->ny, ts.th);
     a.xcd_chunk = xcd_chunk(a.ntx * a.nty);

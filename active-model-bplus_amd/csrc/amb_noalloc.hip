@@ -94,7 +94,6 @@ int run_noalloc(T* field, T* work, int64_t ny, int64_t nx, const amb_stencil& st
     StepArgs<T> a{};
     a.ny = (int)ny;
     a.nx = (int)nx;
-    a.nx4 = (nx % 4) == 0;
     a.ntx = grid_tiles(nx, ts.tw);
     a.nty = grid_tiles(ny, ts.th);
     a.xcd_chunk = xcd_chunk(a.ntx * a.nty);

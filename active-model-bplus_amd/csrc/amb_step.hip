@@ -30,16 +30,17 @@ namespace amb {
 // ---- single-field kernel ----------------------------------------------------------
 
 template <typename T, int TW, int TH, int NT, int NOISE>
-__global__ __launch_bounds__(NT, (min_waves_per_eu<T, TW, TH, NT>())) void step_kernel(const StepArgs<T> p)
+__global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) void step_kernel(const StepArgs<T> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // Tile index; with xcd_chunk the round-robin XCD dispatch gets contiguous tiles.
     int t = blockIdx.x;
     if (p.xcd_chunk > 0) t = (t & 7) * p.xcd_chunk + (t >> 3);
     const int ty = t / p.ntx, tx = t - ty * p.ntx;
-    const uint64_t step = NOISE == kNoisePhilox ? (uint64_t)(*p.step_base) + (uint64_t)p.step_off : 0;
-    step_tile<T, TW, TH, NT, NOISE>(reinterpret_cast<T*>(smem_raw), p.in, p.out, p.ny, p.nx, p.nx4, tx * TW, ty * TH,
-                                    p.k, p.key0, p.key1, step, p.noise, p.part ? p.part + 2 * (size_t)t : nullptr);
+    constexpr bool kPhilox = NOISE == kNoisePhilox || NOISE == kNoisePhiloxOdd;
+    const uint64_t step = kPhilox ? (uint64_t)(*p.step_base) + (uint64_t)p.step_off : 0;
+    step_tile<T, TW, TH, NT, NOISE>(reinterpret_cast<T*>(smem_raw), p.in, p.out, p.ny, p.nx, tx * TW, ty * TH, p.k,
+                                    p.key0, p.key1, step, p.noise, p.part ? p.part + 2 * (size_t)t : nullptr);
 }
 
 // ---- tile table ---------------------------------------------------------------
@@ -72,9 +73,10 @@ static hipError_t launch_one(const StepArgs<T>& a, hipStream_t s)
 template <typename T, int TW, int TH, int NT>
 static hipError_t launch_noise(const StepArgs<T>& a, int noise, hipStream_t s)
 {
-    switch (noise) {
+    switch (noise == kNoisePhilox ? philox_mode(a.nx) : noise) {
     case kNoiseNone: return launch_one<T, TW, TH, NT, kNoiseNone>(a, s);
     case kNoisePhilox: return launch_one<T, TW, TH, NT, kNoisePhilox>(a, s);
+    case kNoisePhiloxOdd: return launch_one<T, TW, TH, NT, kNoisePhiloxOdd>(a, s);
     default: return launch_one<T, TW, TH, NT, kNoiseBuffer>(a, s);
     }
 }
@@ -141,6 +143,9 @@ static hipError_t raise_lds_limit()
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void*)step_kernel<T, TW, TH, NT, kNoisePhilox>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)step_kernel<T, TW, TH, NT, kNoisePhiloxOdd>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void*)step_kernel<T, TW, TH, NT, kNoiseBuffer>,

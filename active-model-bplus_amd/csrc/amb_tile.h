@@ -61,6 +61,15 @@ constexpr int min_waves_per_eu()
     return w < 1 ? 1 : w > 8 ? 8 : w;
 }
 
+// The same for a step kernel's noise mode: aligned FP64 noisy tiles of 512 threads are held to
+// 102 VGPRs (91 used), where the compiler's schedule is faster than the one it takes with 128
+// (109 used): 512^2 8.82 -> 8.65 us a step, 1024^2 20.3 -> 19.9 us.
+template <typename T, int TW, int TH, int NT, int NOISE>
+constexpr int step_waves_per_eu()
+{
+    return min_waves_per_eu<T, TW, TH, NT>() + (sizeof(T) == 8 && NT == 512 && NOISE == kNoisePhilox ? 1 : 0);
+}
+
 // ---- Box-Muller ---------------------------------------------------------------
 
 __device__ __forceinline__ void box_muller(uint32_t wa, uint32_t wb, float& z0, float& z1)
@@ -184,7 +193,7 @@ __device__ __forceinline__ void lds_store4(double* p, const double v[4])
 
 template <typename T, int TW, int TH, int NT, int NOISE>
 __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in, T* __restrict__ out, const int ny,
-                                          const int nx, const int nx4, const int x0, const int y0,
+                                          const int nx, const int x0, const int y0,
                                           const StepCoef<T>& K, const uint32_t key0, const uint32_t key1,
                                           const uint64_t step, const double* noise, double* const red_out)
 {
@@ -213,7 +222,8 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
     // 4096^2 against no priorities: FP32 noisy 107.4 -> 104.6 us, noiseless 90.7 -> 87.2 us,
     // FP64 noisy 266.0 -> 252.2 us; 1024^2 FP32 noisy 11.05 -> 10.2 us.  (Priorities change
     // only the order in which a SIMD picks ready waves, not what any wave computes.)
-    constexpr bool kNoisyKernel = NOISE == kNoisePhilox || NOISE == kNoiseBuffer;
+    constexpr bool kPhilox = NOISE == kNoisePhilox || NOISE == kNoisePhiloxOdd;
+    constexpr bool noisy = kPhilox || NOISE == kNoiseBuffer;
     __builtin_amdgcn_s_setprio(1);
     // ---- stage 0: phi with a 9-site halo -> LDS.  Each thread owns fixed region
     // columns and walks rows; loads are independent and unrolled.
@@ -242,7 +252,7 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
         }
     }
     __syncthreads();
-    if constexpr (!kNoisyKernel) __builtin_amdgcn_s_setprio(0);
+    if constexpr (!noisy) __builtin_amdgcn_s_setprio(0);
 
     T phi_c[R];
 #pragma unroll
@@ -341,7 +351,7 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
         }
     }
     __syncthreads();
-    if constexpr (kNoisyKernel) __builtin_amdgcn_s_setprio(0);
+    if constexpr (noisy) __builtin_amdgcn_s_setprio(0);
 
     // ---- stage N (noisy steps): the currents through D8, J = amp xi - (1/dx) D8 mu_p,
     // each formed as soon as its normal is drawn and written over the phi buffer: J_x on
@@ -349,8 +359,6 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
     // their D8 divergence, the passive and the noise term in one.  Every path below
     // evaluates J in the same order (amp xi, then j = 1..4), so all give the same bits.
     // FP32 noisy steps also form the active current C here (active_current below).
-    bool noisy = NOISE == kNoisePhilox || NOISE == kNoiseBuffer;
-    if constexpr (NOISE == kNoiseRuntime) noisy = K.amp != T(0);
     T* const s_jx = sm;  // aliases s_phi after stage A
     T* const s_jy = sm + L::XW * L::XH;
     auto mup = [&](int r, int col) -> const T* { return s_mup + (r + 8) * L::MW + col + 8; };
@@ -411,8 +419,8 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
     // slower (242 -> 250.5 us), so FP64 and the smaller FP32 fields keep the 5x5 stencil.
     // The choice depends on the precision and the field's size only, so every tile shape
     // and the batched kernels give the same bits.
-    constexpr bool kActiveCurrent = sizeof(T) == 4 && NOISE != kNoiseNone;
-    const bool active = kActiveCurrent && noisy && (long long)ny * nx >= kActiveCurrentSites;
+    constexpr bool kActiveCurrent = sizeof(T) == 4 && noisy;
+    const bool active = kActiveCurrent && (long long)ny * nx >= kActiveCurrentSites;
     auto active_current = [&]() {
         if constexpr (kActiveCurrent) {
             constexpr int CW = TW + 2, CH = TH + 2, CSEG = 4, NSEG = (CH + CSEG - 1) / CSEG;
@@ -467,13 +475,13 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
             }
         }
     };
-    if (NOISE == kNoisePhilox || (NOISE == kNoiseRuntime && noisy)) {
+    if constexpr (kPhilox) {
         // Philox items: xi_x groups (rows [0,TH), tile-relative column groups [-1, TW/4])
         // and xi_y groups (rows [-4,TH+4), groups [0, TW/4)), four normals per call.
         constexpr int GXN = TW / 4 + 2, GYN = TW / 4;
         constexpr int NXI = GXN * TH, NYI = GYN * L::YH, NITEMS = NXI + NYI;
         constexpr int PERX = (NXI + NT - 1) / NT;
-        if (nx4 && interior) {
+        if (interior) {
             // Items past the end of a list are skipped, not recomputed: a wave whose lanes
             // are all past it branches over the call.  The xi_y items go in vertical pairs,
             // dealt from the thread after the last xi_x item (modulo the workgroup), so the
@@ -535,7 +543,7 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
                     lds_store4(s_jy + (r + 5) * L::YW + c0, accB);
                 }
             }
-        } else if (nx4) {
+        } else if constexpr (NOISE == kNoisePhilox) {
             constexpr int PER = (NITEMS + NT - 1) / NT;
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
@@ -567,29 +575,44 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
                 }
             }
         } else {
-            // Column groups straddle the periodic seam: one call per site.
+            // Seam tiles of fields whose columns do not split into fours: the column groups
+            // inside the field are Philox groups all the same, one call each; only those that
+            // leave it at the left or the right straddle two and are left to the loop below.
             for (int i = tid; i < NITEMS; i += NT) {
+                T z[4];
                 if (i < NXI) {
-                    const int r = i / GXN, gl = i - r * GXN - 1;
-                    const int grow = wrap_index(y0 + r, ny);
-                    T* dst = s_jx + r * L::XW + 4 * (gl + 1);
-                    for (int l = 0; l < 4; ++l)
-                        dst[l] = jx1(r, 4 * gl + l,
-                                     normal1<T>(grow, wrap_index(x0 + 4 * gl + l, nx), step, 1, key0, key1));
+                    const int r = i / GXN, c0 = 4 * (i - r * GXN - 1);
+                    if (x0 + c0 >= 0 && x0 + c0 + 3 < nx) {
+                        normals4<T>((uint32_t)((x0 + c0) >> 2), (uint32_t)wrap_index(y0 + r, ny), step, 1, key0, key1,
+                                    z);
+                        emit_x4(r, c0, z);
+                    }
                 } else {
-                    const int j = i - NXI;
-                    const int rr = j / GYN, gl = j - rr * GYN;
-                    T z[4];
+                    const int rr = (i - NXI) / GYN, gl = (i - NXI) - rr * GYN;
                     normals4<T>((uint32_t)((x0 >> 2) + gl), (uint32_t)wrap_index(y0 + rr - 4, ny), step, 0, key0,
                                 key1, z);
-                    T* dst = s_jy + rr * L::YW + 4 * gl;
-                    for (int l = 0; l < 4; ++l) dst[l] = jy1(rr - 4, 4 * gl + l, z[l]);
+                    emit_y4(rr - 4, 4 * gl, z);
                 }
+            }
+            // The sites of the straddling groups that an output reads, one call each: four a row
+            // left of column 0, and from the last whole group to four past the last column, at
+            // most seven.  (Against a call per site for every x group of such fields, interior
+            // tiles included, a step at T = 0.05 went from 15.3 to 13.0 us at 715 x 1021 FP32,
+            // 25.6 to 20.2 us in FP64, and 58.8 to 46.1 us at 1536 x 1535 FP64.)
+            const int nl = x0 == 0 ? 4 : 0;
+            const bool right = x0 + TW + 4 > nx;
+            const int first = right ? (nx - x0) & ~3 : 0;
+            const int ne = nl + (right ? (nx - x0 < TW ? nx - x0 : TW) + 4 - first : 0);
+            for (int i = tid; i < ne * TH; i += NT) {
+                const int e = i / TH, r = i - e * TH;
+                const int tc = e < nl ? e - 4 : first + e - nl;
+                const T z = normal1<T>(wrap_index(y0 + r, ny), wrap_index(x0 + tc, nx), step, 1, key0, key1);
+                s_jx[r * L::XW + tc + 4] = jx1(r, tc, z);
             }
         }
         if (active) active_current();
         __syncthreads();
-    } else if (NOISE == kNoiseBuffer) {
+    } else if constexpr (NOISE == kNoiseBuffer) {
         const size_t n = (size_t)ny * nx;
         for (int i = tid; i < L::XW * L::XH; i += NT) {
             const int r = i / L::XW, col = i - r * L::XW - 4;
@@ -603,24 +626,20 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
         __syncthreads();
     }
 
-    if constexpr (kNoisyKernel && sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
+    if constexpr (noisy && sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
 
     // ---- stage B: one column strip of R output rows per thread.  Row-wise partial
     // sums of the separable stencils are formed once per row and shared by the
     // output rows that need them.
     // With noise the D8 part is the divergence of J; without, D8oD8 of mu_p as one 17-tap
     // stencil per axis (cheaper when there is no noise current to form).
-    constexpr bool kAlwaysNoisy = NOISE == kNoisePhilox || NOISE == kNoiseBuffer;
-    constexpr bool kNeverNoisy = NOISE == kNoiseNone;
     const int c = cx, r0 = rg * R;
     T* orow = out + (size_t)(y0 + r0) * nx + (x0 + c);
-    T mcol[kAlwaysNoisy ? 1 : R + 16];  // mu_p at rows r0-8 .. r0+R+7 of this column
-    if constexpr (!kAlwaysNoisy) {
-        if (!noisy) {
-            const auto Mc = lds_base(s_mup + r0 * L::MW + c + 8);
+    T mcol[noisy ? 1 : R + 16];  // mu_p at rows r0-8 .. r0+R+7 of this column
+    if constexpr (!noisy) {
+        const auto Mc = lds_base(s_mup + r0 * L::MW + c + 8);
 #pragma unroll
-            for (int k = 0; k < R + 16; ++k) mcol[k] = Mc[k * L::MW];
-        }
+        for (int k = 0; k < R + 16; ++k) mcol[k] = Mc[k * L::MW];
     }
     // The strip's neighbouring rows, each formed just before the first output row that
     // needs it rather than all up front: the same values, fewer of them live at once (FP64
@@ -630,7 +649,7 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
     const bool lambda_b = !active;  // stage B applies G3xoG3x, G3yoG3y to mu_a
     T d2x[R + 4], sx[R + 4];        // mu_a rows r0-2 .. r0+R+1
     T hx[R + 2], sy[R + 2];         // rows r0-1 .. r0+R of q, or of C (above)
-    T ycol[kNeverNoisy ? 1 : R + 8];  // J_y at rows r0-4 .. r0+R+3 of this column
+    T ycol[noisy ? R + 8 : 1];  // J_y at rows r0-4 .. r0+R+3 of this column
     const auto Ab = lds_base(s_mua + r0 * L::AW + c + 2);
     const auto Qxb = lds_base(s_qx + (r0 + 1) * L::QW + c + 2);
     const auto Qyb = lds_base(s_qy + (r0 + 1) * L::QW + c + 2);
@@ -650,9 +669,7 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
         sy[k] = K.gyc * Qy[0] + K.gye * (Qy[-1] + Qy[1]);
     };
     auto row_y = [&](int k) {
-        if constexpr (!kNeverNoisy) {
-            if (noisy) ycol[k] = Yc[k * L::YW];
-        }
+        if constexpr (noisy) ycol[k] = Yc[k * L::YW];
     };
 #pragma unroll
     for (int k = 0; k < 4; ++k) row_a(k);
@@ -670,29 +687,24 @@ __device__ __forceinline__ void step_tile(T* const sm, const T* __restrict__ in,
         row_q(k + 2);
         row_y(k + 8);
         T acc = T(0);
-        if constexpr (!kNeverNoisy) {
-            if (noisy) {
-                // passive and noise: (1/dx) D8_x J_x + (1/dy) D8_y J_y
-                const auto X = Xb + k * L::XW;
-                acc = K.dxw[1] * (X[1] - X[-1]);
-                acc = fma(K.dyw[1], ycol[k + 5] - ycol[k + 3], acc);
+        if constexpr (noisy) {
+            // passive and noise: (1/dx) D8_x J_x + (1/dy) D8_y J_y
+            const auto X = Xb + k * L::XW;
+            acc = K.dxw[1] * (X[1] - X[-1]);
+            acc = fma(K.dyw[1], ycol[k + 5] - ycol[k + 3], acc);
 #pragma unroll
-                for (int j = 2; j <= 4; ++j) {
-                    acc = fma(K.dxw[j], X[j] - X[-j], acc);
-                    acc = fma(K.dyw[j], ycol[k + 4 + j] - ycol[k + 4 - j], acc);
-                }
+            for (int j = 2; j <= 4; ++j) {
+                acc = fma(K.dxw[j], X[j] - X[-j], acc);
+                acc = fma(K.dyw[j], ycol[k + 4 + j] - ycol[k + 4 - j], acc);
             }
-        }
-        if constexpr (!kAlwaysNoisy) {
-            if (!noisy) {
-                // passive: -(1/dx^2) D8oD8_x mu_p - (1/dy^2) D8oD8_y mu_p
-                const auto m = Mb + k * L::MW;
-                acc = K.p0 * mcol[k + 8];
+        } else {
+            // passive: -(1/dx^2) D8oD8_x mu_p - (1/dy^2) D8oD8_y mu_p
+            const auto m = Mb + k * L::MW;
+            acc = K.p0 * mcol[k + 8];
 #pragma unroll
-                for (int j = 1; j <= 8; ++j) {
-                    acc = fma(K.px[j], m[j] + m[-j], acc);
-                    acc = fma(K.py[j], mcol[k + 8 + j] + mcol[k + 8 - j], acc);
-                }
+            for (int j = 1; j <= 8; ++j) {
+                acc = fma(K.px[j], m[j] + m[-j], acc);
+                acc = fma(K.py[j], mcol[k + 8 + j] + mcol[k + 8 - j], acc);
             }
         }
         if (lambda_b) {
