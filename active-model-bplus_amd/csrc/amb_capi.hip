@@ -151,6 +151,9 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
     static_assert(sizeof(kF64) / sizeof(kF64[0]) == 0 AMB_F64_TILES(AMB_COUNT_ONE),
                   "the FP64 order must list every FP64 tile shape");
 #undef AMB_COUNT_ONE
+    // the index that stands for strips on large fields (step_grid), where they pay
+    const int strips = precision == AMB_F32 ? kSquare512F32 : kSquare512F64;
+    if (step_grid(precision, strips, noise, ny, nx).seg_rows > 0) return strips;
     const int n = tile_count(precision);
     const int* order = precision != AMB_F32 ? kF64 : noise == kNoiseNone ? kNoiselessF32 : kNoisyF32;
     int best = 0;
@@ -225,6 +228,7 @@ struct amb_handle {
     double* d_part = nullptr;
     unsigned long long* d_bad_part = nullptr;
     double* d_tile_part = nullptr;         // (sum, non-finite count) per tile, written by a run's last step
+    int64_t parts = 0;                     // how many of them the last step wrote
     double* d_sum = nullptr;
     unsigned long long* d_bad = nullptr;
     double last_sum = 0.0;                 // mass and non-finite count found by the last amb_run
@@ -250,13 +254,14 @@ template <typename T>
 StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int noise_mode, bool reduce = false)
 {
     StepArgs<T> a{};
-    const TileShape ts = tile_shape(h->precision, h->tile);
+    const StepGrid g = step_grid(h->precision, h->tile, noise_mode, h->ny, h->nx);
     a.in = static_cast<const T*>(h->buf[parity_in & 1]);
     a.out = static_cast<T*>(h->buf[(parity_in + 1) & 1]);
     a.ny = (int)h->ny;
     a.nx = (int)h->nx;
-    a.ntx = grid_tiles(h->nx, ts.tw);
-    a.nty = grid_tiles(h->ny, ts.th);
+    a.ntx = g.ntx;
+    a.nty = g.nty;
+    a.seg_rows = g.seg_rows;
     a.xcd_chunk = xcd_chunk(a.ntx * a.nty);
     a.k = make_coef<T>(h->stencil, h->model);
     a.key0 = (uint32_t)h->options.seed;
@@ -281,10 +286,11 @@ hipError_t launch_step(const amb_handle* h, int parity_in, int step_off, int noi
                            h->stream);
 }
 
-int64_t tiles_of(const amb_handle* h, int tile)
+// Workgroups of one step, each writing one partial of the fused finite check.
+int64_t parts_of(const amb_handle* h, int noise)
 {
-    const TileShape ts = tile_shape(h->precision, tile);
-    return (int64_t)grid_tiles(h->nx, ts.tw) * grid_tiles(h->ny, ts.th);
+    const StepGrid g = step_grid(h->precision, h->tile, noise, h->ny, h->nx);
+    return (int64_t)g.ntx * g.nty;
 }
 
 int noise_mode_of(const amb_handle* h)
@@ -338,6 +344,7 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
         if (mode == kNoiseBuffer) {
             if ((e = launch_step(h, h->cur, 0, mode, true)) != hipSuccess) return fail_hip(e, "step launch");
             if ((e = launch_advance(h->d_step, 1, h->stream)) != hipSuccess) return fail_hip(e, "advance launch");
+            h->parts = parts_of(h, mode);
             h->cur ^= 1;
             ++h->noise_used;
             --left;
@@ -352,12 +359,14 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
             const int64_t reps = left / kGraphSteps;
             for (int64_t r = 0; r < reps; ++r)
                 if ((e = hipGraphLaunch(h->graph[p], h->stream)) != hipSuccess) return fail_hip(e, "hipGraphLaunch");
+            h->parts = parts_of(h, mode);
             left -= reps * kGraphSteps;
             continue;
         }
         for (int k = 0; k < left; ++k)
             if ((e = launch_step(h, h->cur + k, k, mode, k == left - 1)) != hipSuccess) return fail_hip(e, "step launch");
         if ((e = launch_advance(h->d_step, left, h->stream)) != hipSuccess) return fail_hip(e, "advance launch");
+        h->parts = parts_of(h, mode);
         h->cur = (int)((h->cur + left) & 1);
         left = 0;
     }
@@ -397,7 +406,7 @@ int finish_run(amb_handle* h, int64_t nsteps, double* sum, int64_t* bad)
         }
         return rc;
     }
-    hipError_t e = launch_reduce_tiles(h->d_tile_part, tiles_of(h, h->tile), h->d_sum, h->d_bad, h->stream);
+    hipError_t e = launch_reduce_tiles(h->d_tile_part, h->parts, h->d_sum, h->d_bad, h->stream);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
     if ((e = hipMemcpyAsync(h->h_sum, h->d_sum, sizeof(double), hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
         return fail_hip(e, "hipMemcpyAsync");
@@ -605,8 +614,13 @@ int amb_create(const double* field, int64_t ny, int64_t nx, const amb_stencil* s
     AMB_CHECK(hipMalloc(&h->d_part, kReduceBlocks * sizeof(double)));
     AMB_CHECK(hipMalloc(&h->d_bad_part, kReduceBlocks * sizeof(unsigned long long)));
     {
-        int64_t most = 1;  // partials for the tile shape with the most tiles (the tile may change)
-        for (int t = 0; t < tile_count(h->precision); ++t) most = std::max(most, tiles_of(h, t));
+        // partials for the tile shape with the most tiles (the tile may change); strips, on
+        // large fields only, are far fewer
+        int64_t most = 1;
+        for (int t = 0; t < tile_count(h->precision); ++t) {
+            const TileShape ts = tile_shape(h->precision, t);
+            most = std::max(most, (int64_t)grid_tiles(nx, ts.tw) * grid_tiles(ny, ts.th));
+        }
         AMB_CHECK(hipMalloc(&h->d_tile_part, (size_t)most * 2 * sizeof(double)));
     }
     AMB_CHECK(hipMalloc(&h->d_sum, sizeof(double)));

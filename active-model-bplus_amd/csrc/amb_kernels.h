@@ -28,6 +28,7 @@ struct StepArgs {
     T* out;
     int ny, nx;
     int ntx, nty;     // tiles along x and y
+    int seg_rows;     // > 0: strips, this many output rows per workgroup
     int xcd_chunk;    // > 0: blockIdx remapped so each XCD gets a contiguous run of tiles
     StepCoef<T> k;
     uint32_t key0, key1;
@@ -52,6 +53,7 @@ struct TileShape {
 // default tile follows an order of preference per kernel (default_tile in amb_capi.hip).
 #define AMB_F32_TILES(X) X(0, 32, 48, 512) X(1, 32, 24, 256) X(2, 32, 32, 256) X(3, 64, 32, 512) X(4, 64, 16, 256) X(5, 32, 16, 256) X(6, 16, 16, 128) X(7, 16, 8, 128) X(8, 8, 8, 64) X(9, 32, 32, 512)
 #define AMB_F64_TILES(X) X(0, 32, 32, 256) X(1, 64, 16, 256) X(2, 32, 16, 256) X(3, 32, 32, 512) X(4, 16, 16, 128) X(5, 16, 8, 128) X(6, 8, 8, 64)
+constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threads
 // FP32 orders of preference, measured on MI355X (the times below predate the step's wave
 // priorities, which took 2-4% off every shape).  Noisy: 32x32 tiles of 512 threads are
 // fastest at 4096^2 (108.1 us per step; 32x48 111.5 us, 32x16 116.9 us, the others 120-139
@@ -73,6 +75,16 @@ struct TileShape {
 // Tile shapes compiled per precision (index = autotuner choice).
 int tile_count(int precision);
 TileShape tile_shape(int precision, int index);
+
+// Workgroups of one step of a whole field: ntx x nty tiles or, on large fields in place of
+// 32x32 tiles of 512 threads, strips of columns each seg_rows rows long (amb_march.h; the
+// rule and its reason are at step_grid).
+struct StepGrid {
+    int ntx, nty;
+    int seg_rows;  // 0: tiles
+};
+StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx);
+int device_cus();  // compute units of the current device
 
 // Launches one fused step.  Returns a hipError_t.
 hipError_t launch_step_f32(const StepArgs<float>& a, int tile, int noise, hipStream_t s);

@@ -90,12 +90,13 @@ int run_noalloc(T* field, T* work, int64_t ny, int64_t nx, const amb_stencil& st
     double* sum = reinterpret_cast<double*>(base + 16);
     unsigned long long* bad = reinterpret_cast<unsigned long long*>(base + 24);
     double* part = reinterpret_cast<double*>(base + kPartOffset);
-    const TileShape ts = tile_shape(sizeof(T) == 4 ? AMB_F32 : AMB_F64, tile);
+    const StepGrid g = step_grid(sizeof(T) == 4 ? AMB_F32 : AMB_F64, tile, noise, ny, nx);
     StepArgs<T> a{};
     a.ny = (int)ny;
     a.nx = (int)nx;
-    a.ntx = grid_tiles(nx, ts.tw);
-    a.nty = grid_tiles(ny, ts.th);
+    a.ntx = g.ntx;
+    a.nty = g.nty;
+    a.seg_rows = g.seg_rows;
     a.xcd_chunk = xcd_chunk(a.ntx * a.nty);
     a.k = make_coef<T>(st, md);
     a.key0 = (uint32_t)seed;

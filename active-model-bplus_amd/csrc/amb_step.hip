@@ -21,7 +21,10 @@
 // halo copies that neighbouring tiles generate are bit-identical to the owner's.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "amb_kernels.h"
+#include "amb_march.h"
 #include "amb_math.h"
 #include "amb_tile.h"
 
@@ -43,6 +46,28 @@ __global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) vo
                                     p.key0, p.key1, step, p.noise, p.part ? p.part + 2 * (size_t)t : nullptr);
 }
 
+// ---- strips (amb_march.h) ------------------------------------------------------
+// Bound by vector issue: at 4096^2 FP32 noisy 140 instructions a site against 219 for 32x32
+// tiles (which compute mu_p, the noise and the currents of their halos about twice over), the
+// vector units busy 90% of the time; 102 -> 71 us a step, FP64 242 -> 169 us.  The noiseless
+// kernel runs 100 a site (tiles 173) but its role B, a chain of 59 a row, leaves them idle a
+// third of the time; 87.6 -> 69.7 us.
+template <typename T, int NOISE, bool ACTIVE>
+__global__ __launch_bounds__((MarchLds<T, NOISE == kNoisePhilox, ACTIVE>::NT),
+                             (MarchLds<T, NOISE == kNoisePhilox, ACTIVE>::min_waves))
+void march_kernel(const StepArgs<T> p)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    int t = blockIdx.x;
+    if (p.xcd_chunk > 0) t = (t & 7) * p.xcd_chunk + (t >> 3);
+    const int sg = t / p.ntx, tx = t - sg * p.ntx;
+    const uint64_t step = NOISE == kNoisePhilox ? (uint64_t)(*p.step_base) + (uint64_t)p.step_off : 0;
+    const int y0 = sg * p.seg_rows;
+    march_strip<T, NOISE, ACTIVE>(reinterpret_cast<T*>(smem_raw), p.in, p.out, p.ny, p.nx, tx * kMarchCols, y0,
+                                  min(p.seg_rows, p.ny - y0), p.k, p.key0, p.key1, step,
+                                  p.part ? p.part + 2 * (size_t)t : nullptr);
+}
+
 // ---- tile table ---------------------------------------------------------------
 
 #define AMB_SHAPE(i, tw, th, nt) {tw, th, nt},
@@ -59,6 +84,96 @@ int tile_count(int precision)
 TileShape tile_shape(int precision, int index)
 {
     return precision == 32 ? kTilesF32[index] : kTilesF64[index];
+}
+
+int device_cus()
+{
+    static std::atomic<int> known[64];  // per device
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    const bool slot = device >= 0 && device < 64;
+    if (slot && (cus = known[device].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    if (slot) known[device].store(cus, std::memory_order_relaxed);
+    return cus;
+}
+
+// March kernel of a field: the active current is formed where step_tile forms it.
+template <typename T>
+static bool march_active(int64_t ny, int64_t nx)
+{
+    return sizeof(T) == 4 && ny * nx >= kActiveCurrentSites;
+}
+
+static int march_per_cu(int precision, int noise, int64_t ny, int64_t nx)
+{
+    if (precision == 32)
+        return noise == kNoiseNone              ? MarchLds<float, false, false>::per_cu
+               : march_active<float>(ny, nx) ? MarchLds<float, true, true>::per_cu
+                                                : MarchLds<float, true, false>::per_cu;
+    return noise == kNoiseNone ? MarchLds<double, false, false>::per_cu : MarchLds<double, true, false>::per_cu;
+}
+
+// Rows per workgroup of the march kernel: the device's workgroup slots filled once, twice ...
+// with segments of equal length, whichever takes least time, a segment costing its rows and
+// kMarchFill rows' time for its first steps, when the later roles still wait for theirs.
+constexpr int kMarchFill = 24;
+
+static int64_t march_cost(int64_t ny, int strips, int slots, int* seg_rows)
+{
+    int64_t best = 0;
+    for (int r = 1; r <= 4; ++r) {
+        const int64_t segs = (int64_t)r * slots / strips;
+        if (segs < 1) continue;
+        const int64_t rows = ((ny + segs - 1) / segs + kMarchRows - 1) / kMarchRows * kMarchRows;
+        const int64_t cost = r * (rows + kMarchFill);
+        if (best == 0 || cost < best) {
+            best = cost;
+            *seg_rows = (int)rows;
+        }
+    }
+    return best;  // 0: more strips than four rounds hold
+}
+
+// Strips take the place of 32x32 tiles of 512 threads where the device's lanes are busy enough
+// with them: the sites over the lane-rows (slots x march_cost x columns of a strip) that their
+// workgroups run through.  A step at T = 0.05 and T = 0, tiles -> strips in us, around the line:
+//   share      FP32 noisy          FP32 quiet          FP64 noisy          FP64 quiet
+//   0.25-0.3   1024^2 11.0 -> 13.8 1024^2  9.4 -> 14.6
+//   0.38-0.42                      1024x2048 15.2->16.5 1024^2 19.7 -> 23.5 1024^2 15.4 -> 21.0
+//   0.47-0.49  1024x2048 18.1->18.3 1024x3072 20.7->20.7 1200^2 29.6 -> 26.2 1200^2 23.5 -> 23.1
+//   0.50-0.54  1664^2 22.0 -> 20.9 1792^2 21.1 -> 18.9 2048x1024 35.5->33.5 2048x1024 26.4->30.6
+//   0.57-0.63  2048^2 30.0 -> 25.2 2048^2 26.5 -> 24.7 1536^2 40.1 -> 33.8 1664^2 40.7 -> 34.2
+//   0.70-0.86  4096^2 102 -> 71.3  4096^2 87.6 -> 69.7 4096^2 242 -> 169   4096^2 173 -> 161
+// Fields whose columns do not split into fours gain more (2050 x 2049 FP32 45.3 -> 26.1).
+// Every field's 32-bit byte offsets must reach it, and an explicit noise buffer takes tiles.
+constexpr double kStripShareF32[2] = {0.495, 0.48}, kStripShareF64[2] = {0.63, 0.482};  // quiet, noisy
+
+StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx)
+{
+    const TileShape ts = tile_shape(precision, tile);
+    StepGrid g{(int)((nx + ts.tw - 1) / ts.tw), (int)((ny + ts.th - 1) / ts.th), 0};
+    const int64_t sites = ny * nx;
+    if (tile != (precision == 32 ? kSquare512F32 : kSquare512F64) || noise == kNoiseBuffer || ny < 4 || nx < 4 ||
+        sites > ((int64_t)1 << 31) / (precision / 8))
+        return g;
+    const int strips = (int)((nx + kMarchCols - 1) / kMarchCols);
+    const int slots = device_cus() * march_per_cu(precision, noise, ny, nx);
+    int seg_rows = 0;
+    const int64_t cost = march_cost(ny, strips, slots, &seg_rows);
+    const double share = (double)sites / ((double)slots * (double)cost * kMarchCols);
+    const double least = (precision == 32 ? kStripShareF32 : kStripShareF64)[noise != kNoiseNone];
+    if (cost == 0 || share < least) return g;
+    g.ntx = strips;
+    g.seg_rows = seg_rows;
+    g.nty = (int)((ny + seg_rows - 1) / seg_rows);
+    return g;
 }
 
 template <typename T, int TW, int TH, int NT, int NOISE>
@@ -81,11 +196,30 @@ static hipError_t launch_noise(const StepArgs<T>& a, int noise, hipStream_t s)
     }
 }
 
+template <typename T, int NOISE, bool ACTIVE>
+static hipError_t launch_march_one(const StepArgs<T>& a, hipStream_t s)
+{
+    using L = MarchLds<T, NOISE == kNoisePhilox, ACTIVE>;
+    hipLaunchKernelGGL((march_kernel<T, NOISE, ACTIVE>), dim3(a.ntx * a.nty), dim3(L::NT), L::bytes, s, a);
+    return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t launch_march(const StepArgs<T>& a, int noise, hipStream_t s)
+{
+    if (noise == kNoiseNone) return launch_march_one<T, kNoiseNone, false>(a, s);
+    if (noise != kNoisePhilox) return hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 4)
+        if (march_active<T>(a.ny, a.nx)) return launch_march_one<T, kNoisePhilox, true>(a, s);
+    return launch_march_one<T, kNoisePhilox, false>(a, s);
+}
+
 #define AMB_CASE_F32(i, tw, th, nt) case i: return launch_noise<float, tw, th, nt>(a, noise, s);
 #define AMB_CASE_F64(i, tw, th, nt) case i: return launch_noise<double, tw, th, nt>(a, noise, s);
 
 hipError_t launch_step_f32(const StepArgs<float>& a, int tile, int noise, hipStream_t s)
 {
+    if (a.seg_rows > 0) return launch_march(a, noise, s);
     switch (tile) {
         AMB_F32_TILES(AMB_CASE_F32)
     default: return hipErrorInvalidValue;
@@ -94,6 +228,7 @@ hipError_t launch_step_f32(const StepArgs<float>& a, int tile, int noise, hipStr
 
 hipError_t launch_step_f64(const StepArgs<double>& a, int tile, int noise, hipStream_t s)
 {
+    if (a.seg_rows > 0) return launch_march(a, noise, s);
     switch (tile) {
         AMB_F64_TILES(AMB_CASE_F64)
     default: return hipErrorInvalidValue;
@@ -162,7 +297,11 @@ hipError_t prepare_step_kernels()
     hipError_t e = hipSuccess;
     AMB_F32_TILES(AMB_RAISE_F32)
     AMB_F64_TILES(AMB_RAISE_F64)
-    return e;
+    using L = MarchLds<double, true, false>;  // the only march kernel above 64 KB
+    static_assert(MarchLds<double, false, false>::bytes <= 65536 && MarchLds<float, true, false>::bytes <= 65536 &&
+                      MarchLds<float, true, true>::bytes <= 65536, "raise their limit too");
+    return hipFuncSetAttribute((const void*)march_kernel<double, kNoisePhilox, false>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes);
 }
 
 // ---- step counter -------------------------------------------------------------

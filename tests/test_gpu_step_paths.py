@@ -30,3 +30,43 @@ def test_ragged_columns_match_oracle(amb, oracle, shape):
         sim.run(20)
         err = np.abs(sim.field - ref).max() / np.abs(ref).max()
         assert err < 1e-12, (shape, tile, err)
+
+
+# Large fields run in strips of 112 columns and segments of rows instead of 32x32 tiles.  The
+# grids have a last strip of one to 111 columns, columns that do and do not split into fours, a
+# last segment shorter than the others and not a multiple of its four rows, and few rows.
+@pytest.mark.parametrize("precision,shape,temperature", [
+    (32, (1787, 1801), 0.0), (32, (2048, 2016), 0.0),
+    (32, (1795, 1793), 0.05), (32, (2051, 2047), 0.05), (32, (2049, 2128), 0.05),
+    (64, (1201, 1203), 0.05), (64, (1667, 1665), 0.0), (64, (61, 40000), 0.05)])
+def test_strips_equal_tiles(amb, precision, shape, temperature):
+    """The same bits as 32x24 (FP32) or 64x16 (FP64) tiles after 5 steps, and a fused mass and
+    finite count equal to a full read of the field."""
+    rng = np.random.default_rng(shape[0])
+    phi = 0.1 + 0.05 * rng.standard_normal(shape, dtype=np.float32).astype(np.float64)
+    st, md = amb.Stencil(5e-3, 1.25, 0.75), amb.Model(-0.25, 0.1, 0.25, 1, 0.5, -1, temperature)
+    out = []
+    for tile in (0, 2):
+        sim = amb.Integrator(phi, st, md, seed=3, precision=precision, tile=tile)
+        sim.run(5)
+        out.append(sim.field)
+        fused, bad = sim.last_mass()
+        full, bad_full = sim.mass()
+        # both are FP64 sums of the same values in different orders: n eps / 2 at worst, with
+        # every value of order 0.1 and n = 4e6 well under 1e-9 of the sum
+        assert bad == 0 and bad_full == 0 and abs(fused - full) <= 1e-9 * abs(full)
+    assert np.array_equal(out[0], out[1])
+
+
+def test_strips_count_nonfinite_sites(amb):
+    phi = np.zeros((2048, 2050))
+    phi[2047, 2049] = np.nan
+    sim = amb.Integrator(phi, amb.Stencil(5e-3, 1, 1), amb.Model(-0.25, 0, 0.25, 1, 0.5, -1, 0), precision=32)
+    with pytest.raises(amb.CudaException):
+        sim.run(1)
+    _, bad = sim.last_mass()
+    _, bad_full = sim.mass()
+    # L3 and G3 spread the site to a 3x3 box of mu_p and mu_a; D8 of D8 takes the box 8 sites
+    # along each axis (a cross of two 3 x 19 bars), G3 of G3 to the 7x7 square, 16 sites of which
+    # the cross misses
+    assert bad == bad_full == (2 * 3 * 19 - 9) + 16
