@@ -538,71 +538,149 @@ __global__ __launch_bounds__(256 * TY) void c12_kernel(const float* __restrict__
 
 // ---- weight gradient ----------------------------------------------------------------
 // part[chunk][tap][co][ci] = sum_{p in chunk} dpre[p][co] * in[p + shift(tap)][ci].
-// 32-pixel K-steps are staged transposed in LDS so each lane reads its 8 pixels as
-// one 16-byte vector.
-template <int NBO, int NBI>
-__global__ __launch_bounds__(256) void wgrad_kernel(const bf16* __restrict__ dpre, const bf16* __restrict__ in,
-                                                    int taps, int H, int W, int chunk, float* __restrict__ part)
+// Contraction over pixels, but both operands lie channels-first in memory: a stage of 128
+// pixels is kept in LDS as it is read (16-byte stores) and the matrix operands, eight
+// pixels of one channel per lane, come from transposing LDS reads (ds_read_b64_tr_b16).
+// A workgroup takes one tap row dy of one chunk, GO x GI of the 16-channel groups and all
+// DX taps of that row: the row's taps are the same LDS image read one pixel apart.  The
+// image has a halo pixel on both sides of every 16 pixels (sides are multiples of 16 at
+// every level, so 16 pixels share a row).  The next stage's loads are in flight during a
+// stage, one barrier per stage.  Each accumulator still takes its chunk's pixels in order.
+// Staging through 2-byte transposed LDS stores, once per tap, the seven layers took
+// 1290 us for 16 samples of 256 x 256, now 253.
+constexpr int kWgStage = 128;
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+
+// Eight pixels of this lane's channel: `src` is the lane's 4-channel piece (lane % 16) % 4
+// of pixel (lane % 16) / 4; the second four pixels follow at `second`.
+__device__ __forceinline__ bf16x8 read_tr(const bf16* src, int second)
 {
-    constexpr int COUT = 16 * NBO, CIN = 16 * NBI, PS = 128, LD = PS + 8;  // 128 pixels per stage
-    constexpr int TILES = NBO * NBI, TPW = (TILES + 3) / 4;
-    __shared__ __align__(16) bf16 sA[COUT * LD];
-    __shared__ __align__(16) bf16 sB[CIN * LD];
-    const int c = blockIdx.x, tap = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)src);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(src + second));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// NW waves as NWO x NW / NWO over the GO x GI channel groups.
+template <int COUT, int CIN, int TAPS, int GO, int GI, int NWO, int NW>
+__global__ __launch_bounds__(64 * NW) void wgrad_kernel(const bf16* __restrict__ dpre, const bf16* __restrict__ in,
+                                                        int H, int W, int chunk, float* __restrict__ part)
+{
+    constexpr int DX = TAPS == 9 ? 3 : 1, HALO = DX / 2, SEG = 16 + 2 * HALO, NSEG = kWgStage / 16;
+    constexpr int NT = 64 * NW, NWI = NW / NWO, MO = GO / NWO, MI = GI / NWI;
+    constexpr int LA = 16 * GO + 8, LB = 16 * GI + 8;  // LDS pixel pitches
+    constexpr int VA = kWgStage * 2 * GO, VB = NSEG * SEG * 2 * GI;  // 16-byte pieces of a stage
+    constexpr int PA = (VA + NT - 1) / NT, PB = (VB + NT - 1) / NT;
+    static_assert(GO % NWO == 0 && GI % NWI == 0 && VA % NT == 0, "wave split");
+    __shared__ __align__(16) bf16 sA[2][kWgStage * LA];
+    __shared__ __align__(16) bf16 sB[2][NSEG * SEG * LB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane >> 4, l16 = lane & 15;
-    const int dy = taps == 9 ? tap / 3 - 1 : 0, dx = taps == 9 ? tap % 3 - 1 : 0;
-    f32x4 acc[TPW];
+    const int c = blockIdx.x, dyi = TAPS == 9 ? blockIdx.y % 3 : 0, grp = TAPS == 9 ? blockIdx.y / 3 : blockIdx.y;
+    const int co0 = 16 * GO * (grp % (COUT / (16 * GO))), ci0 = 16 * GI * (grp / (COUT / (16 * GO)));
+    const int dy = TAPS == 9 ? dyi - 1 : 0;
+    const size_t pbeg = (size_t)c * chunk;
+
+    // the thread's pieces of `in`: 16-pixel segment (column xs, row), advanced by a stage
+    const int ws = W / 16, rstep = NSEG / ws, xstep = NSEG - rstep * ws;
+    int bx[PB], by[PB];
+    size_t brow[PB];
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int pbeg = c * chunk;
-    for (int p0 = pbeg; p0 < pbeg + chunk; p0 += PS) {
-        // 16-byte loads (8 channels of one pixel), written transposed into LDS
-        for (int e = threadIdx.x; e < PS * (COUT / 8); e += 256) {
-            const int pl = e / (COUT / 8), c8 = (e - pl * (COUT / 8)) * 8;
-            const u32x4 v = load8u(dpre + (size_t)(p0 + pl) * COUT + c8);
+    for (int k = 0; k < PB; ++k) {
+        const int i = min(tid + NT * k, VB - 1), seg = i / (2 * GI) / SEG;
+        const size_t g = pbeg / 16 + seg;
+        brow[k] = g / ws;
+        bx[k] = (int)(g - brow[k] * ws);
+        by[k] = (int)(brow[k] % H);
+    }
+    u32x4 va[PA], vb[PB];
+    size_t pa = pbeg;
+    auto fetch = [&]() {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sA[(c8 + 2 * j) * LD + pl] = (bf16)(v[j] & 0xffffu);
-                sA[(c8 + 2 * j + 1) * LD + pl] = (bf16)(v[j] >> 16);
-            }
+        for (int k = 0; k < PA; ++k) {
+            const int i = tid + NT * k, px = i / (2 * GO), c8 = 8 * (i % (2 * GO));
+            va[k] = load8u(dpre + (pa + px) * COUT + co0 + c8);
         }
-        for (int e = threadIdx.x; e < PS * (CIN / 8); e += 256) {
-            const int pl = e / (CIN / 8), c8 = (e - pl * (CIN / 8)) * 8;
-            const int p = p0 + pl;
-            const int x = p % W, t = p / W, y = t % H, n = t / H;
-            const u32x4 v = load8u(in + (((size_t)n * H + wrapi(y + dy, H)) * W + wrapi(x + dx, W)) * CIN + c8);
+        pa += kWgStage;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sB[(c8 + 2 * j) * LD + pl] = (bf16)(v[j] & 0xffffu);
-                sB[(c8 + 2 * j + 1) * LD + pl] = (bf16)(v[j] >> 16);
+        for (int k = 0; k < PB; ++k) {
+            const int i = min(tid + NT * k, VB - 1), sl = i / (2 * GI) % SEG, c8 = 8 * (i % (2 * GI));
+            const int yy = by[k] + dy;
+            const size_t row = brow[k] + dy + (yy < 0 ? H : (yy >= H ? -H : 0));
+            vb[k] = load8u(in + (row * W + wrapi(16 * bx[k] + sl - HALO, W)) * CIN + ci0 + c8);
+            bx[k] += xstep;
+            int r = rstep;
+            if (bx[k] >= ws) {
+                bx[k] -= ws;
+                ++r;
             }
+            brow[k] += r;
+            by[k] += r;
+            if (by[k] >= H) by[k] -= H;
         }
-        __syncthreads();
+    };
+    auto put = [&](int buf) {
 #pragma unroll
-        for (int ks = 0; ks < PS; ks += 32) {
+        for (int k = 0; k < PA; ++k) {
+            const int i = tid + NT * k;
+            *reinterpret_cast<u32x4*>(sA[buf] + i / (2 * GO) * LA + 8 * (i % (2 * GO))) = va[k];
+        }
 #pragma unroll
-            for (int i = 0; i < TPW; ++i) {
-                const int tile = wave + 4 * i;
-                if (tile < TILES) {
-                    const int ib = tile / NBI, jb = tile - ib * NBI;
-                    const bf16x8 a = load8(sA + (16 * ib + l16) * LD + ks + 8 * q);
-                    const bf16x8 b = load8(sB + (16 * jb + l16) * LD + ks + 8 * q);
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i], 0, 0, 0);
+        for (int k = 0; k < PB; ++k) {
+            const int i = tid + NT * k;
+            if (i < VB) *reinterpret_cast<u32x4*>(sB[buf] + i / (2 * GI) * LB + 8 * (i % (2 * GI))) = vb[k];
+        }
+    };
+
+    f32x4 acc[DX][MO][MI];
+#pragma unroll
+    for (int d = 0; d < DX; ++d)
+#pragma unroll
+        for (int o = 0; o < MO; ++o)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) acc[d][o][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int wo = (wave % NWO) * MO, wi = (wave / NWO) * MI;
+    // lane's piece of a K-step of 32 pixels: quarter q takes pixels 8q .. 8q + 7
+    const int la = (8 * q + (l16 >> 2)) * LA + 4 * (l16 & 3) + 16 * wo;
+    const int lb = ((q >> 1) * SEG + 8 * (q & 1) + (l16 >> 2)) * LB + 4 * (l16 & 3) + 16 * wi;
+    const int stages = chunk / kWgStage;
+    fetch();
+    put(0);
+    if (stages > 1) fetch();
+    __syncthreads();
+    for (int sg = 0; sg < stages; ++sg) {
+        const int buf = sg & 1;
+        if (sg + 1 < stages) put(buf ^ 1);  // the other buffer was last read before the barrier
+        if (sg + 2 < stages) fetch();
+#pragma unroll
+        for (int ks = 0; ks < kWgStage / 32; ++ks) {
+            bf16x8 a[MO];
+#pragma unroll
+            for (int o = 0; o < MO; ++o) a[o] = read_tr(sA[buf] + la + 32 * ks * LA + 16 * o, 4 * LA);
+#pragma unroll
+            for (int d = 0; d < DX; ++d)
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const bf16x8 b = read_tr(sB[buf] + lb + (2 * ks * SEG + d) * LB + 16 * i, 4 * LB);
+#pragma unroll
+                    for (int o = 0; o < MO; ++o)
+                        acc[d][o][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[o], b, acc[d][o][i], 0, 0, 0);
                 }
-            }
         }
         __syncthreads();
     }
-    float* dst = part + ((size_t)c * taps + tap) * COUT * CIN;
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        const int tile = wave + 4 * i;
-        if (tile < TILES) {
-            const int ib = tile / NBI, jb = tile - ib * NBI;
+    for (int d = 0; d < DX; ++d) {
+        float* dst = part + (((size_t)c * TAPS + dyi * DX + d) * COUT + co0) * CIN + ci0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dst[(16 * ib + 4 * q + r) * CIN + 16 * jb + l16] = acc[i][r];
-        }
+        for (int o = 0; o < MO; ++o)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    dst[(size_t)(16 * (wo + o) + 4 * q + r) * CIN + 16 * (wi + i) + l16] = acc[d][o][i][r];
     }
 }
 
@@ -1316,27 +1394,31 @@ hipError_t conv(const ConvIn& in, int cin, const bf16* w, const float* bias, int
 
 ConvIn plain(const bf16* a) { return ConvIn{a, nullptr, nullptr, nullptr}; }
 
-template <int NBO, int NBI>
-hipError_t wgrad_launch(const bf16* dpre, const bf16* in, int taps, int H, int W, int npix, float* part, hipStream_t st)
+template <int COUT, int CIN, int TAPS, int GO, int GI, int NWO, int NW>
+hipError_t wgrad_launch(const bf16* dpre, const bf16* in, int H, int W, int npix, float* part, hipStream_t st)
 {
     const int chunk = chunk_for(npix);
-    hipLaunchKernelGGL((wgrad_kernel<NBO, NBI>), dim3(npix / chunk, taps), dim3(256), 0, st, dpre, in, taps, H, W,
-                       chunk, part);
+    const int groups = COUT / (16 * GO) * (CIN / (16 * GI)) * (TAPS == 9 ? 3 : 1);
+    hipLaunchKernelGGL((wgrad_kernel<COUT, CIN, TAPS, GO, GI, NWO, NW>), dim3(npix / chunk, groups), dim3(64 * NW), 0,
+                       st, dpre, in, H, W, chunk, part);
     return hipGetLastError();
 }
 
+// The channel groups of a workgroup shrink with the level: a chunk's sum is one chain, so
+// a level of a sixteenth of the pixels has a sixteenth of the chunks to fill the device.
 hipError_t wgrad(const bf16* dpre, int cout, const bf16* in, int cin, int taps, int H, int W, int npix, float* part,
                  hipStream_t st)
 {
-#define AMB_WG(co, ci) \
-    if (cout == 16 * co && cin == 16 * ci) return wgrad_launch<co, ci>(dpre, in, taps, H, W, npix, part, st);
-    AMB_WG(2, 1)  // c1: 32 <- 16
-    AMB_WG(4, 2)  // c2: 64 <- 32
-    AMB_WG(8, 4)  // c3: 128 <- 64
-    AMB_WG(4, 8)  // c4: 64 <- 128
-    AMB_WG(4, 4)  // c5: 64 <- 64
-    AMB_WG(2, 4)  // c6: 32 <- 64
-    AMB_WG(2, 2)  // c7: 32 <- 32
+#define AMB_WG(co, ci, t, go, gi, nwo, nw) \
+    if (cout == co && cin == ci && taps == t)  \
+        return wgrad_launch<co, ci, t, go, gi, nwo, nw>(dpre, in, H, W, npix, part, st);
+    AMB_WG(32, 16, 9, 2, 1, 2, 2)   // c1
+    AMB_WG(64, 32, 9, 4, 2, 2, 4)   // c2
+    AMB_WG(128, 64, 9, 4, 2, 2, 4)  // c3
+    AMB_WG(64, 128, 1, 2, 2, 2, 4)  // c4
+    AMB_WG(64, 64, 9, 4, 2, 2, 4)   // c5
+    AMB_WG(32, 64, 1, 2, 2, 2, 4)   // c6
+    AMB_WG(32, 32, 9, 2, 2, 2, 4)   // c7
 #undef AMB_WG
     return hipErrorInvalidValue;
 }
