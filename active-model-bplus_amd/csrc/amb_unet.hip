@@ -85,7 +85,7 @@ __device__ __forceinline__ float hi_f(uint32_t w) { return __uint_as_float(w & 0
 
 // ---- convolution forward / backward-data --------------------------------------------
 
-enum ConvMode { kOutBf16 = 0, kOutBf16Gelu = 1, kOutF32 = 2 };
+enum ConvMode { kOutBf16 = 0, kOutBf16Gelu = 1, kOutF32 = 2, kOutGeluBwd = 3 };
 // Where the A operand comes from: a plain NHWC tensor; the 2x2 average of a tensor of
 // twice the resolution (fused avgpool); up2(coarse) + skip (fused up-sampling add);
 // or the network input assembled from phi and the parameters (fused input layer).
@@ -140,95 +140,152 @@ __device__ __forceinline__ bf16x8 load_a(const ConvIn& src, int cin, int n, int 
     }
 }
 
-// out[p][co] = bias[co] + sum_{tap, ci} A[p + shift(tap)][ci] * w[tap][co][ci]
-// (flip: shift negated, used for the data gradient with the [tap][cin][cout] layout).
-// The next K-step's operands are loaded before the current step's MFMAs issue.
-template <int MB, int NB, int MODE, int SRC>
-__global__ __launch_bounds__(256) void conv_kernel(const ConvIn src, int cin, const bf16* __restrict__ w,
-                                                   const float* __restrict__ bias, int taps, int flip, int H, int W,
-                                                   void* __restrict__ out, bf16* __restrict__ pre)
+// Training convolution: out[p][co] = bias[co] + sum_{tap, ci} in[p + shift(tap)][ci] *
+// w[tap][co][ci] (FLIP: shift negated, the data gradient with the [tap][cin][cout] layout),
+// then MODE: bfloat16 (pre-activation and GELU of it; or the sum itself), FP32, or bfloat16
+// of the sum times gelu'(pre), the gradient at a pre-activation `pre`.
+//
+// A block takes TY x 16 pixels: the padded input tile is staged in LDS once for all taps and
+// all output channels, and each of the NWC x NWR waves holds the weights of its NB / NWC
+// channel blocks over all of K in registers and runs down its TY / NWR rows.  Weights are the
+// left operand, so a lane of the result holds 4 NBW neighbouring channels of one pixel
+// (channel block rows are dealt out that way) and stores 8 to 32 bytes at once.  What is left
+// is mostly the activations' trip to and from memory.  Reading both operands from global
+// memory at every K-step and storing two bytes at a time, the twelve convolutions, and the
+// passes that applied gelu' to their FP32 results, took 780 us for 16 samples of 256 x 256,
+// now 345 us.  The sum runs over K in the same 32-wide steps as the inference kernels'.
+template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP>
+__global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __restrict__ in, const bf16* __restrict__ w,
+                                                              const float* __restrict__ bias, int H, int W,
+                                                              void* __restrict__ out, bf16* __restrict__ pre)
 {
-    constexpr int COUT = 16 * NB;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int COUT = 16 * NB, K = TAPS * CIN, NS = (K + 31) / 32, NBW = NB / NWC, MR = TY / NWR;
+    constexpr int HALO = TAPS == 9 ? 1 : 0, PW = 16 + 2 * HALO, PH = TY + 2 * HALO, LD = CIN + 8;
+    constexpr int NT = 64 * NWC * NWR, ITEMS = PH * PW * (CIN / 8), PER = (ITEMS + NT - 1) / NT;
+    static_assert(NB % NWC == 0 && TY % NWR == 0 && CIN % 16 == 0, "tile shape");
+    __shared__ __align__(16) bf16 tile[PH * PW * LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane >> 4, l16 = lane & 15;
-    const int pix0 = (blockIdx.x * 4 + wave) * (16 * MB);
-    int pn[MB], py[MB], px[MB];
-#pragma unroll
-    for (int m = 0; m < MB; ++m) {
-        const int p = pix0 + 16 * m + l16;
-        px[m] = p % W;
-        const int t = p / W;
-        py[m] = t % H;
-        pn[m] = t / H;
+    const int wc = wave % NWC, wr = wave / NWC;
+    // neighbouring tiles to one XCD (gfx950 dispatches block b to XCD b % 8): their halos overlap
+    const int nt = gridDim.x, b = nt % 8 ? blockIdx.x : (blockIdx.x % 8) * (nt / 8) + blockIdx.x / 8;
+    int x0 = 0, y0 = 0;
+    size_t base;  // the sample's first pixel (3x3) or the block's (1x1)
+    if constexpr (TAPS == 9) {
+        const int tx = W / 16, ty = H / TY, t = b / tx, n = t / ty;
+        x0 = 16 * (b - t * tx);
+        y0 = TY * (t - n * ty);
+        base = (size_t)n * H * W;
+    } else {
+        base = (size_t)b * (16 * TY);
     }
-    f32x4 acc[MB][NB];
+
+    u32x4 sv[PER];
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int n = 0; n < NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int K = taps * cin;
-    const bf16x8 zero = {};
-    bf16x8 a[MB], b[NB];
-    auto fetch = [&](int kb, bf16x8* av, bf16x8* bv) {
-        const int k0 = kb + 8 * q;
-        if (k0 < K) {
-            const int tap = k0 / cin, ci = k0 - tap * cin;
-            int dy = 0, dx = 0;
-            if (taps == 9) {
-                dy = tap / 3 - 1;
-                dx = tap % 3 - 1;
-                if (flip) {
-                    dy = -dy;
-                    dx = -dx;
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < MB; ++m)
-                av[m] = load_a<SRC>(src, cin, pn[m], wrapi(py[m] + dy, H), wrapi(px[m] + dx, W), H, W, ci);
-#pragma unroll
-            for (int n = 0; n < NB; ++n) bv[n] = load8(w + ((size_t)tap * COUT + 16 * n + l16) * cin + ci);
+    for (int k = 0; k < PER; ++k) {
+        const int i = min(tid + NT * k, ITEMS - 1), c8 = 8 * (i % (CIN / 8)), pp = i / (CIN / 8);
+        size_t px;
+        if constexpr (TAPS == 9) {
+            const int ry = pp / PW, rx = pp - ry * PW;
+            px = base + (size_t)wrapi(y0 + ry - 1, H) * W + wrapi(x0 + rx - 1, W);
         } else {
-#pragma unroll
-            for (int m = 0; m < MB; ++m) av[m] = zero;
-#pragma unroll
-            for (int n = 0; n < NB; ++n) bv[n] = zero;
+            px = base + pp;
         }
-    };
-    fetch(0, a, b);
-    for (int kb = 0; kb < K; kb += 32) {
-        bf16x8 an[MB], bn[NB];
-        if (kb + 32 < K) fetch(kb + 32, an, bn);
+        sv[k] = load8u(in + px * CIN + c8);
+    }
+    // row r of channel block n of the wave is channel 4 NBW (r / 4) + 4 n + r % 4
+    const int cbase = 16 * NBW * wc;
+    bf16x8 wv[NS][NBW];
 #pragma unroll
-        for (int m = 0; m < MB; ++m)
+    for (int st = 0; st < NS; ++st) {
+        const int k0 = 32 * st + 8 * q, tap = k0 / CIN, ci = k0 - tap * CIN;
 #pragma unroll
-            for (int n = 0; n < NB; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[n], acc[m][n], 0, 0, 0);
-        if (kb + 32 < K) {
-#pragma unroll
-            for (int m = 0; m < MB; ++m) a[m] = an[m];
-#pragma unroll
-            for (int n = 0; n < NB; ++n) b[n] = bn[n];
+        for (int n = 0; n < NBW; ++n) {
+            const int co = cbase + 4 * NBW * (l16 >> 2) + 4 * n + (l16 & 3);
+            bf16x8 v = {};
+            if (K % 32 == 0 || k0 < K) v = load8(w + ((size_t)tap * COUT + co) * CIN + ci);
+            wv[st][n] = v;
         }
     }
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+    for (int k = 0; k < PER; ++k) {
+        const int i = tid + NT * k;
+        if (i < ITEMS) *reinterpret_cast<u32x4*>(tile + i / (CIN / 8) * LD + 8 * (i % (CIN / 8))) = sv[k];
+    }
+    const int co = cbase + 4 * NBW * q;  // the lane's 4 NBW output channels
+    f32x4 bv[NBW];
+    if constexpr (MODE == kOutBf16 || MODE == kOutBf16Gelu) {
 #pragma unroll
-        for (int n = 0; n < NB; ++n) {
-            const int co = 16 * n + l16;
-            const float bco = MODE == kOutF32 ? 0.f : bias[co];
+        for (int n = 0; n < NBW; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const size_t idx = (size_t)(pix0 + 16 * m + 4 * q + r) * COUT + co;
-                const float v = acc[m][n][r] + bco;
-                if constexpr (MODE == kOutF32) {
-                    static_cast<float*>(out)[idx] = v;
-                } else if constexpr (MODE == kOutBf16Gelu) {
-                    if (pre) pre[idx] = f2bf(v);
-                    static_cast<bf16*>(out)[idx] = f2bf(gelu(v));
-                } else {
-                    static_cast<bf16*>(out)[idx] = f2bf(v);
-                }
+            for (int e = 0; e < 4; ++e) bv[n][e] = bias[co + 4 * n + e];
+    }
+    __syncthreads();
+
+    typedef uint32_t u32xn __attribute__((ext_vector_type(2 * NBW)));
+    constexpr int RB = MR % 2 ? 1 : 2;  // rows in flight
+    for (int r0 = wr * MR; r0 < (wr + 1) * MR; r0 += RB) {
+        size_t px[RB];
+        u32xn pv[RB];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            px[r] = (TAPS == 9 ? base + (size_t)(y0 + r0 + r) * W + x0 : base + 16 * (r0 + r)) + l16;
+            if constexpr (MODE == kOutGeluBwd) pv[r] = *reinterpret_cast<const u32xn*>(pre + px[r] * COUT + co);
+        }
+        f32x4 acc[RB][NBW];
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) acc[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            // K-step st of the lane: tap and channels (a lane past K takes zeros)
+            int off;
+            if constexpr (CIN >= 32) {
+                const int tap = 32 * st / CIN, dy = TAPS == 9 ? tap / 3 : 0, dx = TAPS == 9 ? tap % 3 : 0;
+                off = ((FLIP && HALO ? 2 - dy : dy) * PW + (FLIP && HALO ? 2 - dx : dx)) * LD + 32 * st % CIN + 8 * q;
+            } else {
+                const int tap = min(2 * st + (q >> 1), TAPS - 1), dy = tap / 3, dx = tap - 3 * dy;
+                off = ((FLIP && HALO ? 2 - dy : dy) * PW + (FLIP && HALO ? 2 - dx : dx)) * LD + 8 * (q & 1);
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                bf16x8 a = *reinterpret_cast<const bf16x8*>(tile + ((r0 + r) * PW + l16) * LD + off);
+                if (32 * st + 32 > K && 32 * st + 8 * q >= K) a = bf16x8{};
+#pragma unroll
+                for (int n = 0; n < NBW; ++n)
+                    acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[st][n], a, acc[r][n], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const size_t o = px[r] * COUT + co;
+            if constexpr (MODE == kOutF32) {
+#pragma unroll
+                for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4*>(static_cast<float*>(out) + o + 4 * n) = acc[r][n];
+            } else {
+                u32xn ov, qv;
+#pragma unroll
+                for (int n = 0; n < NBW; ++n)
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        const int j = 2 * n + e / 2;
+                        if constexpr (MODE == kOutGeluBwd) {
+                            ov[j] = (uint32_t)f2bf(acc[r][n][e] * gelu_grad(lo_f(pv[r][j]))) |
+                                    ((uint32_t)f2bf(acc[r][n][e + 1] * gelu_grad(hi_f(pv[r][j]))) << 16);
+                        } else {
+                            const float v0 = acc[r][n][e] + bv[n][e], v1 = acc[r][n][e + 1] + bv[n][e + 1];
+                            qv[j] = (uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16);
+                            if constexpr (MODE == kOutBf16Gelu)
+                                ov[j] = (uint32_t)f2bf(gelu(v0)) | ((uint32_t)f2bf(gelu(v1)) << 16);
+                        }
+                    }
+                if constexpr (MODE == kOutBf16Gelu) *reinterpret_cast<u32xn*>(pre + o) = qv;
+                if constexpr (MODE == kOutBf16) ov = qv;
+                *reinterpret_cast<u32xn*>(static_cast<bf16*>(out) + o) = ov;
+            }
+        }
+    }
 }
 
 // Inference convolution (3x3, periodic) on a TY x 16 pixel tile per block.  The block
@@ -954,26 +1011,50 @@ __global__ __launch_bounds__(512) void c7_head_flux_kernel(const bf16* __restric
     }
 }
 
-// dd1[p][ci] = sum_{tap, c} dJ[p - shift(tap)][c] * wh[tap][c][ci]
-__global__ void head_bwd_data_kernel(const float* __restrict__ dJ, const float* __restrict__ wh, int H, int W, int npix,
-                                     float* __restrict__ dd1)
+// dpre[p][ci] = bf16(gelu'(pre[p][ci]) * sum_{tap, c} dJ[p - shift(tap)][c] * wh[tap][c][ci]):
+// the head's data gradient taken on to c7's pre-activation, 64 pixels a block.  Each wave sums
+// eight channels, so its weights are scalars; LDS turns the sums so that `pre` is read and dpre
+// written 16 bytes a lane in order.  Bound by those two and by the 576 multiply-adds of a pixel;
+// with the FP32 gradient stored and read back by a pass of its own this was 130 us for 16
+// samples of 256 x 256, now 42 us.
+__global__ __launch_bounds__(256) void head_bwd_data_kernel(const float* __restrict__ dJ, const float* __restrict__ wh,
+                                                            const bf16* __restrict__ pre, int H, int W,
+                                                            bf16* __restrict__ dpre)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    const int x = p % W, t = p / W, y = t % H, n = t / H;
-    float acc[32];
+    constexpr int LD = 36;  // floats of a pixel: 32 channels and padding
+    __shared__ __align__(16) float s[64 * LD];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int c0 = 8 * __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t p0 = (size_t)blockIdx.x * 64;
+    const u32x4 pv = load8u(pre + (p0 + (tid >> 2)) * 32 + 8 * (tid & 3));
+    {
+        // sides are multiples of 64: the block's pixels share a row
+        const int row = blockIdx.x * 64 / W, x = blockIdx.x * 64 - row * W + lane, y = row % H;
+        float acc[8];
 #pragma unroll
-    for (int ci = 0; ci < 32; ++ci) acc[ci] = 0.f;
-    for (int tap = 0; tap < 9; ++tap) {
-        const int yy = wrapi(y - (tap / 3 - 1), H), xx = wrapi(x - (tap % 3 - 1), W);
-        const size_t q = ((size_t)n * H + yy) * W + xx;
-        const float g0 = dJ[2 * q], g1 = dJ[2 * q + 1];
-        const float* w0 = wh + tap * 64;
+        for (int ci = 0; ci < 8; ++ci) acc[ci] = 0.f;
 #pragma unroll
-        for (int ci = 0; ci < 32; ++ci) acc[ci] = fmaf(g0, w0[ci], fmaf(g1, w0[32 + ci], acc[ci]));
+        for (int tap = 0; tap < 9; ++tap) {
+            const int yy = wrapi(y - (tap / 3 - 1), H), xx = wrapi(x - (tap % 3 - 1), W);
+            const float2 g = *reinterpret_cast<const float2*>(dJ + 2 * ((size_t)(row - y + yy) * W + xx));
+            const float* w0 = wh + tap * 64 + c0;
+#pragma unroll
+            for (int ci = 0; ci < 8; ++ci) acc[ci] = fmaf(g.x, w0[ci], fmaf(g.y, w0[32 + ci], acc[ci]));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            *reinterpret_cast<f32x4*>(s + lane * LD + c0 + 4 * h) = f32x4{acc[4 * h], acc[4 * h + 1], acc[4 * h + 2], acc[4 * h + 3]};
     }
+    __syncthreads();
+    const float* v = s + (tid >> 2) * LD + 8 * (tid & 3);
+    const f32x4 v0 = *reinterpret_cast<const f32x4*>(v), v1 = *reinterpret_cast<const f32x4*>(v + 4);
+    u32x4 r;
 #pragma unroll
-    for (int ci = 0; ci < 32; ++ci) dd1[(size_t)p * 32 + ci] = acc[ci];
+    for (int j = 0; j < 4; ++j) {
+        const float a = j < 2 ? v0[2 * j] : v1[2 * j - 4], b = j < 2 ? v0[2 * j + 1] : v1[2 * j - 3];
+        r[j] = (uint32_t)f2bf(a * gelu_grad(lo_f(pv[j]))) | ((uint32_t)f2bf(b * gelu_grad(hi_f(pv[j]))) << 16);
+    }
+    *reinterpret_cast<u32x4*>(dpre + (p0 + (tid >> 2)) * 32 + 8 * (tid & 3)) = r;
 }
 
 // part[chunk][tap*64 + c*32 + ci] = sum_p dJ[p][c] d1[p + shift(tap)][ci]; part[chunk][576 + c] = sum_p dJ[p][c]
@@ -1293,9 +1374,9 @@ struct amb_surrogate {
     // activations (bf16 NHWC) and gradients
     bf16 *x0 = nullptr, *e1 = nullptr, *e1p = nullptr, *p1 = nullptr, *e2 = nullptr, *e2p = nullptr, *p2 = nullptr;
     bf16 *bt = nullptr, *btp = nullptr, *u2 = nullptr, *s2 = nullptr, *d2 = nullptr, *d2p = nullptr, *u1 = nullptr;
-    bf16 *s1 = nullptr, *d1 = nullptr, *d1p = nullptr, *dpre = nullptr;
+    bf16 *s1 = nullptr, *d1 = nullptr, *d1p = nullptr, *dpre = nullptr, *dpre2 = nullptr;
     float *J = nullptr, *phi = nullptr, *target = nullptr, *params = nullptr, *norm = nullptr, *pred = nullptr;
-    float *g = nullptr, *dJ = nullptr, *dd1 = nullptr, *ds1 = nullptr, *dd2 = nullptr, *ds2 = nullptr, *dbt = nullptr;
+    float *g = nullptr, *dJ = nullptr, *ds1 = nullptr, *ds2 = nullptr;
     float *dp2 = nullptr, *dp1 = nullptr, *part = nullptr, *part2 = nullptr, *loss_part = nullptr,
           *sumsq_part = nullptr;
     size_t part_len = 0, part2_len = 0;
@@ -1326,9 +1407,9 @@ namespace {
 std::vector<void*> all_buffers(amb_surrogate* s)
 {
     std::vector<void*> v = {s->master, s->grad, s->adam_m, s->adam_v, s->x0, s->e1, s->e1p, s->p1, s->e2, s->e2p,
-                            s->p2, s->bt, s->btp, s->u2, s->s2, s->d2, s->d2p, s->u1, s->s1, s->d1, s->d1p, s->dpre,
-                            s->J, s->phi, s->target, s->params, s->norm, s->pred, s->g, s->dJ, s->dd1, s->ds1,
-                            s->dd2, s->ds2, s->dbt, s->dp2, s->dp1, s->part, s->part2, s->audit_part, s->audit_buf, s->p3,
+                            s->p2, s->bt, s->btp, s->u2, s->s2, s->d2, s->d2p, s->u1, s->s1, s->d1, s->d1p, s->dpre, s->dpre2,
+                            s->J, s->phi, s->target, s->params, s->norm, s->pred, s->g, s->dJ, s->ds1,
+                            s->ds2, s->dp2, s->dp1, s->part, s->part2, s->audit_part, s->audit_buf, s->p3,
                             s->loss_part, s->sumsq_part, s->d_idx,
                             s->ds_in, s->ds_out, s->ds_par, s->ds_norm, s->wf0_8};
     for (int l = 0; l < 7; ++l) {
@@ -1352,15 +1433,6 @@ void release(amb_surrogate* s)
     delete s;
 }
 
-template <int MB, int NB, int MODE, int SRC>
-hipError_t conv_launch(const ConvIn& in, int cin, const bf16* w, const float* bias, int taps, int flip, int npix, int H,
-                       int W, void* out, bf16* pre, hipStream_t st)
-{
-    hipLaunchKernelGGL((conv_kernel<MB, NB, MODE, SRC>), dim3(npix / (64 * MB)), dim3(256), 0, st, in, cin, w, bias,
-                       taps, flip, H, W, out, pre);
-    return hipGetLastError();
-}
-
 template <int SRC, int CIN, int NB, int TY, int WM, int WN, int NB2 = 0, int KW = 1>
 hipError_t conv_tile_launch(const ConvIn& in, const bf16* w, const float* bias, int n, int H, int W, bf16* out,
                             hipStream_t st, const bf16* w2 = nullptr, const float* b2 = nullptr)
@@ -1371,25 +1443,14 @@ hipError_t conv_tile_launch(const ConvIn& in, const bf16* w, const float* bias, 
     return hipGetLastError();
 }
 
-// Dispatch on output channels (16 NB); MB (16-pixel rows per wave) is 2 for large
-// launches and 1 for small.
-template <int MODE, int SRC = kSrcPlain>
-hipError_t conv(const ConvIn& in, int cin, const bf16* w, const float* bias, int cout, int taps, int flip, int npix,
-                int H, int W, void* out, bf16* pre, hipStream_t st)
+template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP = false>
+hipError_t conv_launch(const bf16* in, const bf16* w, const float* bias, int npix, int H, int W, void* out, bf16* pre,
+                       hipStream_t st)
 {
-    const bool big = npix >= 16 * 2048;
-    switch (cout) {
-    case 32:
-        return big ? conv_launch<2, 2, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st)
-                   : conv_launch<1, 2, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st);
-    case 64:
-        return big ? conv_launch<2, 4, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st)
-                   : conv_launch<1, 4, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st);
-    case 128:
-        return big ? conv_launch<2, 8, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st)
-                   : conv_launch<1, 8, MODE, SRC>(in, cin, w, bias, taps, flip, npix, H, W, out, pre, st);
-    default: return hipErrorInvalidValue;
-    }
+    if (H % 16 || W % 16 || npix % (16 * TY)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((conv_kernel<CIN, NB, TAPS, TY, NWC, NWR, MODE, FLIP>), dim3(npix / (16 * TY)),
+                       dim3(64 * NWC * NWR), 0, st, in, w, bias, H, W, out, pre);
+    return hipGetLastError();
 }
 
 ConvIn plain(const bf16* a) { return ConvIn{a, nullptr, nullptr, nullptr}; }
@@ -1489,21 +1550,21 @@ int forward(amb_surrogate* s, int n, const float* phi, const float* params, floa
     const float* M = s->master;
     hipLaunchKernelGGL(input_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, phi, params, H * W, P1, s->x0);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(conv<kOutBf16Gelu>(plain(s->x0), kCin0, s->wf[0], M + s->b_off[0], 32, 9, 0, P1, H, W, s->e1, s->e1p, st));
+    SUR_CHECK((conv_launch<kCin0, 2, 9, 16, 1, 4, kOutBf16Gelu>(s->x0, s->wf[0], M + s->b_off[0], P1, H, W, s->e1, s->e1p, st)));
     hipLaunchKernelGGL(avgpool_kernel, dim3(blocks_for((size_t)P2 * 32)), dim3(kEw), 0, st, s->e1, H, W, 32, P2 * 32, s->p1);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(conv<kOutBf16Gelu>(plain(s->p1), 32, s->wf[1], M + s->b_off[1], 64, 9, 0, P2, H2, W2, s->e2, s->e2p, st));
+    SUR_CHECK((conv_launch<32, 4, 9, 16, 2, 2, kOutBf16Gelu>(s->p1, s->wf[1], M + s->b_off[1], P2, H2, W2, s->e2, s->e2p, st)));
     hipLaunchKernelGGL(avgpool_kernel, dim3(blocks_for((size_t)P3 * 64)), dim3(kEw), 0, st, s->e2, H2, W2, 64, P3 * 64, s->p2);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(conv<kOutBf16Gelu>(plain(s->p2), 64, s->wf[2], M + s->b_off[2], 128, 9, 0, P3, H4, W4, s->bt, s->btp, st));
-    SUR_CHECK(conv<kOutBf16>(plain(s->bt), 128, s->wf[3], M + s->b_off[3], 64, 1, 0, P3, H4, W4, s->u2, nullptr, st));
+    SUR_CHECK((conv_launch<64, 8, 9, 8, 8, 1, kOutBf16Gelu>(s->p2, s->wf[2], M + s->b_off[2], P3, H4, W4, s->bt, s->btp, st)));
+    SUR_CHECK((conv_launch<128, 4, 1, 8, 2, 2, kOutBf16>(s->bt, s->wf[3], M + s->b_off[3], P3, H4, W4, s->u2, nullptr, st)));
     hipLaunchKernelGGL(upadd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->u2, s->e2, H2, W2, 64, P2 * 64, s->s2);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(conv<kOutBf16Gelu>(plain(s->s2), 64, s->wf[4], M + s->b_off[4], 64, 9, 0, P2, H2, W2, s->d2, s->d2p, st));
-    SUR_CHECK(conv<kOutBf16>(plain(s->d2), 64, s->wf[5], M + s->b_off[5], 32, 1, 0, P2, H2, W2, s->u1, nullptr, st));
+    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutBf16Gelu>(s->s2, s->wf[4], M + s->b_off[4], P2, H2, W2, s->d2, s->d2p, st)));
+    SUR_CHECK((conv_launch<64, 2, 1, 16, 1, 4, kOutBf16>(s->d2, s->wf[5], M + s->b_off[5], P2, H2, W2, s->u1, nullptr, st)));
     hipLaunchKernelGGL(upadd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->u1, s->e1, H, W, 32, P1 * 32, s->s1);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(conv<kOutBf16Gelu>(plain(s->s1), 32, s->wf[6], M + s->b_off[6], 32, 9, 0, P1, H, W, s->d1, s->d1p, st));
+    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutBf16Gelu>(s->s1, s->wf[6], M + s->b_off[6], P1, H, W, s->d1, s->d1p, st)));
     hipLaunchKernelGGL(head_fwd_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, s->d1, M + s->w_off[7], M + s->b_off[7],
                        H, W, P1, J);
     SUR_CHECK(hipGetLastError());
@@ -1557,43 +1618,37 @@ int loss_and_grad(amb_surrogate* s, int n, double* loss_out)
     hipLaunchKernelGGL(dj_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, s->g, H, W, P1, s->dJ);
     SUR_CHECK(hipGetLastError());
     // head
-    hipLaunchKernelGGL(head_bwd_data_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, s->dJ, M + s->w_off[7], H, W, P1,
-                       s->dd1);
+    hipLaunchKernelGGL(head_bwd_data_kernel, dim3(P1 / 64), dim3(256), 0, st, s->dJ, M + s->w_off[7], s->d1p, H, W,
+                       s->dpre);
     const int hch = P1 / kHeadChunk;
     hipLaunchKernelGGL(head_bwd_weight_kernel, dim3(blocks_for(hch, 4)), dim3(256), 0, st, s->dJ, s->d1, H, W, hch,
                        s->part);
     SUR_CHECK(hipGetLastError());
     SUR_CHECK(reduce_parts(s, hch, 578, s->grad + s->w_off[7]));
     // c7 (in s1), then s1 = up(u1) + e1
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->dd1, nullptr, s->d1p,
-                       H, W, 32, P1 * 32, s->dpre);
     if ((rc = layer_grads(s, 6, s->dpre, s->s1, H, W, P1)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 32, s->wb[6], nullptr, 32, 9, 1, P1, H, W, s->ds1, nullptr, st));
+    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutF32, true>(s->dpre, s->wb[6], nullptr, P1, H, W, s->ds1, nullptr, st)));
     hipLaunchKernelGGL(sumpool_kernel, dim3(blocks_for((size_t)P2 * 32)), dim3(kEw), 0, st, s->ds1, H, W, 32, P2 * 32,
                        s->dpre);
     // c6 (1x1, in d2)
     if ((rc = layer_grads(s, 5, s->dpre, s->d2, H2, W2, P2)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 32, s->wb[5], nullptr, 64, 1, 1, P2, H2, W2, s->dd2, nullptr, st));
     // c5 (in s2), then s2 = up(u2) + e2
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->dd2, nullptr, s->d2p,
-                       H2, W2, 64, P2 * 64, s->dpre);
-    if ((rc = layer_grads(s, 4, s->dpre, s->s2, H2, W2, P2)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 64, s->wb[4], nullptr, 64, 9, 1, P2, H2, W2, s->ds2, nullptr, st));
+    SUR_CHECK((conv_launch<32, 4, 1, 16, 2, 2, kOutGeluBwd>(s->dpre, s->wb[5], nullptr, P2, H2, W2, s->dpre2, s->d2p, st)));
+    if ((rc = layer_grads(s, 4, s->dpre2, s->s2, H2, W2, P2)) != AMB_OK) return rc;
+    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutF32, true>(s->dpre2, s->wb[4], nullptr, P2, H2, W2, s->ds2, nullptr, st)));
     hipLaunchKernelGGL(sumpool_kernel, dim3(blocks_for((size_t)P3 * 64)), dim3(kEw), 0, st, s->ds2, H2, W2, 64, P3 * 64,
                        s->dpre);
     // c4 (1x1, in bt)
     if ((rc = layer_grads(s, 3, s->dpre, s->bt, H4, W4, P3)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 64, s->wb[3], nullptr, 128, 1, 1, P3, H4, W4, s->dbt, nullptr, st));
     // c3 (in p2)
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P3 * 128)), dim3(kEw), 0, st, s->dbt, nullptr, s->btp,
-                       H4, W4, 128, P3 * 128, s->dpre);
-    if ((rc = layer_grads(s, 2, s->dpre, s->p2, H4, W4, P3)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 128, s->wb[2], nullptr, 64, 9, 1, P3, H4, W4, s->dp2, nullptr, st));
+    SUR_CHECK((conv_launch<64, 8, 1, 8, 4, 1, kOutGeluBwd>(s->dpre, s->wb[3], nullptr, P3, H4, W4, s->dpre2, s->btp, st)));
+    if ((rc = layer_grads(s, 2, s->dpre2, s->p2, H4, W4, P3)) != AMB_OK) return rc;
+    SUR_CHECK((conv_launch<128, 4, 9, 8, 4, 1, kOutF32, true>(s->dpre2, s->wb[2], nullptr, P3, H4, W4, s->dp2, nullptr, st)));
     // c2 (in p1): de2 = ds2 + pool_grad(dp2)
     hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->ds2, s->dp2, s->e2p,
                        H2, W2, 64, P2 * 64, s->dpre);
     if ((rc = layer_grads(s, 1, s->dpre, s->p1, H2, W2, P2)) != AMB_OK) return rc;
-    SUR_CHECK(conv<kOutF32>(plain(s->dpre), 64, s->wb[1], nullptr, 32, 9, 1, P2, H2, W2, s->dp1, nullptr, st));
+    SUR_CHECK((conv_launch<64, 2, 9, 16, 2, 2, kOutF32, true>(s->dpre, s->wb[1], nullptr, P2, H2, W2, s->dp1, nullptr, st)));
     // c1 (in x0): de1 = ds1 + pool_grad(dp1)
     hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->ds1, s->dp1, s->e1p,
                        H, W, 32, P1 * 32, s->dpre);
@@ -1740,6 +1795,7 @@ int amb_surrogate_create(int64_t ny, int64_t nx, int max_batch, uint64_t seed, a
     A(&s->d1, P1 * 32 * 2);
     A(&s->d1p, P1 * 32 * 2);
     A(&s->dpre, P1 * 32 * 2);
+    A(&s->dpre2, P2 * 64 * 2);
     A(&s->J, P1 * 2 * 4);
     A(&s->phi, P1 * 4);
     A(&s->target, P1 * 4);
@@ -1748,11 +1804,8 @@ int amb_surrogate_create(int64_t ny, int64_t nx, int max_batch, uint64_t seed, a
     A(&s->pred, P1 * 4);
     A(&s->g, P1 * 4);
     A(&s->dJ, P1 * 2 * 4);
-    A(&s->dd1, P1 * 32 * 4);
     A(&s->ds1, P1 * 32 * 4);
-    A(&s->dd2, P2 * 64 * 4);
     A(&s->ds2, P2 * 64 * 4);
-    A(&s->dbt, P3 * 128 * 4);
     A(&s->dp2, P3 * 64 * 4);
     A(&s->dp1, P2 * 32 * 4);
     A(&s->part, s->part_len * 4);
