@@ -85,7 +85,7 @@ __device__ __forceinline__ float hi_f(uint32_t w) { return __uint_as_float(w & 0
 
 // ---- convolution forward / backward-data --------------------------------------------
 
-enum ConvMode { kOutBf16 = 0, kOutBf16Gelu = 1, kOutF32 = 2, kOutGeluBwd = 3 };
+enum ConvMode { kOutBf16, kOutBf16Gelu, kOutBf16GeluPool, kOutF32, kOutF32SumPool, kOutGeluBwd };
 // Where the A operand comes from: a plain NHWC tensor; the 2x2 average of a tensor of
 // twice the resolution (fused avgpool); up2(coarse) + skip (fused up-sampling add);
 // or the network input assembled from phi and the parameters (fused input layer).
@@ -143,7 +143,11 @@ __device__ __forceinline__ bf16x8 load_a(const ConvIn& src, int cin, int n, int 
 // Training convolution: out[p][co] = bias[co] + sum_{tap, ci} in[p + shift(tap)][ci] *
 // w[tap][co][ci] (FLIP: shift negated, the data gradient with the [tap][cin][cout] layout),
 // then MODE: bfloat16 (pre-activation and GELU of it; or the sum itself), FP32, or bfloat16
-// of the sum times gelu'(pre), the gradient at a pre-activation `pre`.
+// of the sum times gelu'(pre), the gradient at a pre-activation `pre`.  The Pool modes also
+// write the 2x2 means (forward) or sums (backward of the up-sampling) to `pooled`, from the
+// rows' registers and the neighbouring lane: 74 us for the four in passes of their own, now 8 us.
+// UPADD: the input is up2(coarse) + skip, formed while staging and written to `sum` for the
+// weight gradient; 140 us for the two in passes of their own, now 32 us.
 //
 // A block takes TY x 16 pixels: the padded input tile is staged in LDS once for all taps and
 // all output channels, and each of the NWC x NWR waves holds the weights of its NB / NWC
@@ -153,16 +157,40 @@ __device__ __forceinline__ bf16x8 load_a(const ConvIn& src, int cin, int n, int 
 // is mostly the activations' trip to and from memory.  Reading both operands from global
 // memory at every K-step and storing two bytes at a time, the twelve convolutions, and the
 // passes that applied gelu' to their FP32 results, took 780 us for 16 samples of 256 x 256,
-// now 345 us.  The sum runs over K in the same 32-wide steps as the inference kernels'.
-template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP>
-__global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __restrict__ in, const bf16* __restrict__ w,
-                                                              const float* __restrict__ bias, int H, int W,
-                                                              void* __restrict__ out, bf16* __restrict__ pre)
+// now 345 us (without pooling and up-sampling).  The sum runs over K in the same 32-wide steps as the inference kernels'.
+struct ConvTrain {
+    const bf16* in;    // UPADD: the skip tensor
+    const bf16* coarse = nullptr;
+    bf16* sum = nullptr;
+    const bf16* w;
+    const float* bias = nullptr;
+    void* out;
+    bf16* pre = nullptr;
+    bf16* pooled = nullptr;
+};
+
+// value of lane ^ 1 (DPP quad_perm 1, 0, 3, 2)
+__device__ __forceinline__ float swap1(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
+}
+
+template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP, bool UPADD>
+__global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const ConvTrain arg, int H, int W)
 {
     constexpr int COUT = 16 * NB, K = TAPS * CIN, NS = (K + 31) / 32, NBW = NB / NWC, MR = TY / NWR;
     constexpr int HALO = TAPS == 9 ? 1 : 0, PW = 16 + 2 * HALO, PH = TY + 2 * HALO, LD = CIN + 8;
     constexpr int NT = 64 * NWC * NWR, ITEMS = PH * PW * (CIN / 8), PER = (ITEMS + NT - 1) / NT;
+    constexpr bool POOL = MODE == kOutBf16GeluPool || MODE == kOutF32SumPool;
+    constexpr bool GELU = MODE == kOutBf16Gelu || MODE == kOutBf16GeluPool;
+    constexpr bool F32 = MODE == kOutF32 || MODE == kOutF32SumPool;
     static_assert(NB % NWC == 0 && TY % NWR == 0 && CIN % 16 == 0, "tile shape");
+    static_assert(!POOL || (TAPS == 9 && MR % 2 == 0), "pooled rows come in pairs");
+    const bf16* __restrict__ in = arg.in;
+    const bf16* __restrict__ w = arg.w;
+    const float* __restrict__ bias = arg.bias;
+    void* __restrict__ out = arg.out;
+    bf16* __restrict__ pre = arg.pre;
     __shared__ __align__(16) bf16 tile[PH * PW * LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane >> 4, l16 = lane & 15;
@@ -171,8 +199,10 @@ __global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __rest
     const int nt = gridDim.x, b = nt % 8 ? blockIdx.x : (blockIdx.x % 8) * (nt / 8) + blockIdx.x / 8;
     int x0 = 0, y0 = 0;
     size_t base;  // the sample's first pixel (3x3) or the block's (1x1)
+    int n = 0;
     if constexpr (TAPS == 9) {
-        const int tx = W / 16, ty = H / TY, t = b / tx, n = t / ty;
+        const int tx = W / 16, ty = H / TY, t = b / tx;
+        n = t / ty;
         x0 = 16 * (b - t * tx);
         y0 = TY * (t - n * ty);
         base = (size_t)n * H * W;
@@ -180,14 +210,17 @@ __global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __rest
         base = (size_t)b * (16 * TY);
     }
 
-    u32x4 sv[PER];
+    u32x4 sv[PER], uv[UPADD ? PER : 1];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int i = min(tid + NT * k, ITEMS - 1), c8 = 8 * (i % (CIN / 8)), pp = i / (CIN / 8);
         size_t px;
         if constexpr (TAPS == 9) {
             const int ry = pp / PW, rx = pp - ry * PW;
-            px = base + (size_t)wrapi(y0 + ry - 1, H) * W + wrapi(x0 + rx - 1, W);
+            const int y = wrapi(y0 + ry - 1, H), x = wrapi(x0 + rx - 1, W);
+            px = base + (size_t)y * W + x;
+            if constexpr (UPADD)
+                uv[k] = load8u(arg.coarse + (((size_t)n * (H / 2) + y / 2) * (W / 2) + x / 2) * CIN + c8);
         } else {
             px = base + pp;
         }
@@ -210,11 +243,20 @@ __global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __rest
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int i = tid + NT * k;
+        if constexpr (UPADD) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                sv[k][j] = (uint32_t)f2bf(lo_f(uv[k][j]) + lo_f(sv[k][j])) |
+                           ((uint32_t)f2bf(hi_f(uv[k][j]) + hi_f(sv[k][j])) << 16);
+            const int c8 = 8 * (i % (CIN / 8)), pp = i / (CIN / 8), ry = pp / PW - 1, rx = pp % PW - 1;
+            if (i < ITEMS && ry >= 0 && ry < TY && rx >= 0 && rx < 16)
+                *reinterpret_cast<u32x4*>(arg.sum + (base + (size_t)(y0 + ry) * W + x0 + rx) * CIN + c8) = sv[k];
+        }
         if (i < ITEMS) *reinterpret_cast<u32x4*>(tile + i / (CIN / 8) * LD + 8 * (i % (CIN / 8))) = sv[k];
     }
     const int co = cbase + 4 * NBW * q;  // the lane's 4 NBW output channels
     f32x4 bv[NBW];
-    if constexpr (MODE == kOutBf16 || MODE == kOutBf16Gelu) {
+    if constexpr (MODE == kOutBf16 || GELU) {
 #pragma unroll
         for (int n = 0; n < NBW; ++n)
 #pragma unroll
@@ -257,33 +299,50 @@ __global__ __launch_bounds__(64 * NWC * NWR) void conv_kernel(const bf16* __rest
                     acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[st][n], a, acc[r][n], 0, 0, 0);
             }
         }
+        u32xn ov[RB];
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             const size_t o = px[r] * COUT + co;
-            if constexpr (MODE == kOutF32) {
+            if constexpr (F32) {
 #pragma unroll
                 for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4*>(static_cast<float*>(out) + o + 4 * n) = acc[r][n];
             } else {
-                u32xn ov, qv;
+                u32xn qv;
 #pragma unroll
                 for (int n = 0; n < NBW; ++n)
 #pragma unroll
                     for (int e = 0; e < 4; e += 2) {
                         const int j = 2 * n + e / 2;
                         if constexpr (MODE == kOutGeluBwd) {
-                            ov[j] = (uint32_t)f2bf(acc[r][n][e] * gelu_grad(lo_f(pv[r][j]))) |
-                                    ((uint32_t)f2bf(acc[r][n][e + 1] * gelu_grad(hi_f(pv[r][j]))) << 16);
+                            ov[r][j] = (uint32_t)f2bf(acc[r][n][e] * gelu_grad(lo_f(pv[r][j]))) |
+                                       ((uint32_t)f2bf(acc[r][n][e + 1] * gelu_grad(hi_f(pv[r][j]))) << 16);
                         } else {
                             const float v0 = acc[r][n][e] + bv[n][e], v1 = acc[r][n][e + 1] + bv[n][e + 1];
                             qv[j] = (uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16);
-                            if constexpr (MODE == kOutBf16Gelu)
-                                ov[j] = (uint32_t)f2bf(gelu(v0)) | ((uint32_t)f2bf(gelu(v1)) << 16);
+                            if constexpr (GELU) ov[r][j] = (uint32_t)f2bf(gelu(v0)) | ((uint32_t)f2bf(gelu(v1)) << 16);
                         }
                     }
-                if constexpr (MODE == kOutBf16Gelu) *reinterpret_cast<u32xn*>(pre + o) = qv;
-                if constexpr (MODE == kOutBf16) ov = qv;
-                *reinterpret_cast<u32xn*>(static_cast<bf16*>(out) + o) = ov;
+                if constexpr (GELU) *reinterpret_cast<u32xn*>(pre + o) = qv;
+                if constexpr (MODE == kOutBf16) ov[r] = qv;
+                *reinterpret_cast<u32xn*>(static_cast<bf16*>(out) + o) = ov[r];
             }
+        }
+        if constexpr (POOL) {
+            u32xn pl;
+            auto pool2 = [](float a, float b) { return a + swap1(a) + b + swap1(b); };  // even lanes: the 2x2 in row order
+#pragma unroll
+            for (int j = 0; j < 2 * NBW; ++j) {
+                if constexpr (F32) {
+                    const int n = j / 2, e = 2 * (j % 2);
+                    pl[j] = (uint32_t)f2bf(pool2(acc[0][n][e], acc[1][n][e])) |
+                            ((uint32_t)f2bf(pool2(acc[0][n][e + 1], acc[1][n][e + 1])) << 16);
+                } else {
+                    pl[j] = (uint32_t)f2bf(0.25f * pool2(lo_f(ov[0][j]), lo_f(ov[1][j]))) |
+                            ((uint32_t)f2bf(0.25f * pool2(hi_f(ov[0][j]), hi_f(ov[1][j]))) << 16);
+                }
+            }
+            const size_t o = ((size_t)n * (H / 2) + (y0 + r0) / 2) * (W / 2) + (x0 + l16) / 2;
+            if (!(l16 & 1)) *reinterpret_cast<u32xn*>(arg.pooled + o * COUT + co) = pl;
         }
     }
 }
@@ -788,40 +847,6 @@ __global__ void input_kernel(const float* __restrict__ phi, const float* __restr
     dst[3] = f2bf(params[3 * n + 2] / kParamScale[2]);
     dst[4] = f2bf((phi[p] - bf2f(f2bf(phi[p]))) * kLoScale);
     for (int c = kCinReal; c < kCin0; ++c) dst[c] = 0;
-}
-
-// out (N, H/2, W/2, C) = mean of 2x2 blocks of in (N, H, W, C).
-__global__ void avgpool_kernel(const bf16* __restrict__ in, int H, int W, int C, int nout, bf16* __restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nout) return;
-    const int c = i % C, t = i / C, Wo = W / 2, Ho = H / 2;
-    const int x = t % Wo, t2 = t / Wo, y = t2 % Ho, n = t2 / Ho;
-    const size_t base = (((size_t)n * H + 2 * y) * W + 2 * x) * C + c;
-    const float s = bf2f(in[base]) + bf2f(in[base + C]) + bf2f(in[base + (size_t)W * C]) + bf2f(in[base + (size_t)W * C + C]);
-    out[i] = f2bf(0.25f * s);
-}
-
-// s (N, H, W, C) = up2(u) + skip, u of size (N, H/2, W/2, C).
-__global__ void upadd_kernel(const bf16* __restrict__ u, const bf16* __restrict__ skip, int H, int W, int C, int n,
-                             bf16* __restrict__ s)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = i % C, t = i / C, x = t % W, t2 = t / W, y = t2 % H, b = t2 / H;
-    const float v = bf2f(u[(((size_t)b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c]) + bf2f(skip[i]);
-    s[i] = f2bf(v);
-}
-
-// Up-sampling backward: out (N, H/2, W/2, C) bf16 = sum of the 2x2 block of g.
-__global__ void sumpool_kernel(const float* __restrict__ g, int H, int W, int C, int nout, bf16* __restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nout) return;
-    const int c = i % C, t = i / C, Wo = W / 2, Ho = H / 2;
-    const int x = t % Wo, t2 = t / Wo, y = t2 % Ho, b = t2 / Ho;
-    const size_t base = (((size_t)b * H + 2 * y) * W + 2 * x) * C + c;
-    out[i] = f2bf(g[base] + g[base + C] + g[base + (size_t)W * C] + g[base + (size_t)W * C + C]);
 }
 
 // dpre = bf16((g + pool_grad) * gelu'(pre)); pool_grad(i) = gc[coarse(i)] / 4 when gc is given.
@@ -1443,13 +1468,12 @@ hipError_t conv_tile_launch(const ConvIn& in, const bf16* w, const float* bias, 
     return hipGetLastError();
 }
 
-template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP = false>
-hipError_t conv_launch(const bf16* in, const bf16* w, const float* bias, int npix, int H, int W, void* out, bf16* pre,
-                       hipStream_t st)
+template <int CIN, int NB, int TAPS, int TY, int NWC, int NWR, int MODE, bool FLIP = false, bool UPADD = false>
+hipError_t conv_launch(const ConvTrain& arg, int npix, int H, int W, hipStream_t st)
 {
     if (H % 16 || W % 16 || npix % (16 * TY)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((conv_kernel<CIN, NB, TAPS, TY, NWC, NWR, MODE, FLIP>), dim3(npix / (16 * TY)),
-                       dim3(64 * NWC * NWR), 0, st, in, w, bias, H, W, out, pre);
+    hipLaunchKernelGGL((conv_kernel<CIN, NB, TAPS, TY, NWC, NWR, MODE, FLIP, UPADD>), dim3(npix / (16 * TY)),
+                       dim3(64 * NWC * NWR), 0, st, arg, H, W);
     return hipGetLastError();
 }
 
@@ -1550,21 +1574,23 @@ int forward(amb_surrogate* s, int n, const float* phi, const float* params, floa
     const float* M = s->master;
     hipLaunchKernelGGL(input_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, phi, params, H * W, P1, s->x0);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK((conv_launch<kCin0, 2, 9, 16, 1, 4, kOutBf16Gelu>(s->x0, s->wf[0], M + s->b_off[0], P1, H, W, s->e1, s->e1p, st)));
-    hipLaunchKernelGGL(avgpool_kernel, dim3(blocks_for((size_t)P2 * 32)), dim3(kEw), 0, st, s->e1, H, W, 32, P2 * 32, s->p1);
-    SUR_CHECK(hipGetLastError());
-    SUR_CHECK((conv_launch<32, 4, 9, 16, 2, 2, kOutBf16Gelu>(s->p1, s->wf[1], M + s->b_off[1], P2, H2, W2, s->e2, s->e2p, st)));
-    hipLaunchKernelGGL(avgpool_kernel, dim3(blocks_for((size_t)P3 * 64)), dim3(kEw), 0, st, s->e2, H2, W2, 64, P3 * 64, s->p2);
-    SUR_CHECK(hipGetLastError());
-    SUR_CHECK((conv_launch<64, 8, 9, 8, 8, 1, kOutBf16Gelu>(s->p2, s->wf[2], M + s->b_off[2], P3, H4, W4, s->bt, s->btp, st)));
-    SUR_CHECK((conv_launch<128, 4, 1, 8, 2, 2, kOutBf16>(s->bt, s->wf[3], M + s->b_off[3], P3, H4, W4, s->u2, nullptr, st)));
-    hipLaunchKernelGGL(upadd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->u2, s->e2, H2, W2, 64, P2 * 64, s->s2);
-    SUR_CHECK(hipGetLastError());
-    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutBf16Gelu>(s->s2, s->wf[4], M + s->b_off[4], P2, H2, W2, s->d2, s->d2p, st)));
-    SUR_CHECK((conv_launch<64, 2, 1, 16, 1, 4, kOutBf16>(s->d2, s->wf[5], M + s->b_off[5], P2, H2, W2, s->u1, nullptr, st)));
-    hipLaunchKernelGGL(upadd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->u1, s->e1, H, W, 32, P1 * 32, s->s1);
-    SUR_CHECK(hipGetLastError());
-    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutBf16Gelu>(s->s1, s->wf[6], M + s->b_off[6], P1, H, W, s->d1, s->d1p, st)));
+    const auto wb = [&](ConvTrain c, int l) {
+        c.w = s->wf[l];
+        c.bias = M + s->b_off[l];
+        return c;
+    };
+    SUR_CHECK((conv_launch<kCin0, 2, 9, 16, 1, 4, kOutBf16GeluPool>(
+        wb({.in = s->x0, .out = s->e1, .pre = s->e1p, .pooled = s->p1}, 0), P1, H, W, st)));
+    SUR_CHECK((conv_launch<32, 4, 9, 16, 2, 2, kOutBf16GeluPool>(
+        wb({.in = s->p1, .out = s->e2, .pre = s->e2p, .pooled = s->p2}, 1), P2, H2, W2, st)));
+    SUR_CHECK((conv_launch<64, 8, 9, 8, 8, 1, kOutBf16Gelu>(wb({.in = s->p2, .out = s->bt, .pre = s->btp}, 2), P3, H4,
+                                                            W4, st)));
+    SUR_CHECK((conv_launch<128, 4, 1, 8, 2, 2, kOutBf16>(wb({.in = s->bt, .out = s->u2}, 3), P3, H4, W4, st)));
+    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutBf16Gelu, false, true>(
+        wb({.in = s->e2, .coarse = s->u2, .sum = s->s2, .out = s->d2, .pre = s->d2p}, 4), P2, H2, W2, st)));
+    SUR_CHECK((conv_launch<64, 2, 1, 16, 1, 4, kOutBf16>(wb({.in = s->d2, .out = s->u1}, 5), P2, H2, W2, st)));
+    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutBf16Gelu, false, true>(
+        wb({.in = s->e1, .coarse = s->u1, .sum = s->s1, .out = s->d1, .pre = s->d1p}, 6), P1, H, W, st)));
     hipLaunchKernelGGL(head_fwd_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, s->d1, M + s->w_off[7], M + s->b_off[7],
                        H, W, P1, J);
     SUR_CHECK(hipGetLastError());
@@ -1627,28 +1653,30 @@ int loss_and_grad(amb_surrogate* s, int n, double* loss_out)
     SUR_CHECK(reduce_parts(s, hch, 578, s->grad + s->w_off[7]));
     // c7 (in s1), then s1 = up(u1) + e1
     if ((rc = layer_grads(s, 6, s->dpre, s->s1, H, W, P1)) != AMB_OK) return rc;
-    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutF32, true>(s->dpre, s->wb[6], nullptr, P1, H, W, s->ds1, nullptr, st)));
-    hipLaunchKernelGGL(sumpool_kernel, dim3(blocks_for((size_t)P2 * 32)), dim3(kEw), 0, st, s->ds1, H, W, 32, P2 * 32,
-                       s->dpre);
+    SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutF32SumPool, true>(
+        {.in = s->dpre, .w = s->wb[6], .out = s->ds1, .pooled = s->dpre2}, P1, H, W, st)));
     // c6 (1x1, in d2)
-    if ((rc = layer_grads(s, 5, s->dpre, s->d2, H2, W2, P2)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, 5, s->dpre2, s->d2, H2, W2, P2)) != AMB_OK) return rc;
     // c5 (in s2), then s2 = up(u2) + e2
-    SUR_CHECK((conv_launch<32, 4, 1, 16, 2, 2, kOutGeluBwd>(s->dpre, s->wb[5], nullptr, P2, H2, W2, s->dpre2, s->d2p, st)));
-    if ((rc = layer_grads(s, 4, s->dpre2, s->s2, H2, W2, P2)) != AMB_OK) return rc;
-    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutF32, true>(s->dpre2, s->wb[4], nullptr, P2, H2, W2, s->ds2, nullptr, st)));
-    hipLaunchKernelGGL(sumpool_kernel, dim3(blocks_for((size_t)P3 * 64)), dim3(kEw), 0, st, s->ds2, H2, W2, 64, P3 * 64,
-                       s->dpre);
+    SUR_CHECK((conv_launch<32, 4, 1, 16, 2, 2, kOutGeluBwd>({.in = s->dpre2, .w = s->wb[5], .out = s->dpre, .pre = s->d2p},
+                                                            P2, H2, W2, st)));
+    if ((rc = layer_grads(s, 4, s->dpre, s->s2, H2, W2, P2)) != AMB_OK) return rc;
+    SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutF32SumPool, true>(
+        {.in = s->dpre, .w = s->wb[4], .out = s->ds2, .pooled = s->dpre2}, P2, H2, W2, st)));
     // c4 (1x1, in bt)
-    if ((rc = layer_grads(s, 3, s->dpre, s->bt, H4, W4, P3)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, 3, s->dpre2, s->bt, H4, W4, P3)) != AMB_OK) return rc;
     // c3 (in p2)
-    SUR_CHECK((conv_launch<64, 8, 1, 8, 4, 1, kOutGeluBwd>(s->dpre, s->wb[3], nullptr, P3, H4, W4, s->dpre2, s->btp, st)));
-    if ((rc = layer_grads(s, 2, s->dpre2, s->p2, H4, W4, P3)) != AMB_OK) return rc;
-    SUR_CHECK((conv_launch<128, 4, 9, 8, 4, 1, kOutF32, true>(s->dpre2, s->wb[2], nullptr, P3, H4, W4, s->dp2, nullptr, st)));
+    SUR_CHECK((conv_launch<64, 8, 1, 8, 4, 1, kOutGeluBwd>({.in = s->dpre2, .w = s->wb[3], .out = s->dpre, .pre = s->btp},
+                                                           P3, H4, W4, st)));
+    if ((rc = layer_grads(s, 2, s->dpre, s->p2, H4, W4, P3)) != AMB_OK) return rc;
+    SUR_CHECK((conv_launch<128, 4, 9, 8, 4, 1, kOutF32, true>({.in = s->dpre, .w = s->wb[2], .out = s->dp2}, P3, H4, W4,
+                                                              st)));
     // c2 (in p1): de2 = ds2 + pool_grad(dp2)
     hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->ds2, s->dp2, s->e2p,
                        H2, W2, 64, P2 * 64, s->dpre);
     if ((rc = layer_grads(s, 1, s->dpre, s->p1, H2, W2, P2)) != AMB_OK) return rc;
-    SUR_CHECK((conv_launch<64, 2, 9, 16, 2, 2, kOutF32, true>(s->dpre, s->wb[1], nullptr, P2, H2, W2, s->dp1, nullptr, st)));
+    SUR_CHECK((conv_launch<64, 2, 9, 16, 2, 2, kOutF32, true>({.in = s->dpre, .w = s->wb[1], .out = s->dp1}, P2, H2, W2,
+                                                              st)));
     // c1 (in x0): de1 = ds1 + pool_grad(dp1)
     hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->ds1, s->dp1, s->e1p,
                        H, W, 32, P1 * 32, s->dpre);
