@@ -800,36 +800,91 @@ __global__ __launch_bounds__(64 * NW) void wgrad_kernel(const bf16* __restrict__
     }
 }
 
-// Bias gradient partials: part[chunk][co] = sum_{p in chunk} dpre[p][co]; threads
-// read consecutive channels of consecutive pixels (coalesced), then reduce in LDS.
-__global__ __launch_bounds__(256) void bgrad_kernel(const bf16* __restrict__ dpre, int cout, int chunk,
-                                                    float* __restrict__ part)
+// Bias gradient partials: part[chunk][co] = sum of dpre[p][co] over the 256 pixels of chunk c.
+// 32 threads a chunk, eight channels (16 bytes) a thread, 16 to 32 loads in flight: a chain of adds
+// per channel and row, so the time is the loads'.  Two bytes a thread and load took 138 us
+// over the seven layers (16 samples of 256 x 256), now 55 us.
+constexpr int kBiasChunk = 256;
+
+template <int COUT>
+__global__ __launch_bounds__(64) void bgrad_kernel(const bf16* __restrict__ dpre, int nchunks, float* __restrict__ part)
 {
-    __shared__ float red[256];
-    const int c = blockIdx.x, co = threadIdx.x % cout, row = threadIdx.x / cout, rows = 256 / cout;
-    float s = 0.f;
-    for (int p = c * chunk + row; p < (c + 1) * chunk; p += rows) s += bf2f(dpre[(size_t)p * cout + co]);
-    red[threadIdx.x] = s;
+    constexpr int ROWS = 256 / COUT, V = COUT / 8, LD = COUT + 4;
+    __shared__ __align__(16) float red[2][ROWS * LD];
+    const int half = threadIdx.x >> 5, sub = threadIdx.x & 31, row = sub / V, c8 = 8 * (sub % V);
+    const int c = blockIdx.x * 2 + half, cc = min(c, nchunks - 1);
+    const bf16* src = dpre + ((size_t)cc * kBiasChunk + row) * COUT + c8;
+    float a[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] = 0.f;
+    constexpr int Q = 16, NQ = kBiasChunk / ROWS / Q;  // loads of a batch, batches
+    u32x4 v[2][Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) v[0][k] = load8u(src + (size_t)k * ROWS * COUT);
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) {
+        if (b + 1 < NQ) {
+#pragma unroll
+            for (int k = 0; k < Q; ++k) v[(b + 1) & 1][k] = load8u(src + (size_t)((b + 1) * Q + k) * ROWS * COUT);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // a batch's loads go out before the adds of the one before
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                a[2 * j] += lo_f(v[b & 1][k][j]);
+                a[2 * j + 1] += hi_f(v[b & 1][k][j]);
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) red[half][row * LD + c8 + j] = a[j];
     __syncthreads();
-    if (threadIdx.x < cout) {
+    if (c >= nchunks) return;
+    for (int co = sub; co < COUT; co += 32) {
         float t = 0.f;
-        for (int r = 0; r < rows; ++r) t += red[r * cout + threadIdx.x];
-        part[(size_t)c * cout + threadIdx.x] = t;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) t += red[half][r * LD + co];
+        part[(size_t)c * COUT + co] = t;
     }
 }
 
-// out[g * len + i] = sum of part[c * len + i] over chunks c of group g (gsize chunks
-// per group, blockIdx.y = g); fixed order, deterministic.
-__global__ void reduce_chunks_kernel(const float* __restrict__ part, int nchunks, int len, int gsize,
-                                     float* __restrict__ out)
+// Sums of partials, all gradients of an iteration in two launches (one per layer and level
+// took 25 launches and 117 us, now 21 us): out[i] = sum over an item's chunks of
+// part[c * len + i], one pass for up to kReduceGroup chunks, else groups of that many into
+// `mid` and then the groups: fixed order, deterministic.
+constexpr int kReduceGroup = 64;  // chunks summed per thread in each level
+
+struct ReduceItem {
+    const float* part;
+    float* mid;
+    float* out;
+    int nchunks, len, groups;
+    int block[2];  // first block of the item in each level
+};
+
+struct ReduceSet {
+    static constexpr int kMax = 16;
+    ReduceItem item[kMax];
+    int count = 0, blocks[2] = {0, 0};
+};
+
+template <int LEVEL>
+__global__ __launch_bounds__(256) void reduce_kernel(const ReduceSet set)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= len) return;
-    const int c0 = blockIdx.y * gsize, c1 = min(nchunks, c0 + gsize);
+    int k = 0;
+    while (k + 1 < set.count && (int)blockIdx.x >= set.item[k + 1].block[LEVEL]) ++k;
+    const ReduceItem& it = set.item[k];
+    const int per = (it.len + 255) / 256, b = blockIdx.x - it.block[LEVEL], g = b / per;
+    const int i = (b - g * per) * 256 + threadIdx.x;
+    if (i >= it.len) return;
+    const float* src = LEVEL == 0 ? it.part : it.mid;
+    const int n = LEVEL == 0 ? it.nchunks : it.groups;
+    const int c0 = LEVEL == 0 ? g * kReduceGroup : 0, c1 = LEVEL == 0 ? min(n, c0 + kReduceGroup) : n;
     float s = 0.f;
 #pragma unroll 8
-    for (int c = c0; c < c1; ++c) s += part[(size_t)c * len + i];
-    out[(size_t)blockIdx.y * len + i] = s;
+    for (int c = c0; c < c1; ++c) s += src[(size_t)c * it.len + i];
+    float* out = LEVEL == 0 && it.groups > 1 ? it.mid + (size_t)g * it.len : it.out;
+    out[i] = s;
 }
 
 // ---- elementwise and resampling ------------------------------------------------------
@@ -849,44 +904,84 @@ __global__ void input_kernel(const float* __restrict__ phi, const float* __restr
     for (int c = kCinReal; c < kCin0; ++c) dst[c] = 0;
 }
 
-// dpre = bf16((g + pool_grad) * gelu'(pre)); pool_grad(i) = gc[coarse(i)] / 4 when gc is given.
-__global__ void gelu_bwd_kernel(const float* __restrict__ g, const float* __restrict__ gc, const bf16* __restrict__ pre,
-                                int H, int W, int C, int n, bf16* __restrict__ dpre)
+// dpre = bf16((g + pool_grad) * gelu'(pre)), pool_grad(i) = gc[coarse(i)] / 4, eight channels a
+// thread: memory bound (1.0 of 2.1 bytes are the FP32 g).  One channel a thread took 183 us for
+// the two uses (16 samples of 256 x 256), now 82 us.
+template <int C>
+__global__ __launch_bounds__(256) void gelu_bwd_kernel(const float* __restrict__ g, const float* __restrict__ gc,
+                                                       const bf16* __restrict__ pre, int H, int W, int npix,
+                                                       bf16* __restrict__ dpre)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float v = g[i];
-    if (gc) {
-        const int c = i % C, t = i / C, x = t % W, t2 = t / W, y = t2 % H, b = t2 / H;
-        v += 0.25f * gc[(((size_t)b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int p = (int)(i / (C / 8)), c = 8 * (int)(i % (C / 8));
+    if (p >= npix) return;
+    const int t = p / W, x = p - t * W, b = t / H, y = t - b * H;
+    const float* gs = g + (size_t)p * C + c;
+    const float* cs = gc + (((size_t)b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c;
+    const u32x4 pv = load8u(pre + (size_t)p * C + c);
+    f32x4 v[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        v[h] = *reinterpret_cast<const f32x4*>(gs + 4 * h);
+        const f32x4 k = *reinterpret_cast<const f32x4*>(cs + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[h][e] += 0.25f * k[e];
     }
-    dpre[i] = f2bf(v * gelu_grad(bf2f(pre[i])));
+    u32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        r[j] = (uint32_t)f2bf(v[j / 2][2 * (j % 2)] * gelu_grad(lo_f(pv[j]))) |
+               ((uint32_t)f2bf(v[j / 2][2 * (j % 2) + 1] * gelu_grad(hi_f(pv[j]))) << 16);
+    *reinterpret_cast<u32x4*>(dpre + (size_t)p * C + c) = r;
 }
 
 // ---- head (32 -> 2 channels, FP32 weights and output) ----------------------------------
 
-__global__ void head_fwd_kernel(const bf16* __restrict__ d1, const float* __restrict__ wh, const float* __restrict__ bh,
-                                int H, int W, int npix, float* __restrict__ J)
+// J = kJScale (bh + sum_{tap, ci} wh[tap][c][ci] d1[p + shift(tap)][ci]) over 16 x 16 pixels a
+// block: the padded tile goes to LDS in 16-byte pieces, a thread takes one pixel and its weights
+// are scalars.  Bound by the 576 multiply-adds of a pixel and the widening of its 288 inputs;
+// with every thread reading its 18 x 32 bytes per tap from global memory this was 58 us for 16
+// samples of 256 x 256, now 40 us.
+__global__ __launch_bounds__(256) void head_fwd_kernel(const bf16* __restrict__ d1, const float* __restrict__ wh,
+                                                       const float* __restrict__ bh, int H, int W,
+                                                       float* __restrict__ J)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    const int x = p % W, t = p / W, y = t % H, n = t / H;
+    constexpr int LD = 40, PW = 18, ITEMS = PW * PW * 4, PER = (ITEMS + 255) / 256;
+    __shared__ __align__(16) bf16 s[PW * PW * LD];
+    const int tid = threadIdx.x;
+    const int nt = gridDim.x, b = nt % 8 ? blockIdx.x : (blockIdx.x % 8) * (nt / 8) + blockIdx.x / 8;  // as conv_kernel
+    const int tx = W / 16, ty = H / 16, t = b / tx, n = t / ty, x0 = 16 * (b - t * tx), y0 = 16 * (t - n * ty);
+    u32x4 sv[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = min(tid + 256 * k, ITEMS - 1), pp = i >> 2, ry = pp / PW, rx = pp - ry * PW;
+        sv[k] = load8u(d1 + (((size_t)n * H + wrapi(y0 + ry - 1, H)) * W + wrapi(x0 + rx - 1, W)) * 32 + 8 * (i & 3));
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = tid + 256 * k;
+        if (i < ITEMS) *reinterpret_cast<u32x4*>(s + (i >> 2) * LD + 8 * (i & 3)) = sv[k];
+    }
+    __syncthreads();
     // one accumulator per tap column, summed as in c7_head_flux_kernel (same rounding)
     float j0[3] = {bh[0], 0.f, 0.f}, j1[3] = {bh[1], 0.f, 0.f};
+    const bf16* src = s + ((tid >> 4) * PW + (tid & 15)) * LD;
 #pragma unroll
     for (int tap = 0; tap < 9; ++tap) {
-        const int yy = wrapi(y + tap / 3 - 1, H), xx = wrapi(x + tap % 3 - 1, W);
-        const bf16* src = d1 + (((size_t)n * H + yy) * W + xx) * 32;
         const float* w0 = wh + tap * 64;
 #pragma unroll
-        for (int ci = 0; ci < 32; ++ci) {
-            const float v = bf2f(src[ci]);
-            j0[tap % 3] = fmaf(v, w0[ci], j0[tap % 3]);
-            j1[tap % 3] = fmaf(v, w0[32 + ci], j1[tap % 3]);
+        for (int c8 = 0; c8 < 4; ++c8) {
+            const u32x4 v = load8u(src + (tap / 3 * PW + tap % 3) * LD + 8 * c8);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float x = j % 2 ? hi_f(v[j / 2]) : lo_f(v[j / 2]);
+                j0[tap % 3] = fmaf(x, w0[8 * c8 + j], j0[tap % 3]);
+                j1[tap % 3] = fmaf(x, w0[32 + 8 * c8 + j], j1[tap % 3]);
+            }
         }
     }
-    J[2 * (size_t)p] = kJScale * ((j0[0] + j0[1]) + j0[2]);
-    J[2 * (size_t)p + 1] = kJScale * ((j1[0] + j1[1]) + j1[2]);
+    const size_t p = ((size_t)n * H + y0 + (tid >> 4)) * W + x0 + (tid & 15);
+    *reinterpret_cast<float2*>(J + 2 * p) = make_float2(kJScale * ((j0[0] + j0[1]) + j0[2]), kJScale * ((j1[0] + j1[1]) + j1[2]));
 }
 
 // Inference tail in one kernel per TYO x 16 tile: c7 (3x3, 32 -> 32, GELU) on the
@@ -1315,34 +1410,48 @@ __global__ void adam_kernel(float* __restrict__ w, const float* __restrict__ g, 
     w[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
 }
 
-// BF16 forward [tap][co][ci] and backward-data [tap][ci][co] copies of a layer's weights.
-__global__ void pack_kernel(const float* __restrict__ master, int taps, int cout, int cin, bf16* __restrict__ wf,
-                            bf16* __restrict__ wb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= taps * cout * cin) return;
-    const int ci = i % cin, t = i / cin, co = t % cout, tap = t / cout;
-    const bf16 v = f2bf(master[i]);
-    wf[i] = v;
-    wb[((size_t)tap * cin + ci) * cout + co] = v;
-}
-
-// c1 inference weights: the first 8 of the 16 input channels (the data channels and
+// BF16 forward [tap][co][ci] and backward-data [tap][ci][co] copies of all layers' weights, and
+// c1's inference weights w8 over the first 8 of its 16 input channels (the data channels and
 // zero pads), [tap][co][8].
-__global__ void pack_c1_kernel(const float* __restrict__ master, bf16* __restrict__ w8)
+struct PackSet {
+    struct Layer {
+        const float* master;
+        bf16 *wf, *wb;
+        int taps, cout, cin, block;  // block: the layer's first
+    } layer[7];
+    bf16* w8;
+};
+
+__global__ __launch_bounds__(256) void pack_kernel(const PackSet set)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 9 * 32 * 8) return;
-    const int ci = i % 8, t = i / 8;  // t = tap * 32 + co
-    w8[i] = f2bf(master[(size_t)t * kCin0 + ci]);
+    int l = 0;
+    while (l < 6 && (int)blockIdx.x >= set.layer[l + 1].block) ++l;
+    const PackSet::Layer& L = set.layer[l];
+    const int i = (blockIdx.x - L.block) * 256 + threadIdx.x;
+    if (i >= L.taps * L.cout * L.cin) return;
+    const int ci = i % L.cin, t = i / L.cin, co = t % L.cout, tap = t / L.cout;
+    const bf16 v = f2bf(L.master[i]);
+    L.wf[i] = v;
+    L.wb[((size_t)tap * L.cin + ci) * L.cout + co] = v;
+    if (l == 0 && ci < 8) set.w8[t * 8 + ci] = v;
 }
 
-__global__ void gather_kernel(const float* __restrict__ src, const int* __restrict__ idx, int per, int count,
-                              float* __restrict__ dst)
+// The batch's fields, targets, parameters and normalisers in one launch: tensor blockIdx.y of
+// the dataset, `per` values a sample.
+struct GatherSet {
+    struct {
+        const float* src;
+        float* dst;
+        int per;
+    } t[4];
+};
+
+__global__ void gather_kernel(const GatherSet set, const int* __restrict__ idx, int count)
 {
+    const auto& t = set.t[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= per * count) return;
-    dst[i] = src[(size_t)idx[i / per] * per + i % per];
+    if (i >= t.per * count) return;
+    t.dst[i] = t.src[(size_t)idx[i / t.per] * t.per + i % t.per];
 }
 
 __global__ void f64_to_f32_kernel(const double* __restrict__ a, int n, float* __restrict__ b)
@@ -1370,8 +1479,6 @@ const LayerDef kLayers[8] = {{kCin0, 32, 9, true}, {32, 64, 9, true},  {64, 128,
 constexpr int kEw = 256;  // threads of elementwise kernels
 
 unsigned blocks_for(size_t n, int t = kEw) { return (unsigned)((n + t - 1) / t); }
-
-constexpr int kReduceGroup = 64;  // chunks summed per thread in each level of the reduction
 
 // Pixels per weight-gradient partial: the largest of 4096 .. 256 dividing npix
 // (npix is always a multiple of 256 since grid sides are multiples of 64).
@@ -1508,52 +1615,90 @@ hipError_t wgrad(const bf16* dpre, int cout, const bf16* in, int cin, int taps, 
     return hipErrorInvalidValue;
 }
 
-// out[i] = sum over nch chunks of s->part[c * len + i]: one pass for up to 64 chunks,
-// else groups of 64 into s->part2 and then the groups (a tree of fixed shape).
-hipError_t reduce_parts(amb_surrogate* s, int nch, int len, float* out)
-{
-    if (nch <= kReduceGroup) {
-        hipLaunchKernelGGL(reduce_chunks_kernel, dim3(blocks_for(len), 1), dim3(kEw), 0, s->stream, s->part, nch, len,
-                           nch, out);
-        return hipGetLastError();
+// Partials of an iteration's gradients in s->part, summed by reduce_all.
+struct Partials {
+    amb_surrogate* s;
+    ReduceSet set;
+    size_t used = 0, mid = 0;
+    bool fits = true;
+
+    // room for nch partials of `len` values that sum to `out`; null when s->part is too small
+    float* add(int nch, int len, float* out)
+    {
+        const int groups = (nch + kReduceGroup - 1) / kReduceGroup, per = (int)blocks_for(len);
+        const size_t n = (size_t)nch * len, m = groups > 1 ? (size_t)groups * len : 0;
+        if (set.count == ReduceSet::kMax || used + n > s->part_len || mid + m > s->part2_len) {
+            fits = false;
+            return nullptr;
+        }
+        ReduceItem& it = set.item[set.count++];
+        it = {s->part + used, s->part2 + mid, out, nch, len, groups, {set.blocks[0], set.blocks[1]}};
+        set.blocks[0] += groups * per;
+        if (groups > 1) set.blocks[1] += per;
+        used += n;
+        mid += m;
+        return s->part + used - n;
     }
-    const int groups = (nch + kReduceGroup - 1) / kReduceGroup;
-    if ((size_t)groups * len > s->part2_len) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3(blocks_for(len), groups), dim3(kEw), 0, s->stream, s->part, nch, len,
-                       kReduceGroup, s->part2);
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3(blocks_for(len), 1), dim3(kEw), 0, s->stream, s->part2, groups, len,
-                       groups, out);
+};
+
+hipError_t reduce_all(Partials& P)
+{
+    hipStream_t st = P.s->stream;
+    hipLaunchKernelGGL(reduce_kernel<0>, dim3(P.set.blocks[0]), dim3(256), 0, st, P.set);
+    if (P.set.blocks[1]) hipLaunchKernelGGL(reduce_kernel<1>, dim3(P.set.blocks[1]), dim3(256), 0, st, P.set);
     return hipGetLastError();
 }
 
-// Weight and bias gradient of conv layer l into s->grad.
-int layer_grads(amb_surrogate* s, int l, const bf16* dpre, const bf16* in, int H, int W, int npix)
+// Weight and bias gradient of conv layer l, as partials that sum into s->grad.
+int layer_grads(amb_surrogate* s, Partials& P, int l, const bf16* dpre, const bf16* in, int H, int W, int npix)
 {
     const LayerDef& L = kLayers[l];
-    const int chunk = chunk_for(npix), nch = npix / chunk;
-    const int len = L.taps * L.cout * L.cin;
-    hipError_t e = wgrad(dpre, L.cout, in, L.cin, L.taps, H, W, npix, s->part, s->stream);
-    if (e == hipSuccess) e = reduce_parts(s, nch, len, s->grad + s->w_off[l]);
+    const int nb = npix / kBiasChunk;
+    float* pw = P.add(npix / chunk_for(npix), L.taps * L.cout * L.cin, s->grad + s->w_off[l]);
+    float* pb = P.add(nb, L.cout, s->grad + s->b_off[l]);
+    if (!P.fits) return fail(AMB_E_STATE, "surrogate weight gradient: partial buffer");
+    hipError_t e = wgrad(dpre, L.cout, in, L.cin, L.taps, H, W, npix, pw, s->stream);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(bgrad_kernel, dim3(npix / 256), dim3(256), 0, s->stream, dpre, L.cout, 256, s->part);
+        const dim3 grid((nb + 1) / 2);
+        if (L.cout == 32) hipLaunchKernelGGL(bgrad_kernel<32>, grid, dim3(64), 0, s->stream, dpre, nb, pb);
+        if (L.cout == 64) hipLaunchKernelGGL(bgrad_kernel<64>, grid, dim3(64), 0, s->stream, dpre, nb, pb);
+        if (L.cout == 128) hipLaunchKernelGGL(bgrad_kernel<128>, grid, dim3(64), 0, s->stream, dpre, nb, pb);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = reduce_parts(s, npix / 256, L.cout, s->grad + s->b_off[l]);
     return e == hipSuccess ? AMB_OK : fail_hip(e, "surrogate weight gradient");
+}
+
+// Floats that the partials of npix full-resolution pixels take, and the sums of their groups.
+void partial_size(int npix, size_t* part, size_t* mid)
+{
+    const int shift_of[8] = {0, 2, 4, 4, 2, 2, 0, 0};
+    *part = *mid = 0;
+    auto add = [&](int nch, size_t len) {
+        *part += nch * len;
+        if (nch > kReduceGroup) *mid += (size_t)((nch + kReduceGroup - 1) / kReduceGroup) * len;
+    };
+    for (int l = 0; l < 8; ++l) {
+        const int np = npix >> shift_of[l];
+        if (l == 7) {
+            add(np / kHeadChunk, 578);
+        } else {
+            add(np / chunk_for(np), (size_t)kLayers[l].taps * kLayers[l].cout * kLayers[l].cin);
+            add(np / kBiasChunk, kLayers[l].cout);
+        }
+    }
 }
 
 int pack_weights(amb_surrogate* s)
 {
+    PackSet set;
+    int blocks = 0;
     for (int l = 0; l < 7; ++l) {
         const LayerDef& L = kLayers[l];
-        const int n = L.taps * L.cout * L.cin;
-        hipLaunchKernelGGL(pack_kernel, dim3(blocks_for(n)), dim3(kEw), 0, s->stream, s->master + s->w_off[l], L.taps,
-                           L.cout, L.cin, s->wf[l], s->wb[l]);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return fail_hip(e, "weight pack");
+        set.layer[l] = {s->master + s->w_off[l], s->wf[l], s->wb[l], L.taps, L.cout, L.cin, blocks};
+        blocks += (int)blocks_for((size_t)L.taps * L.cout * L.cin);
     }
-    hipLaunchKernelGGL(pack_c1_kernel, dim3(blocks_for(9 * 32 * 8)), dim3(kEw), 0, s->stream, s->master + s->w_off[0],
-                       s->wf0_8);
+    set.w8 = s->wf0_8;
+    hipLaunchKernelGGL(pack_kernel, dim3(blocks), dim3(kEw), 0, s->stream, set);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AMB_OK : fail_hip(e, "weight pack");
 }
@@ -1591,8 +1736,7 @@ int forward(amb_surrogate* s, int n, const float* phi, const float* params, floa
     SUR_CHECK((conv_launch<64, 2, 1, 16, 1, 4, kOutBf16>(wb({.in = s->d2, .out = s->u1}, 5), P2, H2, W2, st)));
     SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutBf16Gelu, false, true>(
         wb({.in = s->e1, .coarse = s->u1, .sum = s->s1, .out = s->d1, .pre = s->d1p}, 6), P1, H, W, st)));
-    hipLaunchKernelGGL(head_fwd_kernel, dim3(blocks_for(P1)), dim3(kEw), 0, st, s->d1, M + s->w_off[7], M + s->b_off[7],
-                       H, W, P1, J);
+    hipLaunchKernelGGL(head_fwd_kernel, dim3(P1 / 256), dim3(256), 0, st, s->d1, M + s->w_off[7], M + s->b_off[7], H, W, J);
     SUR_CHECK(hipGetLastError());
     return AMB_OK;
 }
@@ -1646,42 +1790,43 @@ int loss_and_grad(amb_surrogate* s, int n, double* loss_out)
     // head
     hipLaunchKernelGGL(head_bwd_data_kernel, dim3(P1 / 64), dim3(256), 0, st, s->dJ, M + s->w_off[7], s->d1p, H, W,
                        s->dpre);
+    Partials P{s};
     const int hch = P1 / kHeadChunk;
-    hipLaunchKernelGGL(head_bwd_weight_kernel, dim3(blocks_for(hch, 4)), dim3(256), 0, st, s->dJ, s->d1, H, W, hch,
-                       s->part);
+    float* hpart = P.add(hch, 578, s->grad + s->w_off[7]);
+    if (!hpart) return fail(AMB_E_STATE, "surrogate weight gradient: partial buffer");
+    hipLaunchKernelGGL(head_bwd_weight_kernel, dim3(blocks_for(hch, 4)), dim3(256), 0, st, s->dJ, s->d1, H, W, hch, hpart);
     SUR_CHECK(hipGetLastError());
-    SUR_CHECK(reduce_parts(s, hch, 578, s->grad + s->w_off[7]));
     // c7 (in s1), then s1 = up(u1) + e1
-    if ((rc = layer_grads(s, 6, s->dpre, s->s1, H, W, P1)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, P, 6, s->dpre, s->s1, H, W, P1)) != AMB_OK) return rc;
     SUR_CHECK((conv_launch<32, 2, 9, 16, 1, 4, kOutF32SumPool, true>(
         {.in = s->dpre, .w = s->wb[6], .out = s->ds1, .pooled = s->dpre2}, P1, H, W, st)));
     // c6 (1x1, in d2)
-    if ((rc = layer_grads(s, 5, s->dpre2, s->d2, H2, W2, P2)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, P, 5, s->dpre2, s->d2, H2, W2, P2)) != AMB_OK) return rc;
     // c5 (in s2), then s2 = up(u2) + e2
     SUR_CHECK((conv_launch<32, 4, 1, 16, 2, 2, kOutGeluBwd>({.in = s->dpre2, .w = s->wb[5], .out = s->dpre, .pre = s->d2p},
                                                             P2, H2, W2, st)));
-    if ((rc = layer_grads(s, 4, s->dpre, s->s2, H2, W2, P2)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, P, 4, s->dpre, s->s2, H2, W2, P2)) != AMB_OK) return rc;
     SUR_CHECK((conv_launch<64, 4, 9, 16, 4, 1, kOutF32SumPool, true>(
         {.in = s->dpre, .w = s->wb[4], .out = s->ds2, .pooled = s->dpre2}, P2, H2, W2, st)));
     // c4 (1x1, in bt)
-    if ((rc = layer_grads(s, 3, s->dpre2, s->bt, H4, W4, P3)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, P, 3, s->dpre2, s->bt, H4, W4, P3)) != AMB_OK) return rc;
     // c3 (in p2)
     SUR_CHECK((conv_launch<64, 8, 1, 8, 4, 1, kOutGeluBwd>({.in = s->dpre2, .w = s->wb[3], .out = s->dpre, .pre = s->btp},
                                                            P3, H4, W4, st)));
-    if ((rc = layer_grads(s, 2, s->dpre, s->p2, H4, W4, P3)) != AMB_OK) return rc;
+    if ((rc = layer_grads(s, P, 2, s->dpre, s->p2, H4, W4, P3)) != AMB_OK) return rc;
     SUR_CHECK((conv_launch<128, 4, 9, 8, 4, 1, kOutF32, true>({.in = s->dpre, .w = s->wb[2], .out = s->dp2}, P3, H4, W4,
                                                               st)));
     // c2 (in p1): de2 = ds2 + pool_grad(dp2)
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P2 * 64)), dim3(kEw), 0, st, s->ds2, s->dp2, s->e2p,
-                       H2, W2, 64, P2 * 64, s->dpre);
-    if ((rc = layer_grads(s, 1, s->dpre, s->p1, H2, W2, P2)) != AMB_OK) return rc;
+    hipLaunchKernelGGL(gelu_bwd_kernel<64>, dim3(blocks_for((size_t)P2 * 8)), dim3(kEw), 0, st, s->ds2, s->dp2, s->e2p, H2,
+                       W2, P2, s->dpre);
+    if ((rc = layer_grads(s, P, 1, s->dpre, s->p1, H2, W2, P2)) != AMB_OK) return rc;
     SUR_CHECK((conv_launch<64, 2, 9, 16, 2, 2, kOutF32, true>({.in = s->dpre, .w = s->wb[1], .out = s->dp1}, P2, H2, W2,
                                                               st)));
     // c1 (in x0): de1 = ds1 + pool_grad(dp1)
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for((size_t)P1 * 32)), dim3(kEw), 0, st, s->ds1, s->dp1, s->e1p,
-                       H, W, 32, P1 * 32, s->dpre);
-    if ((rc = layer_grads(s, 0, s->dpre, s->x0, H, W, P1)) != AMB_OK) return rc;
-    SUR_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(gelu_bwd_kernel<32>, dim3(blocks_for((size_t)P1 * 4)), dim3(kEw), 0, st, s->ds1, s->dp1, s->e1p, H, W,
+                       P1, s->dpre);
+    if ((rc = layer_grads(s, P, 0, s->dpre, s->x0, H, W, P1)) != AMB_OK) return rc;
+    SUR_CHECK(reduce_all(P));
     if (loss_out) {
         std::vector<float> lp(lb);
         SUR_CHECK(hipMemcpyAsync(lp.data(), s->loss_part, lb * sizeof(float), hipMemcpyDeviceToHost, st));
@@ -1779,17 +1924,12 @@ int amb_surrogate_create(int64_t ny, int64_t nx, int max_batch, uint64_t seed, a
     }
     s->nparams = off;
     const size_t B = max_batch, P1 = B * ny * nx, P2 = P1 / 4, P3 = P1 / 16;
-    // Partial-sum buffer: the most chunks x entries any layer needs at any batch size.
-    s->part_len = 0;
+    // Partial-sum buffers: the most that any batch size needs.
     for (int b = 1; b <= max_batch; ++b) {
-        const int lv[3] = {(int)(b * ny * nx), (int)(b * ny * nx / 4), (int)(b * ny * nx / 16)};
-        const int level_of[8] = {0, 1, 2, 2, 1, 1, 0, 0};
-        for (int l = 0; l < 8; ++l) {
-            const int npix = lv[level_of[l]];
-            const size_t len = l == 7 ? 578 : (size_t)kLayers[l].taps * kLayers[l].cout * kLayers[l].cin;
-            s->part_len = std::max(s->part_len, (size_t)(npix / chunk_for(npix)) * len);
-            s->part_len = std::max(s->part_len, (size_t)(npix / 256) * (l == 7 ? 578 : kLayers[l].cout));
-        }
+        size_t part, mid;
+        partial_size((int)(b * ny * nx), &part, &mid);
+        s->part_len = std::max(s->part_len, part);
+        s->part2_len = std::max(s->part2_len, mid);
     }
     hipError_t e = hipSuccess;
     auto A = [&](auto** p, size_t bytes) {
@@ -1837,7 +1977,6 @@ int amb_surrogate_create(int64_t ny, int64_t nx, int max_batch, uint64_t seed, a
     A(&s->dp2, P3 * 64 * 4);
     A(&s->dp1, P2 * 32 * 4);
     A(&s->part, s->part_len * 4);
-    s->part2_len = s->part_len / kReduceGroup + 9 * 128 * 64;
     A(&s->part2, s->part2_len * 4);
     A(&s->audit_part, kAuditBlocks * 2 * sizeof(double));
     A(&s->audit_buf, (size_t)ny * nx * sizeof(float));
@@ -1989,13 +2128,9 @@ int amb_surrogate_train(amb_surrogate* s, int64_t iterations, int batch, double 
             } while (dup);
         }
         SUR_CHECK(hipMemcpyAsync(s->d_idx, idx.data(), batch * sizeof(int), hipMemcpyHostToDevice, s->stream));
-        hipLaunchKernelGGL(gather_kernel, dim3(blocks_for((size_t)hw * batch)), dim3(kEw), 0, s->stream, s->ds_in,
-                           s->d_idx, hw, batch, s->phi);
-        hipLaunchKernelGGL(gather_kernel, dim3(blocks_for((size_t)hw * batch)), dim3(kEw), 0, s->stream, s->ds_out,
-                           s->d_idx, hw, batch, s->target);
-        hipLaunchKernelGGL(gather_kernel, dim3(blocks_for(3 * batch)), dim3(kEw), 0, s->stream, s->ds_par, s->d_idx, 3,
-                           batch, s->params);
-        hipLaunchKernelGGL(gather_kernel, dim3(1), dim3(kEw), 0, s->stream, s->ds_norm, s->d_idx, 1, batch, s->norm);
+        const GatherSet set = {{{s->ds_in, s->phi, hw}, {s->ds_out, s->target, hw}, {s->ds_par, s->params, 3}, {s->ds_norm, s->norm, 1}}};
+        hipLaunchKernelGGL(gather_kernel, dim3(blocks_for((size_t)hw * batch), 4), dim3(kEw), 0, s->stream, set, s->d_idx,
+                           batch);
         if (s->train_noise > 0.f) {
             hipLaunchKernelGGL(train_noise_kernel, dim3(blocks_for((size_t)hw * batch)), dim3(kEw), 0, s->stream, s->phi,
                                s->norm, s->H, s->W, hw * batch, s->train_noise, s->noise_iter++,
