@@ -69,7 +69,15 @@ __global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) vo
 // resident member's trajectory equals a plain integrator's bit for bit.  The last act of a
 // launch is the member's partial of the fused finite check (its FP64 sum and non-finite
 // count, reduced in a fixed order) at part[slot].
-constexpr size_t kResidentLds = 80 * 1024;
+//
+// A step of a lone workgroup is a chain of phases and barriers, so its time goes with the
+// number of tiles: members up to 64x64 (FP32) or 48x44 (FP64) that need several 256-thread
+// tiles take the whole member as one tile of 1024 or 704 threads, which nearly fills a CU's LDS.
+// A 64x64 FP32 member takes 6.2 us a step at T = 0 and 8.2 us with noise, against 15.5 and
+// 21.7 us in four 32x32 tiles (and 5.5 and 6.5 us as a launch of tiles per step, alone on the
+// device); a 40x40 FP64 member 6.9 and 9.7 us against 20.2 and 30.4 us.
+constexpr size_t kResidentLds = 80 * 1024;       // two field buffers and one small tile's scratch
+constexpr size_t kResidentWholeLds = 160 * 1024; // the same with the whole member's scratch
 
 template <typename T>
 __host__ __device__ constexpr size_t resident_field_bytes(int64_t n)
@@ -143,45 +151,76 @@ template <typename T>
 struct ResidentShape;
 template <>
 struct ResidentShape<float> {
-    static constexpr int tw = 32, th = 32, nt = 256;
+    static constexpr int tw = 32, th = 32, nt = 256;           // small members
+    static constexpr int wtw = 64, wth = 64, wnt = 1024;       // whole members
 };
 template <>
 struct ResidentShape<double> {
     static constexpr int tw = 32, th = 16, nt = 256;
+    static constexpr int wtw = 44, wth = 48, wnt = 704;
 };
 
-template <typename T>
+template <typename T, bool WHOLE>
 constexpr size_t resident_lds(int64_t n)
 {
     using S = ResidentShape<T>;
-    return 2 * resident_field_bytes<T>(n) + Lds<T, S::tw, S::th, S::nt>::bytes;
+    return 2 * resident_field_bytes<T>(n) +
+           (WHOLE ? Lds<T, S::wtw, S::wth, S::wnt>::bytes : Lds<T, S::tw, S::th, S::nt>::bytes);
 }
 
-// A member runs resident when its two buffers and one tile's scratch fit kResidentLds.
+// A member runs resident when its two buffers and one small tile's scratch fit kResidentLds.
+template <typename T>
+static bool fits_resident_t(int64_t ny, int64_t nx)
+{
+    return resident_lds<T, false>(ny * nx) <= kResidentLds;
+}
+
 static bool fits_resident(int precision, int64_t ny, int64_t nx)
 {
-    const int64_t n = ny * nx;
-    return precision == AMB_F32 ? resident_lds<float>(n) <= kResidentLds : resident_lds<double>(n) <= kResidentLds;
+    return precision == AMB_F32 ? fits_resident_t<float>(ny, nx) : fits_resident_t<double>(ny, nx);
+}
+
+// A resident member is stepped as one tile when it needs more than two small ones and fits the
+// large one.  Two small tiles take as long as the large one (32x32 FP64: 6.8 / 7.0 us a step,
+// noisy 10.1 / 9.7), but several such members share a CU (1024 of them: 17 / 27 us).
+template <typename T>
+static bool resident_whole_t(int64_t ny, int64_t nx)
+{
+    using S = ResidentShape<T>;
+    const int64_t small = ((ny + S::th - 1) / S::th) * ((nx + S::tw - 1) / S::tw);
+    return small > 2 && ny <= S::wth && nx <= S::wtw &&
+           resident_lds<T, true>(ny * nx) <= kResidentWholeLds;
+}
+
+static bool resident_whole(int precision, int64_t ny, int64_t nx)
+{
+    return precision == AMB_F32 ? resident_whole_t<float>(ny, nx) : resident_whole_t<double>(ny, nx);
 }
 
 template <typename T, int NOISE>
-static hipError_t launch_resident_t(const void* desc, const int* members, int count, int64_t max_n, const void* in,
-                                    void* out, const long long* step, int nsteps, double* part, int64_t part_base,
-                                    hipStream_t s)
+static hipError_t launch_resident_t(bool whole, const void* desc, const int* members, int count, int64_t max_n,
+                                    const void* in, void* out, const long long* step, int nsteps, double* part,
+                                    int64_t part_base, hipStream_t s)
 {
     using S = ResidentShape<T>;
-    hipLaunchKernelGGL((resident_kernel<T, S::tw, S::th, S::nt, NOISE>), dim3(count), dim3(S::nt),
-                       resident_lds<T>(max_n), s, static_cast<const BatchDesc<T>*>(desc), members,
-                       static_cast<const T*>(in), static_cast<T*>(out), step, nsteps, part, part_base);
+    const auto* d = static_cast<const BatchDesc<T>*>(desc);
+    if (whole)
+        hipLaunchKernelGGL((resident_kernel<T, S::wtw, S::wth, S::wnt, NOISE>), dim3(count), dim3(S::wnt),
+                           (resident_lds<T, true>(max_n)), s, d, members, static_cast<const T*>(in),
+                           static_cast<T*>(out), step, nsteps, part, part_base);
+    else
+        hipLaunchKernelGGL((resident_kernel<T, S::tw, S::th, S::nt, NOISE>), dim3(count), dim3(S::nt),
+                           (resident_lds<T, false>(max_n)), s, d, members, static_cast<const T*>(in),
+                           static_cast<T*>(out), step, nsteps, part, part_base);
     return hipGetLastError();
 }
 
-static hipError_t launch_resident(int precision, int noise, const void* desc, const int* members, int count,
+static hipError_t launch_resident(int precision, int noise, bool whole, const void* desc, const int* members, int count,
                                   int64_t max_n, const void* in, void* out, const long long* step, int nsteps,
                                   double* part, int64_t part_base, hipStream_t s)
 {
 #define AMB_RESIDENT(T, mode) \
-    launch_resident_t<T, mode>(desc, members, count, max_n, in, out, step, nsteps, part, part_base, s)
+    launch_resident_t<T, mode>(whole, desc, members, count, max_n, in, out, step, nsteps, part, part_base, s)
     if (precision == AMB_F32)
         return noise == kNoiseNone     ? AMB_RESIDENT(float, kNoiseNone)
                : noise == kNoisePhilox ? AMB_RESIDENT(float, kNoisePhilox)
@@ -192,18 +231,23 @@ static hipError_t launch_resident(int precision, int noise, const void* desc, co
 #undef AMB_RESIDENT
 }
 
-template <typename T>
+template <typename T, int NOISE>
 static hipError_t raise_resident_lds_t()
 {
     using S = ResidentShape<T>;
-    hipError_t e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, kNoiseNone>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, kNoisePhilox>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, kNoisePhiloxOdd>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
+    const hipError_t e = hipFuncSetAttribute((const void*)resident_kernel<T, S::tw, S::th, S::nt, NOISE>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentLds);
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute((const void*)resident_kernel<T, S::wtw, S::wth, S::wnt, NOISE>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResidentWholeLds);
+}
+
+template <typename T>
+static hipError_t raise_resident_lds()
+{
+    hipError_t e = raise_resident_lds_t<T, kNoiseNone>();
+    if (e == hipSuccess) e = raise_resident_lds_t<T, kNoisePhilox>();
+    if (e == hipSuccess) e = raise_resident_lds_t<T, kNoisePhiloxOdd>();
     return e;
 }
 
@@ -232,8 +276,8 @@ static hipError_t prepare_batch_kernels()
     hipError_t e = hipSuccess;
     AMB_F32_TILES(AMB_BRAISE_F32)
     AMB_F64_TILES(AMB_BRAISE_F64)
-    if ((e = raise_resident_lds_t<float>()) != hipSuccess) return e;
-    return raise_resident_lds_t<double>();
+    if ((e = raise_resident_lds<float>()) != hipSuccess) return e;
+    return raise_resident_lds<double>();
 }
 
 template <typename T, int TW, int TH, int NT>
@@ -283,6 +327,14 @@ namespace {
 
 constexpr int kBatchGraphSteps = 32;
 
+// Resident members of one noise mode and tile, advanced by one launch.
+struct ResidentGroup {
+    int noise = 0;
+    bool whole = false;
+    int64_t first = 0, count = 0;  // in the resident member list
+    int64_t max_n = 0;             // sites of its largest member
+};
+
 struct Group {
     int tile = 0;
     int noise = 0;  // kNoiseNone, kNoisePhilox or kNoisePhiloxOdd
@@ -316,13 +368,11 @@ struct amb_batch {
     int64_t last_bad = 0;
     // members kept in LDS by the resident kernel (when enabled and they fit)
     bool resident_on = true;
-    std::vector<int> resident;         // grouped by noise mode:
-    int64_t resident_of[4] = {};       // how many of each (kNoiseNone, kNoisePhilox, -, kNoisePhiloxOdd)
+    std::vector<int> resident;         // in the order of the groups
+    std::vector<ResidentGroup> resident_groups;
     int* d_resident = nullptr;
-    int64_t resident_max_n = 0;
-    hipStream_t side = nullptr;     // capture branch of the resident launch, beside the tiled steps
-    hipEvent_t fork = nullptr, join = nullptr;
-    std::vector<hipStream_t> branch;      // capture branch per tile-shape group
+    hipEvent_t fork = nullptr;
+    std::vector<hipStream_t> branch;      // capture branch per tile-shape group and resident group
     std::vector<hipEvent_t> branch_done;
     double* d_part = nullptr;
     unsigned long long* d_bad_part = nullptr;
@@ -356,7 +406,6 @@ void release(amb_batch* b)
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     drop_graphs(b);
     free_groups(b);
-    if (b->side) (void)hipStreamSynchronize(b->side);
     for (void* p : {b->buf[0], b->buf[1], (void*)b->d_step, (void*)b->d_step_scratch, b->d_desc, (void*)b->d_part,
                     (void*)b->d_bad_part, (void*)b->d_sum, (void*)b->d_bad, (void*)b->d_tile_part,
                     (void*)b->d_resident})
@@ -365,8 +414,6 @@ void release(amb_batch* b)
     for (hipEvent_t ev : b->branch_done) (void)hipEventDestroy(ev);
     for (hipStream_t st : b->branch) (void)hipStreamDestroy(st);
     if (b->fork) (void)hipEventDestroy(b->fork);
-    if (b->join) (void)hipEventDestroy(b->join);
-    if (b->side) (void)hipStreamDestroy(b->side);
     if (b->h_sum) (void)hipHostFree(b->h_sum);
     if (b->h_bad) (void)hipHostFree(b->h_bad);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -399,22 +446,23 @@ int rebuild_groups(amb_batch* b)
     drop_graphs(b);
     free_groups(b);
     std::map<std::pair<int, int>, std::vector<int>> by_tile;  // (tile, noise mode) -> members
-    std::vector<int> kept[4];  // resident members per noise mode
-    b->resident_max_n = 0;
+    std::map<std::pair<int, bool>, std::vector<int>> kept;  // (noise mode, whole) -> resident members
     for (size_t r = 0; r < b->desc.size(); ++r) {
         const amb_realisation& m = b->desc[r];
         const int noise = m.model.T > 0.0 ? philox_mode(m.nx) : kNoiseNone;
         if (b->resident_on && fits_resident(b->precision, m.ny, m.nx)) {
-            kept[noise].push_back((int)r);
-            b->resident_max_n = std::max(b->resident_max_n, m.ny * m.nx);
+            kept[{noise, resident_whole(b->precision, m.ny, m.nx)}].push_back((int)r);
         } else {
             by_tile[{b->tile_of[r], noise}].push_back((int)r);
         }
     }
     b->resident.clear();
-    for (int m = 0; m < 4; ++m) {
-        b->resident.insert(b->resident.end(), kept[m].begin(), kept[m].end());
-        b->resident_of[m] = (int64_t)kept[m].size();
+    b->resident_groups.clear();
+    for (const auto& kv : kept) {
+        ResidentGroup g{kv.first.first, kv.first.second, (int64_t)b->resident.size(), (int64_t)kv.second.size(), 0};
+        for (int r : kv.second) g.max_n = std::max<int64_t>(g.max_n, b->desc[r].ny * b->desc[r].nx);
+        b->resident.insert(b->resident.end(), kv.second.begin(), kv.second.end());
+        b->resident_groups.push_back(g);
     }
     if (b->d_resident) (void)hipFree(b->d_resident);
     b->d_resident = nullptr;
@@ -501,31 +549,27 @@ hipError_t launch_groups(amb_batch* b, int parity_in, const long long* step, int
     return hipSuccess;
 }
 
-// nsteps steps of every resident member in one launch on stream s, from buffer
+// nsteps steps of a group of resident members in one launch on stream s, from buffer
 // `parity_in` to buffer parity_in + nsteps.
-hipError_t launch_resident_members(amb_batch* b, int parity_in, int nsteps, hipStream_t s)
+hipError_t launch_resident_group(amb_batch* b, const ResidentGroup& g, int parity_in, int nsteps, hipStream_t s)
 {
-    if (b->resident.empty() || nsteps <= 0) return hipSuccess;
-    hipError_t e = hipSuccess;
-    int64_t first = 0;
-    for (int m = 0; m < 4 && e == hipSuccess; ++m) {
-        if (b->resident_of[m] > 0)
-            e = launch_resident(b->precision, m, b->d_desc, b->d_resident + first, (int)b->resident_of[m],
-                                b->resident_max_n, b->buf[parity_in & 1], b->buf[(parity_in + nsteps) & 1], b->d_step,
-                                nsteps, b->d_tile_part, b->ntiles_total + first, s);
-        first += b->resident_of[m];
-    }
-    return e;
+    return launch_resident(b->precision, g.noise, g.whole, b->d_desc, b->d_resident + g.first, (int)g.count, g.max_n,
+                           b->buf[parity_in & 1], b->buf[(parity_in + nsteps) & 1], b->d_step, nsteps, b->d_tile_part,
+                           b->ntiles_total + g.first, s);
 }
 
-// The graph of kBatchGraphSteps steps: the resident members' one launch on a branch of
-// its own (fork from and join to the main stream), beside the tiled members' steps.
+// The graph of kBatchGraphSteps steps: the resident groups' launches and the tile-shape
+// groups' chains of steps, each on a branch of its own (fork from and join to the main stream).
 int build_graph(amb_batch* b, int parity)
 {
-    // one capture branch per tile-shape group (its kBatchGraphSteps steps in a chain) and
-    // one for the resident members: the groups touch disjoint members, so their chains run
-    // side by side and one group's last, partial round of workgroups overlaps the others'
-    while (b->branch.size() < b->groups.size()) {
+    // one capture branch per tile-shape group (its kBatchGraphSteps steps in a chain) and per
+    // resident group: the groups touch disjoint members, so their chains run side by side and
+    // one group's last, partial round of workgroups overlaps the others'.  A fifth chain has
+    // no hardware queue of its own and holds up another (8 members of 64 to 512 a side: 10.2 us
+    // a step with four chains, 18 with five), so the resident groups share what is left of four.
+    const size_t nres = std::min(b->resident_groups.size(), b->groups.size() < 3 ? 4 - b->groups.size() : 1);
+    const size_t nbranch = nres + b->groups.size();
+    while (b->branch.size() < nbranch) {
         hipStream_t st = nullptr;
         hipEvent_t ev = nullptr;
         hipError_t ce = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
@@ -541,14 +585,14 @@ int build_graph(amb_batch* b, int parity)
     hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return fail_hip(e, "hipStreamBeginCapture");
     e = hipEventRecord(b->fork, b->stream);
-    if (e == hipSuccess && !b->resident.empty()) {
-        e = hipStreamWaitEvent(b->side, b->fork, 0);
-        if (e == hipSuccess) e = launch_resident_members(b, parity, kBatchGraphSteps, b->side);
-        if (e == hipSuccess) e = hipEventRecord(b->join, b->side);
-    }
+    // resident groups first: their few workgroups run through the whole graph
+    for (size_t i = 0; i < nres && e == hipSuccess; ++i) e = hipStreamWaitEvent(b->branch[i], b->fork, 0);
+    for (size_t i = 0; i < b->resident_groups.size() && e == hipSuccess; ++i)
+        e = launch_resident_group(b, b->resident_groups[i], parity, kBatchGraphSteps, b->branch[i % nres]);
+    for (size_t i = 0; i < nres && e == hipSuccess; ++i) e = hipEventRecord(b->branch_done[i], b->branch[i]);
     for (size_t i = 0; i < b->groups.size() && e == hipSuccess; ++i) {
         const Group& gr = b->groups[i];
-        hipStream_t st = b->branch[i];
+        hipStream_t st = b->branch[nres + i];
         e = hipStreamWaitEvent(st, b->fork, 0);
         for (int k = 0; k < kBatchGraphSteps && e == hipSuccess; ++k) {
             const int pin = parity + k;
@@ -556,10 +600,9 @@ int build_graph(amb_batch* b, int parity)
                              b->buf[(pin + 1) & 1], b->d_step, k,
                              k == kBatchGraphSteps - 1 ? b->d_tile_part + 2 * gr.part_base : nullptr, st);
         }
-        if (e == hipSuccess) e = hipEventRecord(b->branch_done[i], st);
+        if (e == hipSuccess) e = hipEventRecord(b->branch_done[nres + i], st);
     }
-    for (size_t i = 0; i < b->groups.size() && e == hipSuccess; ++i) e = hipStreamWaitEvent(b->stream, b->branch_done[i], 0);
-    if (e == hipSuccess && !b->resident.empty()) e = hipStreamWaitEvent(b->stream, b->join, 0);
+    for (size_t i = 0; i < nbranch && e == hipSuccess; ++i) e = hipStreamWaitEvent(b->stream, b->branch_done[i], 0);
     if (e == hipSuccess) e = launch_advance(b->d_step, kBatchGraphSteps, b->stream);
     const hipError_t e2 = hipStreamEndCapture(b->stream, &g);
     if (e != hipSuccess) {
@@ -590,8 +633,9 @@ int enqueue(amb_batch* b, int64_t nsteps)
             if ((e = hipGraphLaunch(b->graph[p], b->stream)) != hipSuccess) return fail_hip(e, "hipGraphLaunch");
         left -= reps * kBatchGraphSteps;
     }
-    if (left > 0 && (e = launch_resident_members(b, b->cur, (int)left, b->stream)) != hipSuccess)
-        return fail_hip(e, "resident launch");
+    for (size_t i = 0; i < b->resident_groups.size() && left > 0; ++i)
+        if ((e = launch_resident_group(b, b->resident_groups[i], b->cur, (int)left, b->stream)) != hipSuccess)
+            return fail_hip(e, "resident launch");
     for (int k = 0; k < left; ++k)
         if ((e = launch_groups(b, b->cur + k, b->d_step, k, k == left - 1)) != hipSuccess)
             return fail_hip(e, "batched launch");
@@ -675,10 +719,17 @@ int amb_batch_create(const amb_realisation* desc, int64_t count, const double* c
         b->off[r] = o;
         o += desc[r].ny * desc[r].nx;
     }
-    b->tile_of.assign(count, 0);
-    for (int64_t r = 0; r < count; ++r)  // the tuning table's entries where it has them
-        (void)tuned_tile(precision, desc[r].ny, desc[r].nx, desc[r].model.T > 0.0 ? kNoisePhilox : kNoiseNone,
-                         &b->tile_of[r]);
+    // Tiles by noise mode alone: members of all sizes share the launches, so it is throughput that
+    // counts.  us a step with 4, 12 and 48 members of sides 64 .. 512, a third of them at T = 0:
+    // FP32 noisy members in 32x32 tiles of 512 threads 9.1, 11.9, 29.6, in 32x48 ones 10.0, 13.0,
+    // 31.5, members at T = 0 in 32x32 ones too 8.9, 11.9, 32.2; FP64 32x32 of 512 threads 12.2,
+    // 20.2, 64, of 256 threads 14.5, 24.3, 79.
+    b->tile_of.resize(count);
+    for (int64_t r = 0; r < count; ++r) {
+        const int noise = desc[r].model.T > 0.0 ? kNoisePhilox : kNoiseNone;
+        b->tile_of[r] = precision == AMB_F64 ? kSquare512F64 : noise == kNoisePhilox ? kSquare512F32 : 0;
+        (void)tuned_tile(precision, desc[r].ny, desc[r].nx, noise, &b->tile_of[r]);  // the tuning table's entry, if any
+    }
     hipError_t e;
 #define AMB_CHECK(call)                           \
     do {                                          \
@@ -692,9 +743,7 @@ int amb_batch_create(const amb_realisation* desc, int64_t count, const double* c
     const size_t desc_bytes = (size_t)count * (precision == AMB_F32 ? sizeof(BatchDesc<float>) : sizeof(BatchDesc<double>));
     AMB_CHECK(prepare_batch_kernels());
     AMB_CHECK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-    AMB_CHECK(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
     AMB_CHECK(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
-    AMB_CHECK(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     AMB_CHECK(hipMalloc(&b->buf[0], (size_t)total * b->esize));
     AMB_CHECK(hipMalloc(&b->buf[1], (size_t)total * b->esize));
     AMB_CHECK(hipMalloc(&b->d_step, sizeof(long long)));

@@ -70,3 +70,23 @@ def test_strips_count_nonfinite_sites(amb):
     # along each axis (a cross of two 3 x 19 bars), G3 of G3 to the 7x7 square, 16 sites of which
     # the cross misses
     assert bad == bad_full == (2 * 3 * 19 - 9) + 16
+
+
+# Resident ensemble members that are one large tile: just past two small tiles (32 x 32 FP32,
+# 32 x 16 FP64), the large tile's own size and one less, columns that do and do not split into
+# fours, and members one row or column past it, which keep to small tiles.
+@pytest.mark.parametrize("precision,shapes", [
+    (32, [(33, 32), (32, 33), (64, 64), (63, 61), (9, 64), (64, 9), (65, 40), (30, 66)]),
+    (64, [(17, 32), (16, 33), (44, 44), (48, 40), (47, 39), (9, 44), (49, 30), (30, 45)])])
+def test_resident_members_equal_integrators(amb, precision, shapes):
+    rng = np.random.default_rng(precision)
+    st = amb.Stencil(5e-3, 1, 1.25)
+    fields = [0.05 * rng.normal(size=s) for s in shapes for _ in range(2)]
+    models = [amb.Model(-0.25, 0, 0.25, 1, 0.5, -1, t) for _ in shapes for t in (0.0, 0.05)]
+    ens = amb.Ensemble(fields, st, models, list(range(len(fields))), precision=precision)
+    assert ens.resident_count == len(fields)
+    ens.run(37)  # a graph of 32 steps and a launch of five
+    for i, f in enumerate(fields):
+        sim = amb.Integrator(f, st, models[i], seed=i, precision=precision)
+        sim.run(37)
+        np.testing.assert_array_equal(ens.field(i), sim.field, err_msg=str((i, f.shape)))
