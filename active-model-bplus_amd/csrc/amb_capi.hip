@@ -373,14 +373,20 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
     return AMB_OK;
 }
 
-int reduce_now(amb_handle* h, double* sum, int64_t* bad)
+// FP64 sum and non-finite count of the field into h->d_sum and h->d_bad.
+hipError_t enqueue_reduce(amb_handle* h)
 {
     const int64_t n = h->ny * h->nx;
-    hipError_t e = h->precision == AMB_F32
-                       ? launch_reduce_f32(static_cast<const float*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part,
-                                           h->d_sum, h->d_bad, h->stream)
-                       : launch_reduce_f64(static_cast<const double*>(h->buf[h->cur]), n, h->d_part,
-                                           h->d_bad_part, h->d_sum, h->d_bad, h->stream);
+    return h->precision == AMB_F32
+               ? launch_reduce_f32(static_cast<const float*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, h->d_sum,
+                                   h->d_bad, h->stream)
+               : launch_reduce_f64(static_cast<const double*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, h->d_sum,
+                                   h->d_bad, h->stream);
+}
+
+int reduce_now(amb_handle* h, double* sum, int64_t* bad)
+{
+    hipError_t e = enqueue_reduce(h);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
     if ((e = hipMemcpyAsync(h->h_sum, h->d_sum, sizeof(double), hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
         return fail_hip(e, "hipMemcpyAsync");
@@ -488,6 +494,14 @@ int handle_view(amb_handle* h, FieldView* v)
     v->nx = h->nx;
     v->precision = h->precision;
     v->stream = h->stream;
+    return AMB_OK;
+}
+
+int handle_field_sum(amb_handle* h, const double** sum)
+{
+    const hipError_t e = enqueue_reduce(h);
+    if (e != hipSuccess) return fail_hip(e, "reduction launch");
+    *sum = h->d_sum;
     return AMB_OK;
 }
 

@@ -35,6 +35,9 @@ struct FieldView {
     hipStream_t stream;
 };
 int handle_view(amb_handle* h, FieldView* v);
+// Enqueues the FP64 sum of the current field on the handle's stream; *sum is where it will be
+// (device memory of the handle, rewritten by the next reduction).
+int handle_field_sum(amb_handle* h, const double** sum);
 // Advances the step counter by `steps` (host and device); with `swapped` the field
 // now lives in the buffer that was `other`.
 int handle_commit(amb_handle* h, int64_t steps, bool swapped);
