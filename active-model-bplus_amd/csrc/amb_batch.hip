@@ -376,9 +376,7 @@ struct amb_batch {
     std::vector<hipEvent_t> branch_done;
     double* d_part = nullptr;
     unsigned long long* d_bad_part = nullptr;
-    double* d_sum = nullptr;
-    unsigned long long* d_bad = nullptr;
-    double* h_sum = nullptr;
+    double* h_sum = nullptr;               // pinned: reductions write their results here
     unsigned long long* h_bad = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -407,7 +405,7 @@ void release(amb_batch* b)
     drop_graphs(b);
     free_groups(b);
     for (void* p : {b->buf[0], b->buf[1], (void*)b->d_step, (void*)b->d_step_scratch, b->d_desc, (void*)b->d_part,
-                    (void*)b->d_bad_part, (void*)b->d_sum, (void*)b->d_bad, (void*)b->d_tile_part,
+                    (void*)b->d_bad_part, (void*)b->d_tile_part,
                     (void*)b->d_resident})
         if (p) (void)hipFree(p);
     for (hipStream_t st : b->branch) (void)hipStreamSynchronize(st);
@@ -650,15 +648,10 @@ int reduce_range(amb_batch* b, int64_t off, int64_t n, double* sum, int64_t* bad
 {
     hipError_t e = b->precision == AMB_F32
                        ? launch_reduce_f32(static_cast<const float*>(b->buf[b->cur]) + off, n, b->d_part,
-                                           b->d_bad_part, b->d_sum, b->d_bad, b->stream)
+                                           b->d_bad_part, b->h_sum, b->h_bad, b->stream)
                        : launch_reduce_f64(static_cast<const double*>(b->buf[b->cur]) + off, n, b->d_part,
-                                           b->d_bad_part, b->d_sum, b->d_bad, b->stream);
+                                           b->d_bad_part, b->h_sum, b->h_bad, b->stream);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
-    if ((e = hipMemcpyAsync(b->h_sum, b->d_sum, sizeof(double), hipMemcpyDeviceToHost, b->stream)) != hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipMemcpyAsync(b->h_bad, b->d_bad, sizeof(unsigned long long), hipMemcpyDeviceToHost, b->stream)) !=
-        hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
     if ((e = hipStreamSynchronize(b->stream)) != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
     *sum = *b->h_sum;
     *bad = (int64_t)*b->h_bad;
@@ -671,14 +664,9 @@ int reduce_range(amb_batch* b, int64_t off, int64_t n, double* sum, int64_t* bad
 int finish_run(amb_batch* b, int64_t nsteps, double* sum, int64_t* bad)
 {
     if (nsteps == 0) return reduce_range(b, 0, b->total, sum, bad);
-    hipError_t e = launch_reduce_tiles(b->d_tile_part, b->ntiles_total + (int64_t)b->resident.size(), b->d_sum,
-                                       b->d_bad, b->stream);
+    hipError_t e = launch_reduce_tiles(b->d_tile_part, b->ntiles_total + (int64_t)b->resident.size(), b->h_sum,
+                                       b->h_bad, b->stream);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
-    if ((e = hipMemcpyAsync(b->h_sum, b->d_sum, sizeof(double), hipMemcpyDeviceToHost, b->stream)) != hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipMemcpyAsync(b->h_bad, b->d_bad, sizeof(unsigned long long), hipMemcpyDeviceToHost, b->stream)) !=
-        hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
     if ((e = hipStreamSynchronize(b->stream)) != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
     *sum = *b->h_sum;
     *bad = (int64_t)*b->h_bad;
@@ -751,8 +739,6 @@ int amb_batch_create(const amb_realisation* desc, int64_t count, const double* c
     AMB_CHECK(hipMalloc(&b->d_desc, desc_bytes));
     AMB_CHECK(hipMalloc(&b->d_part, kReduceBlocks * sizeof(double)));
     AMB_CHECK(hipMalloc(&b->d_bad_part, kReduceBlocks * sizeof(unsigned long long)));
-    AMB_CHECK(hipMalloc(&b->d_sum, sizeof(double)));
-    AMB_CHECK(hipMalloc(&b->d_bad, sizeof(unsigned long long)));
     AMB_CHECK(hipHostMalloc(&b->h_sum, sizeof(double), hipHostMallocDefault));
     AMB_CHECK(hipHostMalloc(&b->h_bad, sizeof(unsigned long long), hipHostMallocDefault));
     AMB_CHECK(hipEventCreate(&b->ev0));

@@ -373,30 +373,34 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
     return AMB_OK;
 }
 
-// FP64 sum and non-finite count of the field into h->d_sum and h->d_bad.
-hipError_t enqueue_reduce(amb_handle* h)
+// FP64 sum and non-finite count of the field into *sum and *bad (device or pinned memory).
+hipError_t enqueue_reduce(amb_handle* h, double* sum, unsigned long long* bad)
 {
     const int64_t n = h->ny * h->nx;
     return h->precision == AMB_F32
-               ? launch_reduce_f32(static_cast<const float*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, h->d_sum,
-                                   h->d_bad, h->stream)
-               : launch_reduce_f64(static_cast<const double*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, h->d_sum,
-                                   h->d_bad, h->stream);
+               ? launch_reduce_f32(static_cast<const float*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, sum, bad,
+                                   h->stream)
+               : launch_reduce_f64(static_cast<const double*>(h->buf[h->cur]), n, h->d_part, h->d_bad_part, sum, bad,
+                                   h->stream);
+}
+
+// The last kernel of a reduction writes its two results straight into the handle's pinned
+// memory: two copies of eight bytes after it cost as much as two steps of a small field (a run of
+// 20 steps of 128^2 FP64 192 us with them, 181 without).
+int wait_reduce(amb_handle* h, double* sum, int64_t* bad)
+{
+    const hipError_t e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
+    *sum = *h->h_sum;
+    *bad = (int64_t)*h->h_bad;
+    return AMB_OK;
 }
 
 int reduce_now(amb_handle* h, double* sum, int64_t* bad)
 {
-    hipError_t e = enqueue_reduce(h);
+    const hipError_t e = enqueue_reduce(h, h->h_sum, h->h_bad);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
-    if ((e = hipMemcpyAsync(h->h_sum, h->d_sum, sizeof(double), hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipMemcpyAsync(h->h_bad, h->d_bad, sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream)) !=
-        hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipStreamSynchronize(h->stream)) != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
-    *sum = *h->h_sum;
-    *bad = (int64_t)*h->h_bad;
-    return AMB_OK;
+    return wait_reduce(h, sum, bad);
 }
 
 // Mass and non-finite count after a run of nsteps: the last step of the run wrote one
@@ -412,16 +416,10 @@ int finish_run(amb_handle* h, int64_t nsteps, double* sum, int64_t* bad)
         }
         return rc;
     }
-    hipError_t e = launch_reduce_tiles(h->d_tile_part, h->parts, h->d_sum, h->d_bad, h->stream);
+    const hipError_t e = launch_reduce_tiles(h->d_tile_part, h->parts, h->h_sum, h->h_bad, h->stream);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
-    if ((e = hipMemcpyAsync(h->h_sum, h->d_sum, sizeof(double), hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipMemcpyAsync(h->h_bad, h->d_bad, sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream)) !=
-        hipSuccess)
-        return fail_hip(e, "hipMemcpyAsync");
-    if ((e = hipStreamSynchronize(h->stream)) != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
-    *sum = *h->h_sum;
-    *bad = (int64_t)*h->h_bad;
+    const int rc = wait_reduce(h, sum, bad);
+    if (rc != AMB_OK) return rc;
     h->last_sum = *sum;
     h->last_bad = *bad;
     return AMB_OK;
@@ -499,7 +497,7 @@ int handle_view(amb_handle* h, FieldView* v)
 
 int handle_field_sum(amb_handle* h, const double** sum)
 {
-    const hipError_t e = enqueue_reduce(h);
+    const hipError_t e = enqueue_reduce(h, h->d_sum, h->d_bad);
     if (e != hipSuccess) return fail_hip(e, "reduction launch");
     *sum = h->d_sum;
     return AMB_OK;

@@ -27,8 +27,8 @@ struct StepArgs {
     const T* in;
     T* out;
     int ny, nx;
-    int ntx, nty;     // tiles along x and y
     int seg_rows;     // > 0: strips, this many output rows per workgroup
+    int ntx, nty;     // tiles along x and y
     int xcd_chunk;    // > 0: blockIdx remapped so each XCD gets a contiguous run of tiles
     StepCoef<T> k;
     uint32_t key0, key1;
