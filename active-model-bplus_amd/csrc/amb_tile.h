@@ -17,9 +17,17 @@ constexpr long long kActiveCurrentSites = 2048LL * 2048;
 
 __device__ __forceinline__ int wrap_index(int g, int n)
 {
-    // Exact for any g; one iteration in the common case, several on tiny grids.
-    while (g < 0) g += n;
-    while (g >= n) g -= n;
+    // Exact for any g.  One period to either side covers every grid but the tiniest; the loops,
+    // which the compiler turns into a division each, are left to those.  (With the loops alone a
+    // seam tile spent several hundred cycles on indices before its first load, and a
+    // step lasts as long as its seam tiles: T = 0.05 1024^2 FP32 10.3 -> 9.0 us, 128^2 FP32 5.9 ->
+    // 5.6 us; T = 0 256^2 FP64 5.52 -> 5.26 us.)
+    g += g < 0 ? n : 0;
+    g -= g >= n ? n : 0;
+    if (__builtin_expect((unsigned)g >= (unsigned)n, 0)) {
+        while (g < 0) g += n;
+        while (g >= n) g -= n;
+    }
     return g;
 }
 
