@@ -175,9 +175,6 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
     return best;
 }
 
-// XCD-contiguous tile order: gfx950 dispatches workgroup i to XCD i % 8.
-int xcd_chunk(int nblocks) { return (nblocks % 8 == 0 && nblocks >= 64) ? nblocks / 8 : 0; }
-
 // ---- tuning table: the autotuners' choices, per (precision, grid, noise) ------------
 namespace {
 std::mutex g_tune_mutex;
@@ -262,7 +259,8 @@ StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int nois
     a.ntx = g.ntx;
     a.nty = g.nty;
     a.seg_rows = g.seg_rows;
-    a.xcd_chunk = xcd_chunk(a.ntx * a.nty);
+    a.xcd_chunk = xcd_chunk((int64_t)a.ntx * a.nty);
+    a.ntx_inv = ntx_inverse(a.ntx, a.nty);
     a.k = make_coef<T>(h->stencil, h->model);
     a.key0 = (uint32_t)h->options.seed;
     a.key1 = (uint32_t)(h->options.seed >> 32);

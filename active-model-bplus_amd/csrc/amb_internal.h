@@ -21,7 +21,6 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise);
 bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile);
 void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile);
 int initial_tile(int precision, int64_t ny, int64_t nx, int noise);
-int xcd_chunk(int nblocks);
 
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);

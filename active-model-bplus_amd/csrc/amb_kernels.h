@@ -29,7 +29,8 @@ struct StepArgs {
     int ny, nx;
     int seg_rows;     // > 0: strips, this many output rows per workgroup
     int ntx, nty;     // tiles along x and y
-    int xcd_chunk;    // > 0: blockIdx remapped so each XCD gets a contiguous run of tiles
+    int xcd_chunk;    // tiles per XCD: block b takes tile (b % 8) xcd_chunk + b / 8 (xcd_chunk below)
+    uint32_t ntx_inv; // floor(2^32 / ntx) + 1, or 0 to divide by ntx (tile_row)
     StepCoef<T> k;
     uint32_t key0, key1;
     const long long* step_base;  // device step counter; noise uses *step_base + step_off
@@ -85,6 +86,27 @@ struct StepGrid {
 };
 StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx);
 int device_cus();  // compute units of the current device
+
+// Order of a step's tiles.  gfx950 dispatches block b to XCD b % 8, and neighbouring tiles read
+// each other's rows, so each XCD takes a contiguous run of xcd_chunk(tiles) tiles and finds
+// those rows in its own L2; the grid is 8 xcd_chunk blocks, those without a tile leave at once.
+// In plain order a step is 1 to 1.5 us longer (640^2 in 800 tiles 7.2 us, 608^2 in 722, which
+// no multiple of eight used to leave in plain order, 8.7).  Fields of few tiles keep to as few
+// XCDs as hold them one to a compute unit: 128^2 FP32 T = 0.05 in 32 tiles 4.9 us on one XCD, 5.3
+// on two, 5.5 on eight; FP64 6.4, 6.8, 7.1; from 3/8 of the device on all eight are as fast.
+inline int xcd_chunk(int64_t tiles)
+{
+    const int64_t cus = device_cus();
+    const int xcds = 8 * tiles <= cus ? 1 : 4 * tiles <= cus ? 2 : 8 * tiles <= 3 * cus ? 4 : 8;
+    return (int)((tiles + xcds - 1) / xcds);
+}
+
+// The tile coordinates of index t without a division at the head of every workgroup: exact
+// while t ntx < 2^32, the host passes 0 where that may not hold.
+inline uint32_t ntx_inverse(int64_t ntx, int64_t nty)
+{
+    return ntx > 1 && ntx * nty * ntx < ((int64_t)1 << 32) ? (uint32_t)(((uint64_t)1 << 32) / (uint64_t)ntx) + 1 : 0;
+}
 
 // Launches one fused step.  Returns a hipError_t.
 hipError_t launch_step_f32(const StepArgs<float>& a, int tile, int noise, hipStream_t s);

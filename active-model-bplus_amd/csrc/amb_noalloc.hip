@@ -97,7 +97,8 @@ int run_noalloc(T* field, T* work, int64_t ny, int64_t nx, const amb_stencil& st
     a.ntx = g.ntx;
     a.nty = g.nty;
     a.seg_rows = g.seg_rows;
-    a.xcd_chunk = xcd_chunk(a.ntx * a.nty);
+    a.xcd_chunk = xcd_chunk((int64_t)a.ntx * a.nty);
+    a.ntx_inv = ntx_inverse(a.ntx, a.nty);
     a.k = make_coef<T>(st, md);
     a.key0 = (uint32_t)seed;
     a.key1 = (uint32_t)(seed >> 32);

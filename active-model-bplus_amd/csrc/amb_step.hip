@@ -32,14 +32,19 @@ namespace amb {
 
 // ---- single-field kernel ----------------------------------------------------------
 
+template <typename T>
+__device__ __forceinline__ int tile_row(const StepArgs<T>& p, int t)
+{
+    return p.ntx_inv ? (int)(((uint64_t)(uint32_t)t * p.ntx_inv) >> 32) : t / p.ntx;
+}
+
 template <typename T, int TW, int TH, int NT, int NOISE>
 __global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) void step_kernel(const StepArgs<T> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    // Tile index; with xcd_chunk the round-robin XCD dispatch gets contiguous tiles.
-    int t = blockIdx.x;
-    if (p.xcd_chunk > 0) t = (t & 7) * p.xcd_chunk + (t >> 3);
-    const int ty = t / p.ntx, tx = t - ty * p.ntx;
+    const int t = (blockIdx.x & 7) * p.xcd_chunk + (blockIdx.x >> 3);
+    if (t >= p.ntx * p.nty) return;
+    const int ty = tile_row(p, t), tx = t - ty * p.ntx;
     constexpr bool kPhilox = NOISE == kNoisePhilox || NOISE == kNoisePhiloxOdd;
     const uint64_t step = kPhilox ? (uint64_t)(*p.step_base) + (uint64_t)p.step_off : 0;
     step_tile<T, TW, TH, NT, NOISE>(reinterpret_cast<T*>(smem_raw), p.in, p.out, p.ny, p.nx, tx * TW, ty * TH, p.k,
@@ -58,8 +63,8 @@ __global__ __launch_bounds__((MarchLds<T, NOISE == kNoisePhilox, ACTIVE>::NT),
 void march_kernel(const StepArgs<T> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    int t = blockIdx.x;
-    if (p.xcd_chunk > 0) t = (t & 7) * p.xcd_chunk + (t >> 3);
+    const int t = (blockIdx.x & 7) * p.xcd_chunk + (blockIdx.x >> 3);
+    if (t >= p.ntx * p.nty) return;
     const int sg = t / p.ntx, tx = t - sg * p.ntx;
     const uint64_t step = NOISE == kNoisePhilox ? (uint64_t)(*p.step_base) + (uint64_t)p.step_off : 0;
     const int y0 = sg * p.seg_rows;
@@ -180,8 +185,7 @@ template <typename T, int TW, int TH, int NT, int NOISE>
 static hipError_t launch_one(const StepArgs<T>& a, hipStream_t s)
 {
     using L = Lds<T, TW, TH, NT>;
-    const int nblocks = a.ntx * a.nty;
-    hipLaunchKernelGGL((step_kernel<T, TW, TH, NT, NOISE>), dim3(nblocks), dim3(NT), L::bytes, s, a);
+    hipLaunchKernelGGL((step_kernel<T, TW, TH, NT, NOISE>), dim3(8 * a.xcd_chunk), dim3(NT), L::bytes, s, a);
     return hipGetLastError();
 }
 
@@ -200,7 +204,7 @@ template <typename T, int NOISE, bool ACTIVE>
 static hipError_t launch_march_one(const StepArgs<T>& a, hipStream_t s)
 {
     using L = MarchLds<T, NOISE == kNoisePhilox, ACTIVE>;
-    hipLaunchKernelGGL((march_kernel<T, NOISE, ACTIVE>), dim3(a.ntx * a.nty), dim3(L::NT), L::bytes, s, a);
+    hipLaunchKernelGGL((march_kernel<T, NOISE, ACTIVE>), dim3(8 * a.xcd_chunk), dim3(L::NT), L::bytes, s, a);
     return hipGetLastError();
 }
 
