@@ -122,7 +122,8 @@ int validate_params(int64_t ny, int64_t nx, const amb_stencil* st, const amb_mod
 
 int grid_tiles(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
-// Default tile: in order of preference (AMB_F32_NOISY_ORDER, AMB_F32_NOISELESS_ORDER or
+// The occupancy rule's tile, which options report when none was chosen (such a field runs in
+// run_tile's) and whose tiles bound amb_run_noalloc's fields: in order of preference (AMB_F32_NOISY_ORDER, AMB_F32_NOISELESS_ORDER or
 // AMB_F64_ORDER), the first shape of 256 or more threads whose tiles fill the device's
 // resident workgroups either for at least 8 rounds or in whole-or-mostly-full rounds (a
 // last round under half full leaves most CUs idle for a round).  Fields too small for one
@@ -145,16 +146,17 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
     static constexpr int kNoiselessF32[] = {AMB_F32_NOISELESS_ORDER};
     static constexpr int kF64[] = {AMB_F64_ORDER};
 #define AMB_COUNT_ONE(i, tw, th, nt) +1
-    static_assert(sizeof(kNoisyF32) / sizeof(kNoisyF32[0]) == 0 AMB_F32_TILES(AMB_COUNT_ONE) &&
-                      sizeof(kNoiselessF32) / sizeof(kNoiselessF32[0]) == 0 AMB_F32_TILES(AMB_COUNT_ONE),
-                  "the FP32 orders must list every FP32 tile shape");
-    static_assert(sizeof(kF64) / sizeof(kF64[0]) == 0 AMB_F64_TILES(AMB_COUNT_ONE),
-                  "the FP64 order must list every FP64 tile shape");
+    static_assert(sizeof(kNoisyF32) / sizeof(kNoisyF32[0]) == kWide512F32 &&
+                      sizeof(kNoiselessF32) / sizeof(kNoiselessF32[0]) == kWide512F32 &&
+                      kWide512F32 + 1 == 0 AMB_F32_TILES(AMB_COUNT_ONE),
+                  "the FP32 orders must list every FP32 tile shape but the last");
+    static_assert(sizeof(kF64) / sizeof(kF64[0]) == kWide512F64 && kWide512F64 + 1 == 0 AMB_F64_TILES(AMB_COUNT_ONE),
+                  "the FP64 order must list every FP64 tile shape but the last");
 #undef AMB_COUNT_ONE
     // the index that stands for strips on large fields (step_grid), where they pay
     const int strips = precision == AMB_F32 ? kSquare512F32 : kSquare512F64;
     if (step_grid(precision, strips, noise, ny, nx).seg_rows > 0) return strips;
-    const int n = tile_count(precision);
+    const int n = precision == AMB_F32 ? kWide512F32 : kWide512F64;
     const int* order = precision != AMB_F32 ? kF64 : noise == kNoiseNone ? kNoiselessF32 : kNoisyF32;
     int best = 0;
     double best_gap = 0.0;
@@ -198,11 +200,11 @@ void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile)
 
 // The tile a new integrator starts with: the tuning table's entry when there is one,
 // otherwise the occupancy rule.
-int initial_tile(int precision, int64_t ny, int64_t nx, int noise)
+int initial_tile(int precision, int64_t ny, int64_t nx, int noise, bool* tuned)
 {
     int t = 0;
-    if (tuned_tile(precision, ny, nx, noise, &t)) return t;
-    return default_tile(precision, ny, nx, noise);
+    *tuned = tuned_tile(precision, ny, nx, noise, &t);
+    return *tuned ? t : default_tile(precision, ny, nx, noise);
 }
 
 }  // namespace amb
@@ -235,7 +237,8 @@ struct amb_handle {
     double* d_obs = nullptr;               // 10 n doubles, allocated by the first getter
     double* d_noise = nullptr;             // explicit normals (test mode)
     int64_t noise_steps = 0, noise_used = 0;
-    int tile = 0;                          // index into the precision's tile table
+    int tile = 0;                          // index into the precision's tile table: chosen, or default_tile's
+    bool tile_chosen = false;              // by an option, the tuning table, amb_set_tile or the autotuner
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     int graph_tile[2] = {-1, -1};
     int graph_noise[2] = {-1, -1};
@@ -247,11 +250,14 @@ namespace {
 
 constexpr int kGraphSteps = 32;  // even: a graph returns the field to the buffer it started in
 
+// The tile of the handle's launches.
+int launch_tile(const amb_handle* h) { return h->tile_chosen ? h->tile : run_tile(h->precision, h->ny, h->nx); }
+
 template <typename T>
 StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int noise_mode, bool reduce = false)
 {
     StepArgs<T> a{};
-    const StepGrid g = step_grid(h->precision, h->tile, noise_mode, h->ny, h->nx);
+    const StepGrid g = step_grid(h->precision, launch_tile(h), noise_mode, h->ny, h->nx);
     a.in = static_cast<const T*>(h->buf[parity_in & 1]);
     a.out = static_cast<T*>(h->buf[(parity_in + 1) & 1]);
     a.ny = (int)h->ny;
@@ -278,16 +284,16 @@ StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int nois
 hipError_t launch_step(const amb_handle* h, int parity_in, int step_off, int noise_mode, bool reduce = false)
 {
     if (h->precision == AMB_F32)
-        return launch_step_f32(step_args<float>(h, parity_in, step_off, noise_mode, reduce), h->tile, noise_mode,
+        return launch_step_f32(step_args<float>(h, parity_in, step_off, noise_mode, reduce), launch_tile(h), noise_mode,
                                h->stream);
-    return launch_step_f64(step_args<double>(h, parity_in, step_off, noise_mode, reduce), h->tile, noise_mode,
+    return launch_step_f64(step_args<double>(h, parity_in, step_off, noise_mode, reduce), launch_tile(h), noise_mode,
                            h->stream);
 }
 
 // Workgroups of one step, each writing one partial of the fused finite check.
 int64_t parts_of(const amb_handle* h, int noise)
 {
-    const StepGrid g = step_grid(h->precision, h->tile, noise, h->ny, h->nx);
+    const StepGrid g = step_grid(h->precision, launch_tile(h), noise, h->ny, h->nx);
     return (int64_t)g.ntx * g.nty;
 }
 
@@ -327,7 +333,7 @@ int build_graph(amb_handle* h, int parity, int noise_mode)
     if (e != hipSuccess) return fail_hip(e, "hipGraphInstantiate");
     if (h->graph[parity]) (void)hipGraphExecDestroy(h->graph[parity]);
     h->graph[parity] = exec;
-    h->graph_tile[parity] = h->tile;
+    h->graph_tile[parity] = launch_tile(h);
     h->graph_noise[parity] = noise_mode;
     return AMB_OK;
 }
@@ -350,7 +356,7 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
         }
         if (left >= kGraphSteps) {
             const int p = h->cur;
-            if (!h->graph[p] || h->graph_tile[p] != h->tile || h->graph_noise[p] != mode) {
+            if (!h->graph[p] || h->graph_tile[p] != launch_tile(h) || h->graph_noise[p] != mode) {
                 const int rc = build_graph(h, p, mode);
                 if (rc != AMB_OK) return rc;
             }
@@ -615,8 +621,10 @@ int amb_create(const double* field, int64_t ny, int64_t nx, const amb_stencil* s
     } while (0)
     AMB_CHECK(hipGetDevice(&h->device));
     AMB_CHECK(prepare_step_kernels());
+    h->tile_chosen = opt.tile > 0;
     h->tile = opt.tile > 0 ? opt.tile - 1
-                           : initial_tile(opt.precision, ny, nx, model->T > 0.0 ? kNoisePhilox : kNoiseNone);
+                           : initial_tile(opt.precision, ny, nx, model->T > 0.0 ? kNoisePhilox : kNoiseNone,
+                                          &h->tile_chosen);
     AMB_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     AMB_CHECK(hipMalloc(&h->buf[0], n * h->esize));
     AMB_CHECK(hipMalloc(&h->buf[1], n * h->esize));
@@ -809,6 +817,7 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
         int t = 0;
         if (tuned_tile(h->precision, h->ny, h->nx, mode0, &t)) {
             h->tile = t;
+            h->tile_chosen = true;
             if (chosen) *chosen = t;
             return AMB_OK;
         }
@@ -841,6 +850,7 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
         trial.d_step = step;
         trial.stream = h->stream;
         trial.tile = t;
+        trial.tile_chosen = true;
         for (int k = 0; k <= reps && e == hipSuccess; ++k) {
             if (k == 1) e = hipEventRecord(h->ev0, h->stream);
             if (e == hipSuccess) e = launch_step(&trial, k, 0, mode);
@@ -860,6 +870,7 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
     trial.stream = nullptr;
     if (e != hipSuccess) return fail_hip(e, "autotune");
     h->tile = best_t;
+    h->tile_chosen = true;
     record_tile(h->precision, h->ny, h->nx, mode0, best_t);
     if (chosen) *chosen = best_t;
     return AMB_OK;
@@ -918,6 +929,7 @@ int amb_set_tile(amb_handle* h, int index)
     if (!h) return fail(AMB_E_ARG, "handle must not be null");
     if (index < 0 || index >= tile_count(h->precision)) return fail(AMB_E_ARG, "tile index out of range");
     h->tile = index;
+    h->tile_chosen = true;
     return AMB_OK;
 }
 

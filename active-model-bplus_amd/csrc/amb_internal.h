@@ -20,7 +20,7 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise);
 // The autotuners' table (process-wide): lookup, record, and the tile a new field starts with.
 bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile);
 void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile);
-int initial_tile(int precision, int64_t ny, int64_t nx, int noise);
+int initial_tile(int precision, int64_t ny, int64_t nx, int noise, bool* tuned);
 
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);

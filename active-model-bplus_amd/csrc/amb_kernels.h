@@ -52,8 +52,8 @@ struct TileShape {
 
 // Compiled tile configurations (index = autotuner choice): X(index, TW, TH, NT).  The
 // default tile follows an order of preference per kernel (default_tile in amb_capi.hip).
-#define AMB_F32_TILES(X) X(0, 32, 48, 512) X(1, 32, 24, 256) X(2, 32, 32, 256) X(3, 64, 32, 512) X(4, 64, 16, 256) X(5, 32, 16, 256) X(6, 16, 16, 128) X(7, 16, 8, 128) X(8, 8, 8, 64) X(9, 32, 32, 512)
-#define AMB_F64_TILES(X) X(0, 32, 32, 256) X(1, 64, 16, 256) X(2, 32, 16, 256) X(3, 32, 32, 512) X(4, 16, 16, 128) X(5, 16, 8, 128) X(6, 8, 8, 64)
+#define AMB_F32_TILES(X) X(0, 32, 48, 512) X(1, 32, 24, 256) X(2, 32, 32, 256) X(3, 64, 32, 512) X(4, 64, 16, 256) X(5, 32, 16, 256) X(6, 16, 16, 128) X(7, 16, 8, 128) X(8, 8, 8, 64) X(9, 32, 32, 512) X(10, 32, 16, 512)
+#define AMB_F64_TILES(X) X(0, 32, 32, 256) X(1, 64, 16, 256) X(2, 32, 16, 256) X(3, 32, 32, 512) X(4, 16, 16, 128) X(5, 16, 8, 128) X(6, 8, 8, 64) X(7, 32, 16, 512)
 constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threads
 // FP32 orders of preference, measured on MI355X (the times below predate the step's wave
 // priorities, which took 2-4% off every shape).  Noisy: 32x32 tiles of 512 threads are
@@ -72,6 +72,23 @@ constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threa
 // 321.0 / 213.2 us for 256 threads, both before the fitted noise polynomials and the priorities); 16x8 serves the smallest fields (256^2: 5.56 us, 16x16
 // 5.77 us, 8x8 5.88 us).
 #define AMB_F64_ORDER 3, 0, 2, 1, 4, 5, 6
+
+// The tile that a field runs in when none was chosen: 32x16 tiles of 512 threads while one
+// round of them holds the field, else 32x32 tiles of 512 threads, or strips (step_grid).  us a
+// step, 32x16 / 32x32 / the tile of the orders above:
+//   side      FP32 T = 0.05        FP32 T = 0           FP64 T = 0.05        FP64 T = 0
+//   64        4.41 / 5.26 / 4.89   3.64 / 4.59 / 4.05   5.64 / 7.16 / 6.16   4.48 / 5.41 / 4.27
+//   128       4.76 / 5.44 / 5.54   3.89 / 4.79 / 4.43   6.28 / 7.26 / 7.17   4.63 / 5.48 / 4.76
+//   256       5.31 / 5.89 / 5.91   4.31 / 5.24 / 4.73   7.00 / 8.02 / 7.96   5.08 / 6.15 / 5.19
+//   512       5.96 / 6.08 / 6.08   4.85 / 5.40 / 5.40   8.33 / 8.00 / 8.00   6.23 / 6.20 / 6.20
+//   608       6.84 / 7.52 / 7.77   5.72 / 6.55 / 6.78   10.1 / 10.6 / 10.6   7.82 / 8.34 / 8.34
+//   704       7.40 / 7.37 / 9.46   6.25 / 6.47 / 8.40   13.5 / 10.6 / 12.6   9.60 / 8.30 / 9.34
+//   768       9.21 / 7.79 / 9.88   7.29 / 6.93 / 8.38   15.1 / 14.7 / 16.0   11.1 / 11.2 / 11.4
+//   1088      14.4 / 11.3 / 15.5   11.2 / 10.2 / 13.4   26.3 / 22.0 / 26.5   18.5 / 16.5 / 19.6
+// (a round is four workgroups per compute unit in FP32, three in FP64).  FP64 32x32 tiles that
+// fit one to a compute unit beat more than 1.5 32x16 tiles to each (448^2 8.30 / 8.46).
+constexpr int kWide512F32 = 10, kWide512F64 = 7;
+int run_tile(int precision, int64_t ny, int64_t nx);
 
 // Tile shapes compiled per precision (index = autotuner choice).
 int tile_count(int precision);

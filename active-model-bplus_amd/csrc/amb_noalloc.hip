@@ -90,7 +90,10 @@ int run_noalloc(T* field, T* work, int64_t ny, int64_t nx, const amb_stencil& st
     double* sum = reinterpret_cast<double*>(base + 16);
     unsigned long long* bad = reinterpret_cast<unsigned long long*>(base + 24);
     double* part = reinterpret_cast<double*>(base + kPartOffset);
-    const StepGrid g = step_grid(sizeof(T) == 4 ? AMB_F32 : AMB_F64, tile, noise, ny, nx);
+    const int precision = sizeof(T) == 4 ? AMB_F32 : AMB_F64;
+    StepGrid g = step_grid(precision, run_tile(precision, ny, nx), noise, ny, nx);
+    if ((int64_t)g.ntx * g.nty <= kNoAllocMaxTiles) tile = run_tile(precision, ny, nx);
+    else g = step_grid(precision, tile, noise, ny, nx);
     StepArgs<T> a{};
     a.ny = (int)ny;
     a.nx = (int)nx;

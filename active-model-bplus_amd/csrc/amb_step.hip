@@ -181,6 +181,19 @@ StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx)
     return g;
 }
 
+int run_tile(int precision, int64_t ny, int64_t nx)
+{
+    const int wide = precision == 32 ? kWide512F32 : kWide512F64, square = precision == 32 ? kSquare512F32 : kSquare512F64;
+    auto tiles = [&](int tile) {
+        const TileShape t = tile_shape(precision, tile);
+        return ((nx + t.tw - 1) / t.tw) * ((ny + t.th - 1) / t.th);
+    };
+    const int64_t cus = device_cus(), n = tiles(wide);
+    if (n > (precision == 32 ? 4 : 3) * cus) return square;
+    if (precision == 64 && tiles(square) <= cus && 2 * n > 3 * cus) return square;
+    return wide;
+}
+
 template <typename T, int TW, int TH, int NT, int NOISE>
 static hipError_t launch_one(const StepArgs<T>& a, hipStream_t s)
 {

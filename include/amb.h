@@ -52,7 +52,8 @@ typedef struct {
     int precision;     /* AMB_F64 or AMB_F32: storage and arithmetic of the field */
     uint64_t seed;     /* Philox key of the conserved noise */
     int64_t timestep;  /* initial step counter (exact resume: field, timestep, seed) */
-    int tile;          /* 0 = default tile; k > 0 selects tile index k-1 (see amb_tile_count) */
+    int tile;          /* k > 0 selects tile index k-1 (see amb_tile_count); 0 = the library chooses among its
+                          tiles and strips by size, and amb_get_options names the occupancy rule's index */
 } amb_options;
 
 typedef struct amb_handle amb_handle;

@@ -90,3 +90,21 @@ def test_resident_members_equal_integrators(amb, precision, shapes):
         sim = amb.Integrator(f, st, models[i], seed=i, precision=precision)
         sim.run(37)
         np.testing.assert_array_equal(ens.field(i), sim.field, err_msg=str((i, f.shape)))
+
+
+# The tile of a field for which none was chosen: 32x16 tiles of 512 threads up to one round of the
+# device, 32x32 tiles beyond, on one, two, four and eight XCDs, tile counts that are and are not
+# multiples of eight, a last row and column of tiles that are whole, one site and partly filled.
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("shape", [(8, 9), (16, 32), (130, 127), (161, 161), (193, 200), (289, 257), (448, 450),
+                                   (640, 641), (900, 868)])
+def test_unchosen_tile_equals_chosen(amb, precision, shape):
+    phi = 0.05 * np.random.default_rng(shape[0]).normal(size=shape)
+    st = amb.Stencil(5e-3, 1, 1.25)
+    for temperature in (0.0, 0.05):
+        md = amb.Model(-0.25, 0, 0.25, 1, 0.5, -1, temperature)
+        sims = [amb.Integrator(phi, st, md, seed=3, precision=precision, tile=tile) for tile in (0, 1)]
+        for sim in sims:
+            sim.run(35)  # a graph of 32 steps and three launches
+        np.testing.assert_array_equal(sims[0].field, sims[1].field, err_msg=str((shape, temperature)))
+        assert sims[0].last_mass()[0] == pytest.approx(sims[1].last_mass()[0], rel=1e-12, abs=1e-9)
