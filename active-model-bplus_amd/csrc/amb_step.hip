@@ -149,16 +149,17 @@ static int64_t march_cost(int64_t ny, int strips, int slots, int* seg_rows)
 // Strips take the place of 32x32 tiles of 512 threads where the device's lanes are busy enough
 // with them: the sites over the lane-rows (slots x march_cost x columns of a strip) that their
 // workgroups run through.  A step at T = 0.05 and T = 0, tiles -> strips in us, around the line:
-//   share      FP32 noisy          FP32 quiet          FP64 noisy          FP64 quiet
-//   0.25-0.3   1024^2 11.0 -> 13.8 1024^2  9.4 -> 14.6
-//   0.38-0.42                      1024x2048 15.2->16.5 1024^2 19.7 -> 23.5 1024^2 15.4 -> 21.0
-//   0.47-0.49  1024x2048 18.1->18.3 1024x3072 20.7->20.7 1200^2 29.6 -> 26.2 1200^2 23.5 -> 23.1
-//   0.50-0.54  1664^2 22.0 -> 20.9 1792^2 21.1 -> 18.9 2048x1024 35.5->33.5 2048x1024 26.4->30.6
-//   0.57-0.63  2048^2 30.0 -> 25.2 2048^2 26.5 -> 24.7 1536^2 40.1 -> 33.8 1664^2 40.7 -> 34.2
-//   0.70-0.86  4096^2 102 -> 71.3  4096^2 87.6 -> 69.7 4096^2 242 -> 169   4096^2 173 -> 161
-// Fields whose columns do not split into fours gain more (2050 x 2049 FP32 45.3 -> 26.1).
+//   share      FP32 noisy           FP32 quiet           FP64 noisy           FP64 quiet
+//   0.25-0.31  1024^2 9.9 -> 13.3   1024^2 8.8 -> 12.2
+//   0.38-0.42  1200^2 13.5 -> 14.9  1440^2 14.8 -> 15.3  1024^2 18.6 -> 23.2  1024^2 14.4 -> 20.3
+//   0.46-0.49  1536^2 18.5 -> 18.9  1664^2 18.6 -> 18.5  1200^2 24.8 -> 25.0  1200^2 19.1 -> 22.3
+//   0.50-0.54  1664^2 21.3 -> 20.2  1800^2 21.0 -> 20.5  1300^2 29.3 -> 27.5  1300^2 21.6 -> 24.5
+//   0.57-0.63  2048^2 28.7 -> 25.0  2048^2 25.4 -> 24.4  1536^2 38.4 -> 34.0  1600^2 30.6 -> 32.3
+//   0.67-0.70  2560^2 43.9 -> 33.6  2560^2 38.9 -> 33.3  1792^2 51.6 -> 40.4  1800^2 38.0 -> 38.2
+//   0.75-0.86  4096^2 100 -> 73     4096^2 88 -> 71      4096^2 234 -> 177    4096^2 170 -> 162
+// Fields whose columns do not split into fours gain more (1787 x 1801 FP64 56.4 -> 44.3).
 // Every field's 32-bit byte offsets must reach it, and an explicit noise buffer takes tiles.
-constexpr double kStripShareF32[2] = {0.495, 0.48}, kStripShareF64[2] = {0.63, 0.482};  // quiet, noisy
+constexpr double kStripShareF32[2] = {0.495, 0.51}, kStripShareF64[2] = {0.69, 0.5};  // quiet, noisy
 
 StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx)
 {

@@ -38,7 +38,7 @@ def test_ragged_columns_match_oracle(amb, oracle, shape):
 @pytest.mark.parametrize("precision,shape,temperature", [
     (32, (1787, 1801), 0.0), (32, (2048, 2016), 0.0),
     (32, (1795, 1793), 0.05), (32, (2051, 2047), 0.05), (32, (2049, 2128), 0.05),
-    (64, (1201, 1203), 0.05), (64, (1667, 1665), 0.0), (64, (61, 40000), 0.05)])
+    (64, (1399, 1401), 0.05), (64, (2203, 2201), 0.0), (64, (120, 40000), 0.05)])
 def test_strips_equal_tiles(amb, precision, shape, temperature):
     """The same bits as 32x24 (FP32) or 64x16 (FP64) tiles after 5 steps, and a fused mass and
     finite count equal to a full read of the field."""
