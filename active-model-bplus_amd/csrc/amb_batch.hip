@@ -374,6 +374,7 @@ struct amb_batch {
     hipEvent_t fork = nullptr;
     std::vector<hipStream_t> branch;      // capture branch per tile-shape group and resident group
     std::vector<hipEvent_t> branch_done;
+    HostStage stage;                      // getters
     double* d_part = nullptr;
     unsigned long long* d_bad_part = nullptr;
     double* h_sum = nullptr;               // pinned: reductions write their results here
@@ -412,6 +413,7 @@ void release(amb_batch* b)
     for (hipEvent_t ev : b->branch_done) (void)hipEventDestroy(ev);
     for (hipStream_t st : b->branch) (void)hipStreamDestroy(st);
     if (b->fork) (void)hipEventDestroy(b->fork);
+    release(b->stage);
     if (b->h_sum) (void)hipHostFree(b->h_sum);
     if (b->h_bad) (void)hipHostFree(b->h_bad);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -819,17 +821,8 @@ int amb_batch_get_field(amb_batch* b, int64_t index, double* out)
     if (!b || !out) return fail(AMB_E_ARG, "batch and out must not be null");
     if (index < 0 || index >= (int64_t)b->desc.size()) return fail(AMB_E_ARG, "realisation index out of range");
     const size_t n = (size_t)(b->desc[index].ny * b->desc[index].nx);
-    hipError_t e = hipStreamSynchronize(b->stream);
-    if (e != hipSuccess) return fail_hip(e, "hipStreamSynchronize");
-    if (b->precision == AMB_F32) {
-        std::vector<float> tmp(n);
-        e = hipMemcpy(tmp.data(), static_cast<const float*>(b->buf[b->cur]) + b->off[index], n * sizeof(float),
-                      hipMemcpyDeviceToHost);
-        for (size_t i = 0; i < n; ++i) out[i] = (double)tmp[i];
-    } else {
-        e = hipMemcpy(out, static_cast<const double*>(b->buf[b->cur]) + b->off[index], n * sizeof(double),
-                      hipMemcpyDeviceToHost);
-    }
+    const hipError_t e = copy_out(b->stage, static_cast<const char*>(b->buf[b->cur]) + (size_t)b->off[index] * b->esize,
+                                  (int64_t)n, b->precision, out, b->stream);
     return e == hipSuccess ? AMB_OK : fail_hip(e, "hipMemcpy (field download)");
 }
 

@@ -25,6 +25,18 @@ int initial_tile(int precision, int64_t ny, int64_t nx, int noise, bool* tuned);
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);
 
+// amb_get_observable with a current's x component to `second`, not after the y component.
+extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
+
+// Two pinned pieces through which results go to the caller's memory, made on first use.
+struct HostStage {
+    void* piece[2] = {nullptr, nullptr};
+    hipEvent_t filled[2] = {nullptr, nullptr};
+};
+// n values of a field (FP32 or FP64) at dev, as doubles to out, after the work on `s`.
+hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, double* out, hipStream_t s);
+void release(HostStage& st);
+
 // Access to an integrator's state for other parts of the library (the surrogate).
 struct FieldView {
     void* cur;          // current field (ny*nx elements of the handle's precision)

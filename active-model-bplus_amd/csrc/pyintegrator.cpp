@@ -19,6 +19,9 @@
 
 #include "amb.h"
 
+// libamb.so: amb_get_observable with a current's two components to separate arrays.
+extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
+
 namespace py = pybind11;
 
 namespace {
@@ -127,14 +130,11 @@ class Integrator {
     // Currents as [y, x] lists of (ny, nx) arrays, as the reference's HostCurrent.
     py::list vector(int which) const
     {
-        py::array_t<double> both({(py::ssize_t)2, ny_, nx_});
-        check(amb_get_observable(h_, which, both.mutable_data()));
+        py::array_t<double> y({ny_, nx_}), x({ny_, nx_});
+        check(amb_get_observable_parts(h_, which, y.mutable_data(), x.mutable_data()));
         py::list out;
-        for (py::ssize_t c = 0; c < 2; ++c) {
-            py::array_t<double> comp({ny_, nx_});
-            std::memcpy(comp.mutable_data(), both.data() + c * ny_ * nx_, sizeof(double) * ny_ * nx_);
-            out.append(comp);
-        }
+        out.append(y);
+        out.append(x);
         return out;
     }
 
