@@ -378,7 +378,7 @@ struct amb_batch {
     double* d_part = nullptr;
     unsigned long long* d_bad_part = nullptr;
     double* h_sum = nullptr;               // pinned: reductions write their results here
-    unsigned long long* h_bad = nullptr;
+    unsigned long long* h_bad = nullptr;   // after h_sum
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
@@ -415,7 +415,6 @@ void release(amb_batch* b)
     if (b->fork) (void)hipEventDestroy(b->fork);
     release(b->stage);
     if (b->h_sum) (void)hipHostFree(b->h_sum);
-    if (b->h_bad) (void)hipHostFree(b->h_bad);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -741,8 +740,8 @@ int amb_batch_create(const amb_realisation* desc, int64_t count, const double* c
     AMB_CHECK(hipMalloc(&b->d_desc, desc_bytes));
     AMB_CHECK(hipMalloc(&b->d_part, kReduceBlocks * sizeof(double)));
     AMB_CHECK(hipMalloc(&b->d_bad_part, kReduceBlocks * sizeof(unsigned long long)));
-    AMB_CHECK(hipHostMalloc(&b->h_sum, sizeof(double), hipHostMallocDefault));
-    AMB_CHECK(hipHostMalloc(&b->h_bad, sizeof(unsigned long long), hipHostMallocDefault));
+    AMB_CHECK(hipHostMalloc(&b->h_sum, 2 * sizeof(double), hipHostMallocDefault));
+    b->h_bad = reinterpret_cast<unsigned long long*>(b->h_sum + 1);
     AMB_CHECK(hipEventCreate(&b->ev0));
     AMB_CHECK(hipEventCreate(&b->ev1));
     const long long zero = 0;

@@ -287,11 +287,11 @@ struct amb_handle {
     double* d_tile_part = nullptr;         // (sum, non-finite count) per tile, written by a run's last step
     int64_t parts = 0;                     // how many of them the last step wrote
     double* d_sum = nullptr;
-    unsigned long long* d_bad = nullptr;
+    unsigned long long* d_bad = nullptr;   // after d_sum
     double last_sum = 0.0;                 // mass and non-finite count found by the last amb_run
     int64_t last_bad = 0;
     double* h_sum = nullptr;               // pinned
-    unsigned long long* h_bad = nullptr;   // pinned
+    unsigned long long* h_bad = nullptr;   // after h_sum
     double* d_obs = nullptr;               // 10 n doubles, allocated by the first getter
     double* d_noise = nullptr;             // explicit normals (test mode)
     int64_t noise_steps = 0, noise_used = 0;
@@ -495,11 +495,10 @@ void release(amb_handle* h)
     drop_graphs(h);
     sk_cache_free(h->sk);
     for (void* p : {h->buf[0], h->buf[1], (void*)h->d_step, (void*)h->d_part, (void*)h->d_bad_part,
-                    (void*)h->d_tile_part, (void*)h->d_sum, (void*)h->d_bad, (void*)h->d_obs, (void*)h->d_noise})
+                    (void*)h->d_tile_part, (void*)h->d_sum, (void*)h->d_obs, (void*)h->d_noise})
         if (p) (void)hipFree(p);
     release(h->stage);
     if (h->h_sum) (void)hipHostFree(h->h_sum);
-    if (h->h_bad) (void)hipHostFree(h->h_bad);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -701,10 +700,11 @@ int amb_create(const double* field, int64_t ny, int64_t nx, const amb_stencil* s
         }
         AMB_CHECK(hipMalloc(&h->d_tile_part, (size_t)most * 2 * sizeof(double)));
     }
-    AMB_CHECK(hipMalloc(&h->d_sum, sizeof(double)));
-    AMB_CHECK(hipMalloc(&h->d_bad, sizeof(unsigned long long)));
-    AMB_CHECK(hipHostMalloc(&h->h_sum, sizeof(double), hipHostMallocDefault));
-    AMB_CHECK(hipHostMalloc(&h->h_bad, sizeof(unsigned long long), hipHostMallocDefault));
+    static_assert(sizeof(double) == sizeof(unsigned long long), "one allocation for both results");
+    AMB_CHECK(hipMalloc(&h->d_sum, 2 * sizeof(double)));
+    h->d_bad = reinterpret_cast<unsigned long long*>(h->d_sum + 1);
+    AMB_CHECK(hipHostMalloc(&h->h_sum, 2 * sizeof(double), hipHostMallocDefault));
+    h->h_bad = reinterpret_cast<unsigned long long*>(h->h_sum + 1);
     AMB_CHECK(hipEventCreate(&h->ev0));
     AMB_CHECK(hipEventCreate(&h->ev1));
     const long long step0 = (long long)h->timestep;
