@@ -120,23 +120,24 @@ int validate_params(int64_t ny, int64_t nx, const amb_stencil* st, const amb_mod
     return AMB_OK;
 }
 
-// Fields above 256 KB of doubles go through two pinned pieces: the copy engine fills one while the
+// Fields above one piece of doubles go through two pinned pieces: the copy engine fills one while the
 // host empties the other into the caller's memory, whose first touch and the widening of FP32
 // values are what takes the time.  A copy to pageable memory stages one piece after the other,
 // and FP32 fields took a vector of their own: a run of 400 steps of 1024^2 FP32 and its field
 // 4.23 ms, now 4.03; a run of 640 steps of 48 members and their fields 22.2 ms, now 20.7.  Small
-// fields are quicker copied at once (128^2 FP64 by 9 us), and four threads, each with pieces
+// fields are quicker copied at once (128^2 FP64 by 9 us; a copy on the stream that is not pinned
+// also made the next integrator 45 us slower to create), and four threads, each with pieces
 // of its own, gained on mu and J of 1024^2 FP64 (2.0 -> 1.8 ms) but lost on its FP32 field (0.3 ms).
 hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, double* out, hipStream_t s)
 {
     constexpr size_t kPiece = (size_t)1 << 20;
     const size_t esize = precision == AMB_F32 ? sizeof(float) : sizeof(double);
     hipError_t e = hipSuccess;
-    if (n <= (1 << 15)) {
+    if (n <= (int64_t)(kPiece / sizeof(double))) {
         std::vector<float> tmp(precision == AMB_F32 ? n : 0);
         void* dst = precision == AMB_F32 ? static_cast<void*>(tmp.data()) : out;
-        if ((e = hipMemcpyAsync(dst, dev, (size_t)n * esize, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+        if ((e = hipMemcpy(dst, dev, (size_t)n * esize, hipMemcpyDeviceToHost)) != hipSuccess) return e;
         for (size_t i = 0; i < tmp.size(); ++i) out[i] = (double)tmp[i];
         return hipSuccess;
     }
