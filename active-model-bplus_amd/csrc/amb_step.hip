@@ -4,8 +4,9 @@
 // (8 B per site in FP32, 16 B in FP64).  The reference needs three launches per
 // step and ~280 B per site (src/integrator.cu:46-262, host loop :507-518).
 //
-// Per tile of TW x TH outputs (one workgroup of NT threads; 32x32 tiles of 512 threads,
-// eight wave64s, on large fields):
+// Large fields run in strips (amb_march.h), the others in tiles.  Per tile of TW x TH outputs
+// (one workgroup of NT threads; 32x16 tiles of 512 threads, eight wave64s, on small fields, 32x32
+// ones beyond):
 //   stage 0  phi on rows [-9, TH+9) x cols [-9, TW+9) -> LDS (periodic wrap)
 //   stage A  on the cross-shaped halo region: G3x phi, G3y phi, L3 phi, then
 //            mu_p (rows/cols +-8), mu_a = lambda|G3 phi|^2 and the circulating current
@@ -52,11 +53,11 @@ __global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) vo
 }
 
 // ---- strips (amb_march.h) ------------------------------------------------------
-// Bound by vector issue: at 4096^2 FP32 noisy 140 instructions a site against 219 for 32x32
+// Bound by vector issue: at 4096^2 FP32 noisy 141 instructions a site against 222 for 32x32
 // tiles (which compute mu_p, the noise and the currents of their halos about twice over), the
-// vector units busy 90% of the time; 102 -> 71 us a step, FP64 242 -> 169 us.  The noiseless
-// kernel runs 100 a site (tiles 173) but its role B, a chain of 59 a row, leaves them idle a
-// third of the time; 87.6 -> 69.7 us.
+// vector units busy 88% of the time; 102 -> 65 us a step, FP64 242 -> 168 us.  The noiseless
+// kernel runs 114 a site (tiles 173) but its role B, a chain of 59 a row, leaves them idle a
+// third of the time; 87.6 -> 64 us.
 template <typename T, int NOISE, bool ACTIVE>
 __global__ __launch_bounds__((MarchLds<T, NOISE == kNoisePhilox, ACTIVE>::NT),
                              (MarchLds<T, NOISE == kNoisePhilox, ACTIVE>::min_waves))
