@@ -141,6 +141,7 @@ hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, do
         for (size_t i = 0; i < tmp.size(); ++i) out[i] = (double)tmp[i];
         return hipSuccess;
     }
+    const std::lock_guard<std::mutex> lock(st.turn);
     for (int k = 0; k < 2; ++k) {
         if (!st.piece[k]) e = hipHostMalloc(&st.piece[k], kPiece, hipHostMallocDefault);
         if (e == hipSuccess && !st.filled[k]) e = hipEventCreateWithFlags(&st.filled[k], hipEventDisableTiming);
@@ -175,8 +176,9 @@ void release(HostStage& st)
     for (int k = 0; k < 2; ++k) {
         if (st.piece[k]) (void)hipHostFree(st.piece[k]);
         if (st.filled[k]) (void)hipEventDestroy(st.filled[k]);
+        st.piece[k] = nullptr;
+        st.filled[k] = nullptr;
     }
-    st = HostStage{};
 }
 
 int grid_tiles(int64_t n, int t) { return (int)((n + t - 1) / t); }

@@ -1,6 +1,7 @@
 // amb_internal.h -- helpers shared by the host runtime's translation units (internal).
 #pragma once
 
+#include <mutex>
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -28,8 +29,10 @@ StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);
 // amb_get_observable with a current's x component to `second`, not after the y component.
 extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
 
-// Two pinned pieces through which results go to the caller's memory, made on first use.
+// Two pinned pieces through which results go to the caller's memory, made on first use.  Getters
+// of one handle may be called from several threads; they take turns.
 struct HostStage {
+    std::mutex turn;
     void* piece[2] = {nullptr, nullptr};
     hipEvent_t filled[2] = {nullptr, nullptr};
 };
