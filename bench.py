@@ -34,8 +34,8 @@ sys.path.insert(0, os.path.join(REPO, "active-model-bplus_amd"))
 sys.path.insert(0, REPO)
 
 HBM_PEAK_GBS = 8000.0
-TRAFFIC_PROFILE = {"c3": "step_c3_fp32_4096", "c3x8192": "step_c3_fp32_8192"}
-VALU_PROFILE = {"c3": "step_c3_fp32_4096"}
+TRAFFIC_PROFILE = {"c3": "step_c3_fp32_4096_strips", "c3x8192": "step_c3_fp32_8192"}
+VALU_PROFILE = {"c3": "step_c3_fp32_4096_strips"}
 # Non-packed FP32 vector issue rate of MI355X: 256 CUs x 4 SIMDs x 16 lanes at 2.4 GHz.
 VALU_ISSUE_PEAK = 256 * 64 * 2.4e9
 METRIC = "site-updates/s, % HBM peak; batched vs plain; surrogate speedup at ≤2% S(k) err"
