@@ -440,6 +440,9 @@ std::vector<int2> tile_list(const amb_batch* b, const std::vector<int>& members,
     return out;
 }
 
+// The noise mode of the kernel that a member runs.
+int member_noise(const amb_realisation& m) { return m.model.T > 0.0 ? philox_mode(m.nx) : kNoiseNone; }
+
 int rebuild_groups(amb_batch* b)
 {
     drop_graphs(b);
@@ -448,7 +451,7 @@ int rebuild_groups(amb_batch* b)
     std::map<std::pair<int, bool>, std::vector<int>> kept;  // (noise mode, whole) -> resident members
     for (size_t r = 0; r < b->desc.size(); ++r) {
         const amb_realisation& m = b->desc[r];
-        const int noise = m.model.T > 0.0 ? philox_mode(m.nx) : kNoiseNone;
+        const int noise = member_noise(m);
         if (b->resident_on && fits_resident(b->precision, m.ny, m.nx)) {
             kept[{noise, resident_whole(b->precision, m.ny, m.nx)}].push_back((int)r);
         } else {
@@ -905,8 +908,7 @@ int amb_batch_autotune(amb_batch* b, int reps, int* chosen)
     for (int r : b->resident) is_resident[r] = true;
     for (size_t r = 0; r < b->desc.size(); ++r)
         if (!is_resident[r])
-            classes[{b->desc[r].ny, b->desc[r].nx, b->desc[r].model.T > 0.0 ? kNoisePhilox : kNoiseNone}].push_back(
-                (int)r);
+            classes[{b->desc[r].ny, b->desc[r].nx, member_noise(b->desc[r])}].push_back((int)r);
     void* saved = nullptr;
     if ((e = hipMalloc(&saved, (size_t)b->total * b->esize)) != hipSuccess) return fail_hip(e, "hipMalloc");
     e = hipMemcpy(saved, b->buf[b->cur], (size_t)b->total * b->esize, hipMemcpyDeviceToDevice);

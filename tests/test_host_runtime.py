@@ -1,0 +1,75 @@
+"""The library's host code over a HIP runtime on the CPU (native/hip_stub.cpp): which kernels it
+launches, on which device it makes its events, what it does with errors.  Each case runs in a process
+of its own, where the stub is loaded ahead of the library."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, json, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import activemodelbplus.integrator as amb
+from activemodelbplus import tuning
+stub.stub_launch.restype = ctypes.c_char_p
+
+def launches():
+    out = []
+    for i in range(stub.stub_launches()):
+        b, t, l = ctypes.c_uint(), ctypes.c_uint(), ctypes.c_size_t()
+        name = stub.stub_launch(i, ctypes.byref(b), ctypes.byref(t), ctypes.byref(l)).decode()
+        out.append((name, b.value, t.value, l.value))
+    return out
+
+def steps():  # names of the step kernels launched since the last call
+    out = [name for name, *_ in launches() if "step_kernel" in name or "march_kernel" in name]
+    stub.stub_clear()
+    return out
+
+def model(T):
+    return amb.Model(-0.25, 0, 0.25, 1, 0.5, -1, T)
+
+stencil = amb.Stencil(5e-3, 1, 1)
+"""
+
+
+@pytest.fixture(scope="module")
+def on_stub(tmp_path_factory):
+    """on_stub(code): what the code, run on the stub, prints as its last line (JSON)."""
+    lib = str(tmp_path_factory.mktemp("hip") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "native", "hip_stub.cpp"), "-o", lib], check=True)
+
+    def run(code):
+        res = subprocess.run([sys.executable, "-c", PRELUDE + code, lib, os.path.join(REPO, "active-model-bplus_amd")],
+                             capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stderr[-2000:]
+        return json.loads(res.stdout.strip().splitlines()[-1])
+
+    return run
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_ensemble_autotune_times_the_kernels_that_run(on_stub, precision):
+    """Members with noise on columns that do and do not split into fours have kernels of their own
+    (noise modes 1 and 3); the autotuner times the one that each member runs."""
+    timed, ran = on_stub(f"""
+fields = [np.zeros((200, 201)), np.zeros((200, 200)), np.zeros((200, 199))]
+ens = amb.Ensemble(fields, stencil, [model(0.05), model(0.05), model(0.0)], [1, 2, 3], precision={precision})
+assert ens.resident_count == 0
+steps()
+ens.autotune(1)
+timed = steps()
+ens.run(1)
+mode = lambda names: sorted(set(n.split("ELi")[3][0] for n in names))
+print(json.dumps([mode(timed), mode(steps())]))
+""")
+    assert ran == ["0", "1", "3"]
+    assert timed == ran
