@@ -120,6 +120,24 @@ int validate_params(int64_t ny, int64_t nx, const amb_stencil* st, const amb_mod
     return AMB_OK;
 }
 
+// The pieces and their events, made on the stream's device, whichever is current (a stream takes
+// its own device's events only).
+static hipError_t make_pieces(HostStage& st, size_t bytes, hipStream_t s)
+{
+    int current = 0;
+    hipDevice_t own = 0;
+    hipError_t e = hipGetDevice(&current);
+    if (e == hipSuccess) e = hipStreamGetDevice(s, &own);
+    if (e == hipSuccess && own != current) e = hipSetDevice(own);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
+        if (!st.piece[k]) e = hipHostMalloc(&st.piece[k], bytes, hipHostMallocDefault);
+        if (e == hipSuccess && !st.filled[k]) e = hipEventCreateWithFlags(&st.filled[k], hipEventDisableTiming);
+    }
+    const hipError_t back = own != current ? hipSetDevice(current) : hipSuccess;
+    return e == hipSuccess ? back : e;
+}
+
 // Fields above one piece of doubles go through two pinned pieces: the copy engine fills one while the
 // host empties the other into the caller's memory, whose first touch and the widening of FP32
 // values are what takes the time.  A copy to pageable memory stages one piece after the other,
@@ -142,11 +160,7 @@ hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, do
         return hipSuccess;
     }
     const std::lock_guard<std::mutex> lock(st.turn);
-    for (int k = 0; k < 2; ++k) {
-        if (!st.piece[k]) e = hipHostMalloc(&st.piece[k], kPiece, hipHostMallocDefault);
-        if (e == hipSuccess && !st.filled[k]) e = hipEventCreateWithFlags(&st.filled[k], hipEventDisableTiming);
-        if (e != hipSuccess) return e;
-    }
+    if (!st.filled[1] && (e = make_pieces(st, kPiece, s)) != hipSuccess) return e;
     const int64_t per = (int64_t)(kPiece / esize), pieces = (n + per - 1) / per;
     auto fill = [&](int64_t i) {
         const int64_t count = std::min(per, n - i * per);

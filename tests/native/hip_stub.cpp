@@ -28,7 +28,6 @@ std::map<const void*, void*> g_symbols;
 std::vector<Launch> g_launches;
 std::string g_fast;           // kernels whose name holds this take 1 ms, the others 2
 double g_clock = 0.0;
-int g_attribute_fails = -1;   // this many calls of hipFuncSetAttribute succeed, the next fails
 std::vector<unsigned long> g_order;  // (thread, launch or copy) in order of the calls
 thread_local int t_device = 0;
 thread_local unsigned long t_id = 0;
@@ -56,7 +55,6 @@ const char* stub_launch(int i, unsigned* blocks, unsigned* threads, size_t* lds)
 }
 void stub_clear() { g_launches.clear(); g_order.clear(); }
 void stub_fast(const char* part) { g_fast = part; }
-void stub_attribute_fails(int after) { g_attribute_fails = after; }
 int stub_order(unsigned long* out, int n)
 {
     for (int i = 0; i < n && i < (int)g_order.size(); ++i) out[i] = g_order[i];
@@ -93,10 +91,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t 
     g_launches.push_back({name, grid.x, block.x, lds});
     return hipSuccess;
 }
-hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int)
-{
-    return g_attribute_fails >= 0 && g_attribute_fails-- == 0 ? hipErrorInvalidValue : hipSuccess;
-}
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { *n = 2; return hipSuccess; }
 
 // ---- devices ---------------------------------------------------------------------------

@@ -73,3 +73,21 @@ print(json.dumps([mode(timed), mode(steps())]))
 """)
     assert ran == ["0", "1", "3"]
     assert timed == ran
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_getters_with_another_device_current(on_stub, precision):
+    """A field of more than one staging piece is read while another GPU is current, and that GPU
+    stays current."""
+    ok = on_stub(f"""
+n = (400, 512)
+phi = np.arange(n[0] * n[1], dtype=np.float64).reshape(n)
+sim = amb.Integrator(phi, stencil, model(0), precision={precision})
+ens = amb.Ensemble([phi[:7], phi], stencil, [model(0)] * 2, [1, 2], precision={precision})
+stub.hipSetDevice(1)
+ok = [bool((sim.field == phi).all()), bool((ens.field(1) == phi).all())]
+d = ctypes.c_int(-1)
+stub.hipGetDevice(ctypes.byref(d))
+print(json.dumps(ok + [d.value]))
+""")
+    assert ok == [True, True, 1]
