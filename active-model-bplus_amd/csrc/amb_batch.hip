@@ -823,6 +823,7 @@ int amb_batch_get_field(amb_batch* b, int64_t index, double* out)
     if (!b || !out) return fail(AMB_E_ARG, "batch and out must not be null");
     if (index < 0 || index >= (int64_t)b->desc.size()) return fail(AMB_E_ARG, "realisation index out of range");
     const size_t n = (size_t)(b->desc[index].ny * b->desc[index].nx);
+    const std::lock_guard<std::mutex> turn(b->stage.turn);
     const hipError_t e = copy_out(b->stage, static_cast<const char*>(b->buf[b->cur]) + (size_t)b->off[index] * b->esize,
                                   (int64_t)n, b->precision, out, b->stream);
     return e == hipSuccess ? AMB_OK : fail_hip(e, "hipMemcpy (field download)");

@@ -159,7 +159,6 @@ hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, do
         for (size_t i = 0; i < tmp.size(); ++i) out[i] = (double)tmp[i];
         return hipSuccess;
     }
-    const std::lock_guard<std::mutex> lock(st.turn);
     if (!st.filled[1] && (e = make_pieces(st, kPiece, s)) != hipSuccess) return e;
     const int64_t per = (int64_t)(kPiece / esize), pieces = (n + per - 1) / per;
     auto fill = [&](int64_t i) {
@@ -784,6 +783,7 @@ int amb_get_field(amb_handle* h, double* out)
 {
     clear_error();
     if (!h || !out) return fail(AMB_E_ARG, "handle and out must not be null");
+    const std::lock_guard<std::mutex> turn(h->stage.turn);
     const hipError_t e = copy_out(h->stage, h->buf[h->cur], h->ny * h->nx, h->precision, out, h->stream);
     return e == hipSuccess ? AMB_OK : fail_hip(e, "hipMemcpy (field download)");
 }
@@ -798,6 +798,7 @@ int amb_get_observable_parts(amb_handle* h, int which, double* out, double* seco
     clear_error();
     if (!h || !out) return fail(AMB_E_ARG, "handle and out must not be null");
     if (which < AMB_OBS_MU || which > AMB_OBS_J_RANDOM) return fail(AMB_E_ARG, "unknown observable");
+    const std::lock_guard<std::mutex> turn(h->stage.turn);  // d_obs too is one for all getters
     const int rc = compute_observable(h, which);
     if (rc != AMB_OK) return rc;
     const int64_t n = h->ny * h->nx;

@@ -30,13 +30,14 @@ StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);
 extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
 
 // Two pinned pieces through which results go to the caller's memory, made on first use.  Getters
-// of one handle may be called from several threads; they take turns.
+// of one handle may be called from several threads: each holds `turn` until its result is out.
 struct HostStage {
     std::mutex turn;
     void* piece[2] = {nullptr, nullptr};
     hipEvent_t filled[2] = {nullptr, nullptr};
 };
-// n values of a field (FP32 or FP64) at dev, as doubles to out, after the work on `s`.
+// n values of a field (FP32 or FP64) at dev, as doubles to out, after the work on `s`.  The caller
+// holds st.turn.
 hipError_t copy_out(HostStage& st, const void* dev, int64_t n, int precision, double* out, hipStream_t s);
 void release(HostStage& st);
 

@@ -4,9 +4,10 @@
  * Plain C types only: doubles, 64-bit sizes and opaque handles.  Every call
  * returns AMB_OK (0) or an error code; amb_last_error() gives a thread-local
  * message for the last failure on the calling thread.  No C++ exception crosses
- * this boundary.  A handle must not be used from two threads at once; separate
- * handles are independent (all parameters travel as kernel arguments, there is
- * no process-global device state).
+ * this boundary.  A handle must not be used from two threads at once, but for
+ * amb_get_field, amb_get_observable and amb_batch_get_field, which take turns;
+ * separate handles are independent (all parameters travel as kernel arguments,
+ * there is no process-global device state).
  *
  * Field layout everywhere: row-major (ny, nx) float64, linear index col + row*nx,
  * periodic in both axes.  Vector quantities are 2*ny*nx doubles laid out

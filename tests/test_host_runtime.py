@@ -91,3 +91,36 @@ stub.hipGetDevice(ctypes.byref(d))
 print(json.dumps(ok + [d.value]))
 """)
     assert ok == [True, True, 1]
+
+
+def test_getters_of_one_field_take_turns(on_stub):
+    """Observables of one field share their device buffer: from the launch of an observable to the
+    copy of its last value no other thread's getter launches or copies anything."""
+    order = on_stub("""
+import threading
+n = (1024, 512)  # four pieces a component
+lib = ctypes.CDLL(sys.argv[2] + "/lib/libamb.so")
+h = ctypes.c_void_p()
+class Options(ctypes.Structure):
+    _fields_ = [("precision", ctypes.c_int), ("seed", ctypes.c_uint64), ("timestep", ctypes.c_int64), ("tile", ctypes.c_int)]
+three, seven = (ctypes.c_double * 3)(5e-3, 1, 1), (ctypes.c_double * 7)(-0.25, 0, 0.25, 1, 0.5, -1, 0.05)
+phi = np.zeros(n)
+opt = Options(32, 1, 0, 0)
+ptr = lambda a: ctypes.c_void_p(a.ctypes.data)
+assert lib.amb_create(ptr(phi), ctypes.c_int64(n[0]), ctypes.c_int64(n[1]), three, seven, ctypes.byref(opt), ctypes.byref(h)) == 0
+stub.stub_clear()
+rc = []
+def get(which):
+    out = np.zeros((2,) + n)
+    rc.append(lib.amb_get_observable(h, which, ptr(out)))
+threads = [threading.Thread(target=get, args=(w,)) for w in (3, 0, 5, 2)]  # ctypes lets them overlap
+for t in threads: t.start()
+for t in threads: t.join()
+assert rc == [0] * 4
+buf = (ctypes.c_ulong * 1000)()
+k = stub.stub_order(buf, 1000)
+print(json.dumps(list(buf[:k])))
+""")
+    threads = [x // 2 for x in order]
+    assert len(set(threads)) == 4
+    assert sum(a != b for a, b in zip(threads, threads[1:])) == 3, threads
