@@ -173,7 +173,8 @@ class HybridIntegrator:
         self.main = main if main is not None else Integrator(field, stencil, model, seed=seed, precision=32)
         self.judge = judge if judge is not None else Integrator(field, stencil, model, seed=seed, precision=32)
         if autotune:
-            self.judge.set_tile(self.main.autotune(4))  # autotune keeps the fastest for main
+            self.main.autotune(4)
+            self.judge.autotune(4, cached=True)  # what main's timing found
         self.delta, self.tol = delta_steps, tol
         self.audit_min = max(1, int(audit_every))
         self.audit_max = max(self.audit_min, int(max_audit_every or audit_every))

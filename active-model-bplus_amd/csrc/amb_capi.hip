@@ -227,9 +227,8 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
     static_assert(sizeof(kF64) / sizeof(kF64[0]) == kWide512F64 && kWide512F64 + 1 == 0 AMB_F64_TILES(AMB_COUNT_ONE),
                   "the FP64 order must list every FP64 tile shape but the last");
 #undef AMB_COUNT_ONE
-    // the index that stands for strips on large fields (step_grid), where they pay
-    const int strips = precision == AMB_F32 ? kSquare512F32 : kSquare512F64;
-    if (step_grid(precision, strips, noise, ny, nx).seg_rows > 0) return strips;
+    // fields that run in strips: the tile that comes next to them
+    if (run_tile(precision, noise, ny, nx) == kStrips) return precision == AMB_F32 ? kSquare512F32 : kSquare512F64;
     const int n = precision == AMB_F32 ? kWide512F32 : kWide512F64;
     const int* order = precision != AMB_F32 ? kF64 : noise == kNoiseNone ? kNoiselessF32 : kNoisyF32;
     int best = 0;
@@ -253,32 +252,28 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
 
 // ---- tuning table: the autotuners' choices, per (precision, grid, noise) ------------
 namespace {
+struct Tuned {
+    int tile;
+    bool strips;  // strips were faster than this, the fastest tile
+};
 std::mutex g_tune_mutex;
-std::map<std::tuple<int, int64_t, int64_t, int>, int> g_tune;
+std::map<std::tuple<int, int64_t, int64_t, int>, Tuned> g_tune;
 }  // namespace
 
-bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile)
+bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile, bool* strips)
 {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     const auto it = g_tune.find({precision, ny, nx, noise != kNoiseNone});
     if (it == g_tune.end()) return false;
-    *tile = it->second;
+    *tile = it->second.tile;
+    if (strips) *strips = it->second.strips;
     return true;
 }
 
-void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile)
+void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, bool strips)
 {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    g_tune[{precision, ny, nx, noise != kNoiseNone}] = tile;
-}
-
-// The tile a new integrator starts with: the tuning table's entry when there is one,
-// otherwise the occupancy rule.
-int initial_tile(int precision, int64_t ny, int64_t nx, int noise, bool* tuned)
-{
-    int t = 0;
-    *tuned = tuned_tile(precision, ny, nx, noise, &t);
-    return *tuned ? t : default_tile(precision, ny, nx, noise);
+    g_tune[{precision, ny, nx, noise != kNoiseNone}] = {tile, strips};
 }
 
 }  // namespace amb
@@ -325,14 +320,17 @@ namespace {
 
 constexpr int kGraphSteps = 32;  // even: a graph returns the field to the buffer it started in
 
-// The tile of the handle's launches.
-int launch_tile(const amb_handle* h) { return h->tile_chosen ? h->tile : run_tile(h->precision, h->ny, h->nx); }
+// The tile (or kStrips) of the handle's launches.
+int launch_tile(const amb_handle* h, int noise)
+{
+    return h->tile_chosen ? h->tile : run_tile(h->precision, noise, h->ny, h->nx);
+}
 
 template <typename T>
-StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int noise_mode, bool reduce = false)
+StepArgs<T> step_args(const amb_handle* h, int tile, int parity_in, int step_off, int noise_mode, bool reduce = false)
 {
     StepArgs<T> a{};
-    const StepGrid g = step_grid(h->precision, launch_tile(h), noise_mode, h->ny, h->nx);
+    const StepGrid g = step_grid(h->precision, tile, noise_mode, h->ny, h->nx);
     a.in = static_cast<const T*>(h->buf[parity_in & 1]);
     a.out = static_cast<T*>(h->buf[(parity_in + 1) & 1]);
     a.ny = (int)h->ny;
@@ -358,17 +356,34 @@ StepArgs<T> step_args(const amb_handle* h, int parity_in, int step_off, int nois
 // of the fused finite check and FP64 mass.
 hipError_t launch_step(const amb_handle* h, int parity_in, int step_off, int noise_mode, bool reduce = false)
 {
+    const int tile = launch_tile(h, noise_mode);
     if (h->precision == AMB_F32)
-        return launch_step_f32(step_args<float>(h, parity_in, step_off, noise_mode, reduce), launch_tile(h), noise_mode,
+        return launch_step_f32(step_args<float>(h, tile, parity_in, step_off, noise_mode, reduce), tile, noise_mode,
                                h->stream);
-    return launch_step_f64(step_args<double>(h, parity_in, step_off, noise_mode, reduce), launch_tile(h), noise_mode,
+    return launch_step_f64(step_args<double>(h, tile, parity_in, step_off, noise_mode, reduce), tile, noise_mode,
                            h->stream);
+}
+
+void choose_tile(amb_handle* h, int tile, bool strips = false)
+{
+    h->tile = tile;
+    h->tile_chosen = !strips;
+}
+
+// The tuning table's entry, when it has one for the handle's field.
+bool take_tuned(amb_handle* h, int noise)
+{
+    int tile = 0;
+    bool strips = false;
+    if (!tuned_tile(h->precision, h->ny, h->nx, noise, &tile, &strips)) return false;
+    choose_tile(h, tile, strips);
+    return true;
 }
 
 // Workgroups of one step, each writing one partial of the fused finite check.
 int64_t parts_of(const amb_handle* h, int noise)
 {
-    const StepGrid g = step_grid(h->precision, launch_tile(h), noise, h->ny, h->nx);
+    const StepGrid g = step_grid(h->precision, launch_tile(h, noise), noise, h->ny, h->nx);
     return (int64_t)g.ntx * g.nty;
 }
 
@@ -408,7 +423,7 @@ int build_graph(amb_handle* h, int parity, int noise_mode)
     if (e != hipSuccess) return fail_hip(e, "hipGraphInstantiate");
     if (h->graph[parity]) (void)hipGraphExecDestroy(h->graph[parity]);
     h->graph[parity] = exec;
-    h->graph_tile[parity] = launch_tile(h);
+    h->graph_tile[parity] = launch_tile(h, noise_mode);
     h->graph_noise[parity] = noise_mode;
     return AMB_OK;
 }
@@ -431,7 +446,7 @@ int enqueue_steps(amb_handle* h, int64_t nsteps)
         }
         if (left >= kGraphSteps) {
             const int p = h->cur;
-            if (!h->graph[p] || h->graph_tile[p] != launch_tile(h) || h->graph_noise[p] != mode) {
+            if (!h->graph[p] || h->graph_tile[p] != launch_tile(h, mode) || h->graph_noise[p] != mode) {
                 const int rc = build_graph(h, p, mode);
                 if (rc != AMB_OK) return rc;
             }
@@ -544,13 +559,13 @@ int compute_observable(amb_handle* h, int which)
     if (!h->d_obs) {
         if ((e = hipMalloc(&h->d_obs, 4 * n * sizeof(double))) != hipSuccess) return fail_hip(e, "hipMalloc");
     }
-    const int mode = noise_mode_of(h);
+    const int mode = noise_mode_of(h), tile = launch_tile(h, mode);
     if (h->precision == AMB_F32) {
-        StepArgs<float> a = step_args<float>(h, h->cur, 0, mode);
+        StepArgs<float> a = step_args<float>(h, tile, h->cur, 0, mode);
         if (mode != kNoiseBuffer) a.noise = nullptr;
         e = launch_observable_f32(a, which, h->d_obs, h->d_obs + 2 * n, h->stream);
     } else {
-        StepArgs<double> a = step_args<double>(h, h->cur, 0, mode);
+        StepArgs<double> a = step_args<double>(h, tile, h->cur, 0, mode);
         if (mode != kNoiseBuffer) a.noise = nullptr;
         e = launch_observable_f64(a, which, h->d_obs, h->d_obs + 2 * n, h->stream);
     }
@@ -696,10 +711,11 @@ int amb_create(const double* field, int64_t ny, int64_t nx, const amb_stencil* s
     } while (0)
     AMB_CHECK(hipGetDevice(&h->device));
     AMB_CHECK(prepare_step_kernels());
-    h->tile_chosen = opt.tile > 0;
-    h->tile = opt.tile > 0 ? opt.tile - 1
-                           : initial_tile(opt.precision, ny, nx, model->T > 0.0 ? kNoisePhilox : kNoiseNone,
-                                          &h->tile_chosen);
+    {
+        const int noise = model->T > 0.0 ? kNoisePhilox : kNoiseNone;
+        if (opt.tile > 0) choose_tile(h, opt.tile - 1);
+        else if (!take_tuned(h, noise)) h->tile = default_tile(opt.precision, ny, nx, noise);
+    }
     AMB_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     AMB_CHECK(hipMalloc(&h->buf[0], n * h->esize));
     AMB_CHECK(hipMalloc(&h->buf[1], n * h->esize));
@@ -887,11 +903,8 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
     if (!h) return fail(AMB_E_ARG, "handle must not be null");
     const int mode0 = h->model.T > 0.0 ? kNoisePhilox : kNoiseNone;
     if (reps < 0) {  // the tuning table's choice, when it has one
-        int t = 0;
-        if (tuned_tile(h->precision, h->ny, h->nx, mode0, &t)) {
-            h->tile = t;
-            h->tile_chosen = true;
-            if (chosen) *chosen = t;
+        if (take_tuned(h, mode0)) {
+            if (chosen) *chosen = h->tile;
             return AMB_OK;
         }
         reps = -reps;
@@ -911,7 +924,11 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
     float best = 1e30f;
     int best_t = h->tile;
     const int mode = h->model.T > 0.0 ? kNoisePhilox : kNoiseNone;
-    for (int t = 0; t < tile_count(h->precision) && e == hipSuccess; ++t) {
+    // every tile shape, then strips where the field runs in them without a choice
+    bool strips = false;
+    const int shapes = tile_count(h->precision);
+    const int trials = shapes + (run_tile(h->precision, mode, h->ny, h->nx) == kStrips ? 1 : 0);
+    for (int t = 0; t < trials && e == hipSuccess; ++t) {
         trial.ny = h->ny;
         trial.nx = h->nx;
         trial.stencil = h->stencil;
@@ -922,7 +939,7 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
         trial.buf[1] = scratch[1];
         trial.d_step = step;
         trial.stream = h->stream;
-        trial.tile = t;
+        trial.tile = t < shapes ? t : kStrips;
         trial.tile_chosen = true;
         for (int k = 0; k <= reps && e == hipSuccess; ++k) {
             if (k == 1) e = hipEventRecord(h->ev0, h->stream);
@@ -934,7 +951,8 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
         if (e == hipSuccess) e = hipEventElapsedTime(&ms, h->ev0, h->ev1);
         if (e == hipSuccess && ms < best) {
             best = ms;
-            best_t = t;
+            if (t < shapes) best_t = t;
+            else strips = true;
         }
     }
     (void)hipStreamSynchronize(h->stream);
@@ -942,9 +960,8 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
         if (p) (void)hipFree(p);
     trial.stream = nullptr;
     if (e != hipSuccess) return fail_hip(e, "autotune");
-    h->tile = best_t;
-    h->tile_chosen = true;
-    record_tile(h->precision, h->ny, h->nx, mode0, best_t);
+    choose_tile(h, best_t, strips);
+    record_tile(h->precision, h->ny, h->nx, mode0, best_t, strips);
     if (chosen) *chosen = best_t;
     return AMB_OK;
 }
@@ -955,7 +972,7 @@ int amb_tuning_set(int precision, int64_t ny, int64_t nx, int noisy, int tile)
     if (precision != AMB_F32 && precision != AMB_F64) return fail(AMB_E_ARG, "bad precision");
     if (ny <= 0 || nx <= 0) return fail(AMB_E_ARG, "bad grid");
     if (tile < 0 || tile >= tile_count(precision)) return fail(AMB_E_ARG, "tile index out of range");
-    record_tile(precision, ny, nx, noisy ? kNoisePhilox : kNoiseNone, tile);
+    record_tile(precision, ny, nx, noisy ? kNoisePhilox : kNoiseNone, tile, false);
     return AMB_OK;
 }
 
@@ -985,7 +1002,7 @@ int amb_tuning_entry(int64_t index, int* precision, int64_t* ny, int64_t* nx, in
     if (ny) *ny = std::get<1>(it->first);
     if (nx) *nx = std::get<2>(it->first);
     if (noisy) *noisy = std::get<3>(it->first);
-    if (tile) *tile = it->second;
+    if (tile) *tile = it->second.tile;
     return AMB_OK;
 }
 
@@ -1001,8 +1018,7 @@ int amb_set_tile(amb_handle* h, int index)
     clear_error();
     if (!h) return fail(AMB_E_ARG, "handle must not be null");
     if (index < 0 || index >= tile_count(h->precision)) return fail(AMB_E_ARG, "tile index out of range");
-    h->tile = index;
-    h->tile_chosen = true;
+    choose_tile(h, index);
     return AMB_OK;
 }
 

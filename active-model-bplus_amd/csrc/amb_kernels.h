@@ -74,7 +74,7 @@ constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threa
 #define AMB_F64_ORDER 3, 0, 2, 1, 4, 5, 6
 
 // The tile that a field runs in when none was chosen: 32x16 tiles of 512 threads while one
-// round of them holds the field, else 32x32 tiles of 512 threads, or strips (step_grid).  us a
+// round of them holds the field, else 32x32 tiles of 512 threads, or kStrips (step_grid).  us a
 // step, 32x16 / 32x32 / the tile of the orders above:
 //   side      FP32 T = 0.05        FP32 T = 0           FP64 T = 0.05        FP64 T = 0
 //   64        4.41 / 5.26 / 4.89   3.64 / 4.59 / 4.05   5.64 / 7.16 / 6.16   4.48 / 5.41 / 4.27
@@ -88,15 +88,16 @@ constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threa
 // (a round is four workgroups per compute unit in FP32, three in FP64).  FP64 32x32 tiles that
 // fit one to a compute unit beat more than 1.5 32x16 tiles to each (448^2 8.30 / 8.46).
 constexpr int kWide512F32 = 10, kWide512F64 = 7;
-int run_tile(int precision, int64_t ny, int64_t nx);
+int run_tile(int precision, int noise, int64_t ny, int64_t nx);
+constexpr int kStrips = -1;  // in a tile's place: strips of columns (step_grid)
 
 // Tile shapes compiled per precision (index = autotuner choice).
 int tile_count(int precision);
 TileShape tile_shape(int precision, int index);
 
-// Workgroups of one step of a whole field: ntx x nty tiles or, on large fields in place of
-// 32x32 tiles of 512 threads, strips of columns each seg_rows rows long (amb_march.h; the
-// rule and its reason are at step_grid).
+// Workgroups of one step of a whole field: ntx x nty tiles of a shape or, on large fields for
+// which none was chosen, strips of columns each seg_rows rows long (amb_march.h; the rule and its
+// reason are at strip_grid).
 struct StepGrid {
     int ntx, nty;
     int seg_rows;  // 0: tiles

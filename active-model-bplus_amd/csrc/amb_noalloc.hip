@@ -91,8 +91,9 @@ int run_noalloc(T* field, T* work, int64_t ny, int64_t nx, const amb_stencil& st
     unsigned long long* bad = reinterpret_cast<unsigned long long*>(base + 24);
     double* part = reinterpret_cast<double*>(base + kPartOffset);
     const int precision = sizeof(T) == 4 ? AMB_F32 : AMB_F64;
-    StepGrid g = step_grid(precision, run_tile(precision, ny, nx), noise, ny, nx);
-    if ((int64_t)g.ntx * g.nty <= kNoAllocMaxTiles) tile = run_tile(precision, ny, nx);
+    const int run = run_tile(precision, noise, ny, nx);
+    StepGrid g = step_grid(precision, run, noise, ny, nx);
+    if ((int64_t)g.ntx * g.nty <= kNoAllocMaxTiles) tile = run;
     else g = step_grid(precision, tile, noise, ny, nx);
     StepArgs<T> a{};
     a.ny = (int)ny;

@@ -162,28 +162,33 @@ static int64_t march_cost(int64_t ny, int strips, int slots, int* seg_rows)
 // Every field's 32-bit byte offsets must reach it, and an explicit noise buffer takes tiles.
 constexpr double kStripShareF32[2] = {0.495, 0.51}, kStripShareF64[2] = {0.69, 0.5};  // quiet, noisy
 
-StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx)
+static bool strip_grid(int precision, int noise, int64_t ny, int64_t nx, StepGrid* g)
 {
-    const TileShape ts = tile_shape(precision, tile);
-    StepGrid g{(int)((nx + ts.tw - 1) / ts.tw), (int)((ny + ts.th - 1) / ts.th), 0};
     const int64_t sites = ny * nx;
-    if (tile != (precision == 32 ? kSquare512F32 : kSquare512F64) || noise == kNoiseBuffer || ny < 4 || nx < 4 ||
-        sites > ((int64_t)1 << 31) / (precision / 8))
-        return g;
+    if (noise == kNoiseBuffer || ny < 4 || nx < 4 || sites > ((int64_t)1 << 31) / (precision / 8)) return false;
     const int strips = (int)((nx + kMarchCols - 1) / kMarchCols);
     const int slots = device_cus() * march_per_cu(precision, noise, ny, nx);
     int seg_rows = 0;
     const int64_t cost = march_cost(ny, strips, slots, &seg_rows);
     const double share = (double)sites / ((double)slots * (double)cost * kMarchCols);
     const double least = (precision == 32 ? kStripShareF32 : kStripShareF64)[noise != kNoiseNone];
-    if (cost == 0 || share < least) return g;
-    g.ntx = strips;
-    g.seg_rows = seg_rows;
-    g.nty = (int)((ny + seg_rows - 1) / seg_rows);
-    return g;
+    if (cost == 0 || share < least) return false;
+    *g = {strips, (int)((ny + seg_rows - 1) / seg_rows), seg_rows};
+    return true;
 }
 
-int run_tile(int precision, int64_t ny, int64_t nx)
+StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx)
+{
+    StepGrid g{};
+    if (tile == kStrips) {
+        (void)strip_grid(precision, noise, ny, nx, &g);  // run_tile has found that there are some
+        return g;
+    }
+    const TileShape ts = tile_shape(precision, tile);
+    return {(int)((nx + ts.tw - 1) / ts.tw), (int)((ny + ts.th - 1) / ts.th), 0};
+}
+
+int run_tile(int precision, int noise, int64_t ny, int64_t nx)
 {
     const int wide = precision == 32 ? kWide512F32 : kWide512F64, square = precision == 32 ? kSquare512F32 : kSquare512F64;
     auto tiles = [&](int tile) {
@@ -191,9 +196,9 @@ int run_tile(int precision, int64_t ny, int64_t nx)
         return ((nx + t.tw - 1) / t.tw) * ((ny + t.th - 1) / t.th);
     };
     const int64_t cus = device_cus(), n = tiles(wide);
-    if (n > (precision == 32 ? 4 : 3) * cus) return square;
-    if (precision == 64 && tiles(square) <= cus && 2 * n > 3 * cus) return square;
-    return wide;
+    if (n <= (precision == 32 ? 4 : 3) * cus && !(precision == 64 && tiles(square) <= cus && 2 * n > 3 * cus)) return wide;
+    StepGrid strips;
+    return strip_grid(precision, noise, ny, nx, &strips) ? kStrips : square;
 }
 
 template <typename T, int TW, int TH, int NT, int NOISE>

@@ -53,8 +53,8 @@ typedef struct {
     int precision;     /* AMB_F64 or AMB_F32: storage and arithmetic of the field */
     uint64_t seed;     /* Philox key of the conserved noise */
     int64_t timestep;  /* initial step counter (exact resume: field, timestep, seed) */
-    int tile;          /* k > 0 selects tile index k-1 (see amb_tile_count); 0 = the library chooses among its
-                          tiles and strips by size, and amb_get_options names the occupancy rule's index */
+    int tile;          /* k > 0 selects the shape of tile index k-1 (see amb_tile_count); 0 = the library chooses among
+                          its tiles and strips by size, and amb_get_options names the occupancy rule's index */
 } amb_options;
 
 typedef struct amb_handle amb_handle;
@@ -134,10 +134,12 @@ int amb_tile_count(int precision, int* count);
 int amb_tile_shape(int precision, int index, int* tile_cols, int* tile_rows, int* threads);
 int amb_set_tile(amb_handle* h, int index);
 
-/* Autotuner for one field: times `reps` steps of every compiled tile shape on a
- * copy of the current state (field and step counter untouched), selects the
- * fastest for this handle, records it in the tuning table and returns its index in
- * `chosen` (nullable).  reps < 0: take the tuning table's entry for this precision,
+/* Autotuner for one field: times `reps` steps of every compiled tile shape, and of
+ * strips where the field runs in them without a choice, on a copy of the current
+ * state (field and step counter untouched), selects the fastest for this handle and
+ * records it in the tuning table; `chosen` (nullable) receives the index of the
+ * fastest shape, also where strips were faster than it (amb_set_tile with that index
+ * then runs the shape).  reps < 0: take the tuning table's entry for this precision,
  * grid and noise mode when there is one (no timing), else time |reps| steps. */
 int amb_autotune(amb_handle* h, int reps, int* chosen);
 

@@ -124,3 +124,58 @@ print(json.dumps(list(buf[:k])))
     threads = [x // 2 for x in order]
     assert len(set(threads)) == 4
     assert sum(a != b for a, b in zip(threads, threads[1:])) == 3, threads
+
+
+LARGE = """
+shape, precision, T = {shape}, {precision}, {T}
+phi = np.zeros(shape)
+make = lambda tile=0: amb.Integrator(phi, stencil, model(T), seed=1, precision=precision, tile=tile)
+shapes = [tuple(s) for s in amb.tile_shapes(precision)]
+square = shapes.index((32, 32, 512))
+def ran(sim):  # "strips" or the shape of the step's tiles
+    stub.stub_clear()
+    sim.run(1)
+    (name,) = steps()
+    return "strips" if "march" in name else tuple(int(x.split("E")[0]) for x in name.split("Li")[1:4])
+"""
+FIELDS = pytest.mark.parametrize("shape,precision,T", [((2050, 2050), 32, 0.05), ((2304, 2304), 32, 0.0),
+                                                       ((1800, 1801), 64, 0.05), ((2304, 2304), 64, 0.0)])
+
+
+@FIELDS
+def test_a_chosen_shape_is_the_shape_that_runs(on_stub, shape, precision, T):
+    """Fields large enough for strips run in them when no tile was chosen; every shape can be chosen,
+    by the option and by set_tile."""
+    out = on_stub(LARGE.format(shape=shape, precision=precision, T=T) + """
+by_option = [ran(make(t + 1)) for t in range(len(shapes))]
+sim = make()
+first = ran(sim)
+by_set = []
+for t in range(len(shapes)):
+    sim.set_tile(t)
+    by_set.append(ran(sim))
+print(json.dumps([first, by_option == shapes, by_set == shapes]))
+""")
+    assert out == ["strips", True, True]
+
+
+@FIELDS
+def test_autotune_times_strips_beside_the_shapes(on_stub, shape, precision, T):
+    """Whichever is fastest runs afterwards, also in new fields of that size and where the table is
+    asked first; the index returned is a shape's either way."""
+    out = on_stub(LARGE.format(shape=shape, precision=precision, T=T) + """
+out = []
+for fast, want in (("march_kernel", "strips"), ("Li32ELi32ELi512E", shapes[square]), ("Li64ELi16ELi256E", (64, 16, 256))):
+    tuning.clear()
+    stub.stub_fast(fast.encode())
+    sim = make()
+    best = sim.autotune(1)
+    timed = len(set(steps()))
+    assert timed == len(shapes) + 1 and 0 <= best < len(shapes)
+    assert amb.tuning_get(precision, shape[0], shape[1], T > 0) == best
+    again = make(3)
+    assert again.autotune(1, cached=True) == best and not steps()
+    out.append([ran(sim) == want, ran(make()) == want, ran(again) == want])
+print(json.dumps(out))
+""")
+    assert out == [[True] * 3] * 3
