@@ -3,10 +3,13 @@
 ``Integrator.autotune`` and ``Ensemble.autotune`` time every compiled tile shape and
 record the fastest in a process-wide table keyed by (precision, ny, nx, noisy); new
 integrators and ensembles of a tabled size start from its entry instead of the
-occupancy rule, and ``autotune(cached=True)`` returns it without timing.  This module
+library's own choice, and ``autotune(cached=True)`` returns it without timing.  This module
 keeps that table across processes as JSON.  Entries are stored by tile shape
 (columns, rows, threads), not by index, so a file written by one build loads into
-another; shapes this build does not compile are skipped.
+another; shapes this build does not compile are skipped.  Large single fields run in
+strips of columns unless a tile is chosen; an entry says whether its tile was timed
+against other tiles alone (an ensemble's, and files without the word), against strips
+too, or was slower than they, and only the second kind takes such a field's strips away.
 
     from activemodelbplus import tuning
     tuning.load("tiles.json")        # before creating integrators
@@ -20,17 +23,20 @@ import os
 
 from .integrator import tile_shapes
 from .integrator import tuning_clear as clear  # noqa: F401  (re-exported)
-from .integrator import tuning_entries, tuning_set
+from .integrator import tuning_entries, tuning_set, tuning_timed
 
 FORMAT = 1
+TIMED = ("tiles", "all", "strips")
 
 
 def entries():
-    """The table as a list of dicts: precision, ny, nx, noisy, tile (cols, rows, threads)."""
+    """The table as a list of dicts: precision, ny, nx, noisy, tile (cols, rows, threads),
+    timed (what the tile was compared with)."""
     out = []
     for precision, ny, nx, noisy, tile in tuning_entries():
         out.append({"precision": int(precision), "ny": int(ny), "nx": int(nx), "noisy": bool(noisy),
-                    "tile": list(tile_shapes(precision)[tile])})
+                    "tile": list(tile_shapes(precision)[tile]),
+                    "timed": TIMED[tuning_timed(precision, ny, nx, noisy)]})
     return out
 
 
@@ -59,6 +65,9 @@ def load(path):
         p = int(e["precision"])
         if p not in shapes or list(e["tile"]) not in shapes[p]:
             continue  # a shape this build does not compile
-        tuning_set(p, int(e["ny"]), int(e["nx"]), bool(e["noisy"]), shapes[p].index(list(e["tile"])))
+        key = p, int(e["ny"]), int(e["nx"]), bool(e["noisy"])
+        tuning_set(*key, shapes[p].index(list(e["tile"])))
+        timed = e.get("timed", "tiles")
+        tuning_timed(*key, set=TIMED.index(timed) if timed in TIMED else 0)
         n += 1
     return n

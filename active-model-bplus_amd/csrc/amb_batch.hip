@@ -964,7 +964,8 @@ int amb_batch_autotune(amb_batch* b, int reps, int* chosen)
         }
         for (int r : kv.second) best_tile[r] = best_t;
         if (e == hipSuccess)
-            record_tile(b->precision, std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first), best_t);
+            record_tile(b->precision, std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first), best_t,
+                        AMB_TUNED_TILES);
     }
     if (e == hipSuccess) e = hipMemcpy(b->buf[b->cur], saved, (size_t)b->total * b->esize, hipMemcpyDeviceToDevice);
     (void)hipFree(saved);

@@ -254,26 +254,30 @@ int default_tile(int precision, int64_t ny, int64_t nx, int noise)
 namespace {
 struct Tuned {
     int tile;
-    bool strips;  // strips were faster than this, the fastest tile
+    int timed;  // AMB_TUNED_*
 };
 std::mutex g_tune_mutex;
 std::map<std::tuple<int, int64_t, int64_t, int>, Tuned> g_tune;
 }  // namespace
 
-bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile, bool* strips)
+bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile, int* timed)
 {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     const auto it = g_tune.find({precision, ny, nx, noise != kNoiseNone});
     if (it == g_tune.end()) return false;
     *tile = it->second.tile;
-    if (strips) *strips = it->second.strips;
+    if (timed) *timed = it->second.timed;
     return true;
 }
 
-void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, bool strips)
+// An ensemble's timing knows nothing of strips: it does not replace an entry that decides between
+// them and a tile for single fields.
+void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, int timed)
 {
+    const bool strips = timed == AMB_TUNED_TILES && run_tile(precision, noise, ny, nx) == kStrips;
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    g_tune[{precision, ny, nx, noise != kNoiseNone}] = {tile, strips};
+    const auto at = g_tune.insert({{precision, ny, nx, noise != kNoiseNone}, {tile, timed}});
+    if (!at.second && !(strips && at.first->second.timed != AMB_TUNED_TILES)) at.first->second = {tile, timed};
 }
 
 }  // namespace amb
@@ -370,13 +374,14 @@ void choose_tile(amb_handle* h, int tile, bool strips = false)
     h->tile_chosen = !strips;
 }
 
-// The tuning table's entry, when it has one for the handle's field.
+// The tuning table's entry, when it has one for the handle's field (one timed among tiles alone
+// is none for a field that runs in strips).
 bool take_tuned(amb_handle* h, int noise)
 {
-    int tile = 0;
-    bool strips = false;
-    if (!tuned_tile(h->precision, h->ny, h->nx, noise, &tile, &strips)) return false;
-    choose_tile(h, tile, strips);
+    int tile = 0, timed = 0;
+    if (!tuned_tile(h->precision, h->ny, h->nx, noise, &tile, &timed)) return false;
+    if (timed == AMB_TUNED_TILES && run_tile(h->precision, noise, h->ny, h->nx) == kStrips) return false;
+    choose_tile(h, tile, timed == AMB_TUNED_STRIPS);
     return true;
 }
 
@@ -961,7 +966,7 @@ int amb_autotune(amb_handle* h, int reps, int* chosen)
     trial.stream = nullptr;
     if (e != hipSuccess) return fail_hip(e, "autotune");
     choose_tile(h, best_t, strips);
-    record_tile(h->precision, h->ny, h->nx, mode0, best_t, strips);
+    record_tile(h->precision, h->ny, h->nx, mode0, best_t, strips ? AMB_TUNED_STRIPS : AMB_TUNED_ALL);
     if (chosen) *chosen = best_t;
     return AMB_OK;
 }
@@ -972,7 +977,7 @@ int amb_tuning_set(int precision, int64_t ny, int64_t nx, int noisy, int tile)
     if (precision != AMB_F32 && precision != AMB_F64) return fail(AMB_E_ARG, "bad precision");
     if (ny <= 0 || nx <= 0) return fail(AMB_E_ARG, "bad grid");
     if (tile < 0 || tile >= tile_count(precision)) return fail(AMB_E_ARG, "tile index out of range");
-    record_tile(precision, ny, nx, noisy ? kNoisePhilox : kNoiseNone, tile, false);
+    record_tile(precision, ny, nx, noisy ? kNoisePhilox : kNoiseNone, tile, AMB_TUNED_ALL);
     return AMB_OK;
 }
 
@@ -981,6 +986,18 @@ int amb_tuning_get(int precision, int64_t ny, int64_t nx, int noisy, int* tile)
     clear_error();
     if (!tile) return fail(AMB_E_ARG, "tile must not be null");
     if (!tuned_tile(precision, ny, nx, noisy ? kNoisePhilox : kNoiseNone, tile)) *tile = -1;
+    return AMB_OK;
+}
+
+int amb_tuning_timed(int precision, int64_t ny, int64_t nx, int noisy, int set, int* timed)
+{
+    clear_error();
+    if (set > AMB_TUNED_STRIPS) return fail(AMB_E_ARG, "unknown kind of tuning entry");
+    std::lock_guard<std::mutex> lock(g_tune_mutex);
+    const auto it = g_tune.find({precision, ny, nx, noisy != 0});
+    if (it == g_tune.end()) return fail(AMB_E_ARG, "no tuning entry");
+    if (set >= 0) it->second.timed = set;
+    if (timed) *timed = it->second.timed;
     return AMB_OK;
 }
 

@@ -18,9 +18,9 @@ int check_device();
 int validate_params(int64_t ny, int64_t nx, const amb_stencil* st, const amb_model* m);
 int grid_tiles(int64_t n, int t);
 int default_tile(int precision, int64_t ny, int64_t nx, int noise);
-// The autotuners' table (process-wide): lookup, record, and the tile a new field starts with.
-bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile, bool* strips = nullptr);
-void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, bool strips = false);
+// The autotuners' table (process-wide): lookup and record (timed: AMB_TUNED_*).
+bool tuned_tile(int precision, int64_t ny, int64_t nx, int noise, int* tile, int* timed = nullptr);
+void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, int timed);
 
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);

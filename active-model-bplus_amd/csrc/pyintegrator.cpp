@@ -656,6 +656,12 @@ PYBIND11_MODULE(integrator, m)
         check(amb_tuning_get(precision, ny, nx, noisy ? 1 : 0, &t));
         return t;
     }, py::arg("precision"), py::arg("ny"), py::arg("nx"), py::arg("noisy"));
+    m.def("tuning_timed", [](int precision, int64_t ny, int64_t nx, bool noisy, int set) {
+        int timed = 0;
+        check(amb_tuning_timed(precision, ny, nx, noisy ? 1 : 0, set, &timed));
+        return timed;
+    }, py::arg("precision"), py::arg("ny"), py::arg("nx"), py::arg("noisy"), py::arg("set") = -1,
+    "what an entry's tile was compared with: 0 other tiles, 1 strips too, 2 strips that were faster");
     m.def("tuning_entries", []() {
         int64_t n = 0;
         check(amb_tuning_count(&n));

@@ -150,6 +150,15 @@ int amb_autotune(amb_handle* h, int reps, int* chosen);
  * amb_tuning_get gives tile = -1 when there is no entry. */
 int amb_tuning_set(int precision, int64_t ny, int64_t nx, int noisy, int tile);
 int amb_tuning_get(int precision, int64_t ny, int64_t nx, int noisy, int* tile);
+/* What an entry's tile was compared with: the other shapes alone (an ensemble's timing),
+ * strips too (a single field's timing; also what amb_tuning_set makes), or strips that
+ * were faster than it.  Members take an entry's tile whichever it is.  A single field that
+ * runs in strips without a choice takes the tile of the second kind only.  set >= 0 changes
+ * the entry's kind; timed (nullable) receives it.  AMB_E_ARG when there is no entry. */
+#define AMB_TUNED_TILES 0
+#define AMB_TUNED_ALL 1
+#define AMB_TUNED_STRIPS 2
+int amb_tuning_timed(int precision, int64_t ny, int64_t nx, int noisy, int set, int* timed);
 int amb_tuning_count(int64_t* count);
 int amb_tuning_entry(int64_t index, int* precision, int64_t* ny, int64_t* nx, int* noisy, int* tile);
 int amb_tuning_clear(void);

@@ -179,3 +179,46 @@ for fast, want in (("march_kernel", "strips"), ("Li32ELi32ELi512E", shapes[squar
 print(json.dumps(out))
 """)
     assert out == [[True] * 3] * 3
+
+
+@FIELDS
+def test_ensemble_timing_leaves_single_fields_their_strips(on_stub, shape, precision, T):
+    """An ensemble's timing, and a file of one that says nothing of strips, neither take them from
+    single fields of that size nor replace what a single field's timing found."""
+    out = on_stub(LARGE.format(shape=shape, precision=precision, T=T) + """
+import os, tempfile
+path = os.path.join(tempfile.mkdtemp(), "tiles.json")
+key = precision, shape[0], shape[1], T > 0
+stub.stub_fast(b"Li64ELi16ELi256E")
+ens = lambda: amb.Ensemble([phi], stencil, [model(T)], [1], precision=precision)
+tile = ens().autotune(1)[0]
+out = [shapes[tile] == (64, 16, 256), amb.tuning_get(*key) == tile, ens().tiles[0] == tile, ran(make()) == "strips"]
+tuning.save(path)
+tuning.clear()
+tuning.load(path)
+out += [ens().tiles[0] == tile, ran(make()) == "strips"]
+data = json.load(open(path))
+for e in data["entries"]:
+    del e["timed"]  # a file of before
+json.dump(data, open(path, "w"))
+tuning.clear()
+assert tuning.load(path) == 1
+out += [ens().tiles[0] == tile, ran(make()) == "strips"]
+steps()
+make().autotune(1, cached=True)  # no entry that would do: times
+out += [len(set(steps())) == len(shapes) + 1, ran(make()) == (64, 16, 256)]
+for fast, runs in (("march_kernel", "strips"), ("Li32ELi16ELi256E", (32, 16, 256))):
+    stub.stub_fast(fast.encode())
+    make().autotune(1)
+    kept = amb.tuning_get(*key)
+    stub.stub_fast(b"Li64ELi16ELi256E")
+    ens().autotune(1)
+    out += [amb.tuning_get(*key) == kept, ran(make()) == runs]
+    tuning.save(path)
+    tuning.clear()
+    tuning.load(path)
+    out += [amb.tuning_get(*key) == kept, ran(make()) == runs]
+amb.tuning_set(*key, 1)
+print(json.dumps(out + [ran(make()) == shapes[1]]))
+""")
+    assert out == [True] * len(out)
