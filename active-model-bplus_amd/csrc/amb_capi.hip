@@ -861,6 +861,21 @@ int amb_get_options(const amb_handle* h, amb_options* options)
     return AMB_OK;
 }
 
+int amb_get_step_shape(const amb_handle* h, int* cols, int* rows, int* threads, int* strips)
+{
+    clear_error();
+    if (!h) return fail(AMB_E_ARG, "handle must not be null");
+    const int noise = noise_mode_of(h), tile = launch_tile(h, noise);
+    TileShape ts;
+    if (tile == kStrips) ts = {kMarchCols, step_grid(h->precision, tile, noise, h->ny, h->nx).seg_rows, march_threads(noise)};
+    else ts = tile_shape(h->precision, tile);
+    if (cols) *cols = ts.tw;
+    if (rows) *rows = ts.th;
+    if (threads) *threads = ts.nt;
+    if (strips) *strips = tile == kStrips;
+    return AMB_OK;
+}
+
 int amb_mass(amb_handle* h, double* sum, int64_t* nonfinite)
 {
     clear_error();

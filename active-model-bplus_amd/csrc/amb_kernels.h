@@ -102,6 +102,8 @@ struct StepGrid {
     int ntx, nty;
     int seg_rows;  // 0: tiles
 };
+constexpr int kMarchCols = 112;  // columns of a strip
+constexpr int march_threads(int noise) { return noise != kNoiseNone ? 512 : 256; }
 StepGrid step_grid(int precision, int tile, int noise, int64_t ny, int64_t nx);
 int device_cus();  // compute units of the current device
 

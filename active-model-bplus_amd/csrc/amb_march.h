@@ -35,7 +35,7 @@
 
 namespace amb {
 
-constexpr int kMarchCols = 112, kMarchRows = 4;
+constexpr int kMarchRows = 4;  // of a step
 
 // LDS rings of a strip (elements).  Columns: mu_p from -8, mu_a, q and C from -2, J_x from -4,
 // J_y from 0.  A ring of 16 or 8 rows holds row rho at slot rho mod 16 or
@@ -56,7 +56,7 @@ struct MarchLds {
     static constexpr int total = off_jy + (NOISY ? 8 * YP : 0);
     static constexpr size_t red_off = (sizeof(T) * (size_t)total + 15) / 16 * 16;
     static constexpr size_t bytes = red_off + 16 * 128;  // a (sum, count) pair per lane of role B
-    static constexpr int NT = NOISY ? 512 : 256;
+    static constexpr int NT = march_threads(NOISY);
     static constexpr int wg = (int)((160 * 1024) / bytes);
     static constexpr int waves_want = wg * (NT / 64) / 4;
     // registers bind the noiseless step (its 17-row window) before LDS does

@@ -221,6 +221,13 @@ class Integrator {
 
     void set_tile(int index) { check(amb_set_tile(h_, index)); }
 
+    py::tuple step_shape() const
+    {
+        int cols = 0, rows = 0, threads = 0, strips = 0;
+        check(amb_get_step_shape(h_, &cols, &rows, &threads, &strips));
+        return py::make_tuple(cols, rows, threads, strips != 0);
+    }
+
     void set_field(const Field& field)
     {
         if (field.ndim() != 2 || field.shape(0) != ny_ || field.shape(1) != nx_)
@@ -597,6 +604,8 @@ PYBIND11_MODULE(integrator, m)
         .def("set_noise", &Integrator::set_noise, py::arg("noise"),
              "test only: explicit unscaled normals (steps, 2, ny, nx) for the next steps")
         .def("set_tile", &Integrator::set_tile, py::arg("index"))
+        .def_property_readonly("step_shape", &Integrator::step_shape,
+                               "(columns, rows, threads, strips?) that the next step's workgroups run in")
         .def("autotune", &Integrator::autotune, py::arg("reps") = 8, py::arg("cached") = false,
              "time every compiled tile shape on a copy of the state and keep the fastest "
              "(cached: take the tuning table's entry when there is one)")

@@ -122,7 +122,8 @@ def cpu_baseline(w, phi, budget_s=15.0, budget_1core_s=8.0):
 
 def read_profile_value(path, tile, tile_key, value_key):
     """The value of `value_key:` in a profile summary under profiles/, or None when the file
-    is missing or its `tile_key:` line names another tile shape than `tile`."""
+    is missing or its `tile_key:` line names another shape than `tile` (of a tile or a strip:
+    columns, rows, threads)."""
     if not os.path.exists(path):
         return None
     fields = {}
@@ -159,7 +160,9 @@ def bench_single(args, key):
     phi = initial_field(w)
     sim = Integrator(phi, Stencil(*w["stencil"]), Model(*w["model"]), seed=w["seed"], precision=w["precision"],
                      tile=args.tile)
-    tile = sim.autotune(4) if args.autotune else sim.options["tile"] - 1
+    if args.autotune:
+        sim.autotune(4)
+    shape = sim.step_shape[:3]  # of a tile, or a strip's columns and its segments' rows
     if args.warmup:
         sim.run(args.warmup)
     t0 = time.perf_counter()
@@ -179,14 +182,14 @@ def bench_single(args, key):
         "data": "synthetic (seeded numpy normal initial field)",
         "config": {"workload": w["label"], "grid": [w["n"], w["n"]], "stencil": w["stencil"],
                    "model": dict(zip(["a", "b", "c", "kappa", "lamb", "zeta", "T"], w["model"])),
-                   "tile": dict(zip(["cols", "rows", "threads"], sim_tile_shape(w["precision"], tile)))},
+                   "tile": dict(zip(["cols", "rows", "threads"], shape))},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": read_traffic(TRAFFIC_PROFILE.get(key, ""), sim_tile_shape(w["precision"], tile))},
+                     "traffic": read_traffic(TRAFFIC_PROFILE.get(key, ""), shape)},
         "device_ms_per_step": device_ms / args.steps,
         "mass_fp64": mass, "nonfinite": bad,
     }
-    valu = read_valu(VALU_PROFILE.get(key, ""), sim_tile_shape(w["precision"], tile))
+    valu = read_valu(VALU_PROFILE.get(key, ""), shape)
     if valu is not None:
         # the bound that holds: vector-ALU issue (the HBM fraction above is the honest one
         # against 8 TB/s, but the step runs out of VALU issue slots first)
@@ -196,11 +199,6 @@ def bench_single(args, key):
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline(w, phi)
     return out
-
-
-def sim_tile_shape(precision, index):
-    from activemodelbplus.integrator import tile_shapes
-    return tile_shapes(precision)[index]
 
 
 def bench_batched(args):

@@ -133,6 +133,11 @@ int amb_run_timed(amb_handle* h, int64_t nsteps, double* device_ms);
 int amb_tile_count(int precision, int* count);
 int amb_tile_shape(int precision, int index, int* tile_cols, int* tile_rows, int* threads);
 int amb_set_tile(amb_handle* h, int index);
+/* What the handle's next step runs in (outputs nullable): the tile shape that was
+ * chosen or that the library chooses, or with strips = 1 the columns of a strip and the
+ * rows of its segments.  (amb_get_options names the occupancy rule's tile where none was
+ * chosen; choosing that index is choosing that shape.) */
+int amb_get_step_shape(const amb_handle* h, int* cols, int* rows, int* threads, int* strips);
 
 /* Autotuner for one field: times `reps` steps of every compiled tile shape, and of
  * strips where the field runs in them without a choice, on a copy of the current

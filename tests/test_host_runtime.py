@@ -222,3 +222,52 @@ amb.tuning_set(*key, 1)
 print(json.dumps(out + [ran(make()) == shapes[1]]))
 """)
     assert out == [True] * len(out)
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_step_shape_names_what_runs(on_stub, precision):
+    """At every size of the library's choice, with a chosen tile, and with an explicit noise buffer
+    (which strips do not take)."""
+    out = on_stub(LARGE.format(shape=(64, 64), precision=precision, T=0.05) + """
+import math
+out, seen = [], set()
+for shape, T in [((64, 64), 0.0), ((256, 256), 0.05), ((512, 512), 0.0), ((704, 704), 0.05), ((1088, 1090), 0.0),
+                 ((1088, 1088), 0.05), ((2050, 2049), 0.05), ((2304, 2304), 0.0)]:
+    for tile in (0, 1, 3):
+        sim = amb.Integrator(np.zeros(shape), stencil, model(T), seed=1, precision=precision, tile=tile)
+        for noise in (False, True):
+            if noise:
+                sim.set_noise(np.zeros((1, 2) + shape))
+            cols, rows, threads, strips = sim.step_shape
+            seen.add("strips" if strips else (cols, rows, threads))
+            stub.stub_clear()
+            sim.run(1)
+            ((name, blocks, nt, _),) = [l for l in launches() if "step_kernel" in l[0] or "march_kernel" in l[0]]
+            work = math.ceil(shape[0] / rows) * math.ceil(shape[1] / cols)
+            out.append(strips == ("march" in name) and nt == threads and work <= blocks)
+            out.append(strips or f"Li{cols}ELi{rows}ELi{threads}E" in name)
+            out.append(not (strips and (noise or tile)))
+print(json.dumps([out, "strips" in seen, (32, 16, 512) in seen, (32, 32, 512) in seen]))
+""")
+    assert out == [[True] * len(out[0]), True, True, True]
+
+
+def test_bench_reads_the_profile_of_what_runs(on_stub):
+    """The benchmark's traffic and instruction counts are those of the default run's strips, and a
+    chosen shape does not get them."""
+    out = on_stub(f"""
+sys.path.insert(0, {REPO!r})
+import bench
+out = []
+for key in ("c3", "c3x8192"):
+    w = bench.WORKLOADS[key]
+    make = lambda tile: amb.Integrator(np.zeros((w["n"], w["n"])), amb.Stencil(*w["stencil"]), amb.Model(*w["model"]),
+                                       precision=w["precision"], tile=tile)
+    run, chosen = make(0).step_shape[:3], make(10).step_shape[:3]
+    out.append(bench.read_traffic(bench.TRAFFIC_PROFILE[key], run) > 8 * w["n"] ** 2)
+    out.append(bench.read_traffic(bench.TRAFFIC_PROFILE[key], chosen) is None)
+    if key in bench.VALU_PROFILE:
+        out.append(bench.read_valu(bench.VALU_PROFILE[key], run) > 0)
+print(json.dumps(out))
+""")
+    assert out == [True] * 5
