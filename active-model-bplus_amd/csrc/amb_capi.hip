@@ -819,6 +819,7 @@ int amb_get_observable_parts(amb_handle* h, int which, double* out, double* seco
     clear_error();
     if (!h || !out) return fail(AMB_E_ARG, "handle and out must not be null");
     if (which < AMB_OBS_MU || which > AMB_OBS_J_RANDOM) return fail(AMB_E_ARG, "unknown observable");
+    if (which > AMB_OBS_MU_ACTIVE && !second) return fail(AMB_E_ARG, "a current needs both components' arrays");
     const std::lock_guard<std::mutex> turn(h->stage.turn);  // d_obs too is one for all getters
     const int rc = compute_observable(h, which);
     if (rc != AMB_OK) return rc;

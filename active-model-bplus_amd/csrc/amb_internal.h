@@ -25,9 +25,6 @@ void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, int
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);
 
-// amb_get_observable with a current's x component to `second`, not after the y component.
-extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
-
 // Two pinned pieces through which results go to the caller's memory, made on first use.  Getters
 // of one handle may be called from several threads: each holds `turn` until its result is out.
 struct HostStage {

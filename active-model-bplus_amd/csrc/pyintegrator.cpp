@@ -19,9 +19,6 @@
 
 #include "amb.h"
 
-// libamb.so: amb_get_observable with a current's two components to separate arrays.
-extern "C" int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
-
 namespace py = pybind11;
 
 namespace {

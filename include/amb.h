@@ -95,6 +95,9 @@ int amb_get_field(amb_handle* h, double* out);
 #define AMB_OBS_J_CIRCULATING 8      /* get_circulating_current */
 #define AMB_OBS_J_RANDOM 9           /* get_random_current */
 int amb_get_observable(amb_handle* h, int which, double* out);
+/* The same with a current's component x to `second` (ny*nx doubles) instead of after
+ * component y; scalars leave `second` alone, and it may then be NULL. */
+int amb_get_observable_parts(amb_handle* h, int which, double* out, double* second);
 
 /* Replaces the current field (ny*nx doubles); the step counter is unchanged.  No
  * reference counterpart (the reference can only construct a new Integrator). */

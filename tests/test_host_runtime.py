@@ -271,3 +271,23 @@ for key in ("c3", "c3x8192"):
 print(json.dumps(out))
 """)
     assert out == [True] * 5
+
+
+def test_observable_parts_is_public_and_checked(on_stub):
+    """Every amb_ function that the Python module calls is declared in amb.h alone, and a current without a
+    place for its second component is refused."""
+    csrc = os.path.join(REPO, "active-model-bplus_amd", "csrc")
+    assert 'extern "C"' not in open(os.path.join(csrc, "pyintegrator.cpp")).read()
+    assert "amb_get_observable_parts(" in open(os.path.join(REPO, "include", "amb.h")).read()
+    out = on_stub("""
+lib = ctypes.CDLL(sys.argv[2] + "/lib/libamb.so")
+ptr = lambda a: ctypes.c_void_p(a.ctypes.data)
+phi, h = np.zeros((8, 8)), ctypes.c_void_p()
+three, seven = (ctypes.c_double * 3)(5e-3, 1, 1), (ctypes.c_double * 7)(-0.25, 0, 0.25, 1, 0.5, -1, 0.05)
+assert lib.amb_create(ptr(phi), ctypes.c_int64(8), ctypes.c_int64(8), three, seven, None, ctypes.byref(h)) == 0
+y, x = np.ones((8, 8)), np.ones((8, 8))
+rc = [lib.amb_get_observable_parts(h, 3, ptr(y), None), lib.amb_get_observable_parts(h, 0, ptr(y), None),
+      lib.amb_get_observable_parts(h, 3, ptr(y), ptr(x))]
+print(json.dumps(rc))
+""")
+    assert out == [1, 0, 0]
