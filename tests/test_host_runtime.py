@@ -291,3 +291,15 @@ rc = [lib.amb_get_observable_parts(h, 3, ptr(y), None), lib.amb_get_observable_p
 print(json.dumps(rc))
 """)
     assert out == [1, 0, 0]
+
+
+def test_strip_tests_run_in_strips(on_stub):
+    """Every grid of test_strips_equal_tiles and the finite check beside it takes strips on a device of 256
+    compute units, with room to the rule's line or not."""
+    import test_gpu_step_paths as paths
+    (cases,) = [m.args[1] for m in paths.test_strips_equal_tiles.pytestmark if m.name == "parametrize"]
+    out = on_stub(f"""
+cases = {list(cases) + [(32, (2048, 2050), 0.0)]!r}
+print(json.dumps([amb.Integrator(np.zeros(s), stencil, model(T), precision=p).step_shape[3] for p, s, T in cases]))
+""")
+    assert len(out) >= 9 and all(out)
