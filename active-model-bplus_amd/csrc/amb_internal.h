@@ -25,6 +25,7 @@ void record_tile(int precision, int64_t ny, int64_t nx, int noise, int tile, int
 template <typename T>
 StepCoef<T> make_coef(const amb_stencil& st, const amb_model& m);
 
+constexpr int64_t kStageDoubles = (int64_t)1 << 17;  // of a piece
 // Two pinned pieces through which results go to the caller's memory, made on first use.  Getters
 // of one handle may be called from several threads: each holds `turn` until its result is out.
 struct HostStage {

@@ -109,6 +109,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n);
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { note(1); std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyWithStream(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
 hipError_t hipGetSymbolAddress(void** p, const void* symbol)
 {
     void*& m = g_symbols[symbol];

@@ -303,3 +303,33 @@ cases = {list(cases) + [(32, (2048, 2050), 0.0)]!r}
 print(json.dumps([amb.Integrator(np.zeros(s), stencil, model(T), precision=p).step_shape[3] for p, s, T in cases]))
 """)
     assert len(out) >= 9 and all(out)
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_a_small_currents_components_come_in_one_copy(on_stub, precision):
+    """To separate arrays (Python's getters) up to 16384 sites, to one array (the C ABI's) at any size
+    of one staging piece; the values are the device's."""
+    out = on_stub(f"""
+lib = ctypes.CDLL(sys.argv[2] + "/lib/libamb.so")
+ptr = lambda a: ctypes.c_void_p(a.ctypes.data)
+three, seven = (ctypes.c_double * 3)(5e-3, 1, 1), (ctypes.c_double * 7)(-0.25, 0, 0.25, 1, 0.5, -1, 0.05)
+class Options(ctypes.Structure):
+    _fields_ = [("precision", ctypes.c_int), ("seed", ctypes.c_uint64), ("timestep", ctypes.c_int64), ("tile", ctypes.c_int)]
+def copies():
+    buf = (ctypes.c_ulong * 1000)()
+    k = stub.stub_order(buf, 1000)
+    stub.stub_clear()
+    return sum(x & 1 for x in buf[:k])
+out = []
+for ny, nx in ((8, 9), (128, 128), (128, 129), (256, 256)):
+    phi, h, opt = np.zeros((ny, nx)), ctypes.c_void_p(), Options({precision}, 1, 0, 0)
+    assert lib.amb_create(ptr(phi), ctypes.c_int64(ny), ctypes.c_int64(nx), three, seven, ctypes.byref(opt), ctypes.byref(h)) == 0
+    y, x, both = np.ones((ny, nx)), np.ones((ny, nx)), np.ones((2, ny, nx))
+    copies()
+    lib.amb_get_observable_parts(h, 3, ptr(y), ptr(x))
+    apart = copies()
+    lib.amb_get_observable(h, 3, ptr(both))
+    out.append([apart, copies(), bool((y == 0).all() and (x == 0).all() and (both == 0).all())])
+print(json.dumps(out))
+""")
+    assert out == [[1, 1, True], [1, 1, True], [2, 1, True], [2, 1, True]]
