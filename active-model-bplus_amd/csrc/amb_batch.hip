@@ -71,11 +71,14 @@ __global__ __launch_bounds__(NT, (step_waves_per_eu<T, TW, TH, NT, NOISE>())) vo
 // count, reduced in a fixed order) at part[slot].
 //
 // A step of a lone workgroup is a chain of phases and barriers, so its time goes with the
-// number of tiles: members up to 64x64 (FP32) or 48x44 (FP64) that need several 256-thread
+// number of tiles: members up to 64x64 (FP32) or, of 48 rows and 44 columns at most, as many
+// FP64 sites as the LDS holds beside the tile (44x44, not 48x44), that need several 256-thread
 // tiles take the whole member as one tile of 1024 or 704 threads, which nearly fills a CU's LDS.
 // A 64x64 FP32 member takes 6.2 us a step at T = 0 and 8.2 us with noise, against 15.5 and
 // 21.7 us in four 32x32 tiles (and 5.5 and 6.5 us as a launch of tiles per step, alone on the
-// device); a 40x40 FP64 member 6.9 and 9.7 us against 20.2 and 30.4 us.
+// device); a 40x40 FP64 member 6.9 and 9.7 us against 20.2 and 30.4 us.  Members that fill the
+// device gain too, though a CU then holds one instead of three: 768 of 40x40 FP32 16.4 us against
+// 19.6 in small tiles (noisy 21.8, 26.8), 2048 of them 42.1 and 53.1 (56.6, 74.2).
 constexpr size_t kResidentLds = 80 * 1024;       // two field buffers and one small tile's scratch
 constexpr size_t kResidentWholeLds = 160 * 1024; // the same with the whole member's scratch
 

@@ -198,8 +198,8 @@ void release(HostStage& st)
 int grid_tiles(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
 // The occupancy rule's tile, which options report when none was chosen (such a field runs in
-// run_tile's) and whose tiles bound amb_run_noalloc's fields: in order of preference (AMB_F32_NOISY_ORDER, AMB_F32_NOISELESS_ORDER or
-// AMB_F64_ORDER), the first shape of 256 or more threads whose tiles fill the device's
+// run_tile's; amb_get_step_shape tells) and whose tiles bound amb_run_noalloc's fields: in order of
+// preference (AMB_F32_NOISY_ORDER, AMB_F32_NOISELESS_ORDER or AMB_F64_ORDER), the first shape of 256 or more threads whose tiles fill the device's
 // resident workgroups either for at least 8 rounds or in whole-or-mostly-full rounds (a
 // last round under half full leaves most CUs idle for a round).  Fields too small for one
 // round of such a shape take the shape that puts nearest 8 waves on each CU (in ratio; the
@@ -207,8 +207,9 @@ int grid_tiles(int64_t n, int t) { return (int)((n + t - 1) / t); }
 // hide, while many small tiles pay their halo several times over.  The tiles of 64 and 128
 // threads only serve that way: their boxes hold 4.5-10.6x their area of phi (32x32 tiles
 // 2.4x), so where they fill a round (FP64 16x8 at 512^2) a half round of 32x32 tiles is
-// still faster (9.0 against 10.2 us).  Measured from 128^2 to 4096^2 in both precisions, with and without noise, this
-// picks the fastest shape or one within 2% of it.
+// still faster (9.0 against 10.2 us).  It picked the fastest of the shapes it lists, or one within
+// 2% of it, before the tiles were handed to the XCDs in runs; run_tile's are up to 1.4 times as
+// fast now (its table).
 int default_tile(int precision, int64_t ny, int64_t nx, int noise)
 {
     int device = 0, cus = 256;

@@ -50,8 +50,9 @@ struct TileShape {
     int tw, th, nt;  // tile columns, tile rows, workgroup size
 };
 
-// Compiled tile configurations (index = autotuner choice): X(index, TW, TH, NT).  The
-// default tile follows an order of preference per kernel (default_tile in amb_capi.hip).
+// Compiled tile configurations (index = autotuner choice): X(index, TW, TH, NT).  A field
+// without a chosen one runs in run_tile's; options name the occupancy rule's, which follows an
+// order of preference per kernel (default_tile in amb_capi.hip).
 #define AMB_F32_TILES(X) X(0, 32, 48, 512) X(1, 32, 24, 256) X(2, 32, 32, 256) X(3, 64, 32, 512) X(4, 64, 16, 256) X(5, 32, 16, 256) X(6, 16, 16, 128) X(7, 16, 8, 128) X(8, 8, 8, 64) X(9, 32, 32, 512) X(10, 32, 16, 512)
 #define AMB_F64_TILES(X) X(0, 32, 32, 256) X(1, 64, 16, 256) X(2, 32, 16, 256) X(3, 32, 32, 512) X(4, 16, 16, 128) X(5, 16, 8, 128) X(6, 8, 8, 64) X(7, 32, 16, 512)
 constexpr int kSquare512F32 = 9, kSquare512F64 = 3;  // 32x32 tiles of 512 threads
@@ -114,6 +115,9 @@ int device_cus();  // compute units of the current device
 // no multiple of eight used to leave in plain order, 8.7).  Fields of few tiles keep to as few
 // XCDs as hold them one to a compute unit: 128^2 FP32 T = 0.05 in 32 tiles 4.9 us on one XCD, 5.3
 // on two, 5.5 on eight; FP64 6.4, 6.8, 7.1; from 3/8 of the device on all eight are as fast.
+// Several such fields at once share the first XCD and still gain: 128^2 FP64 on 1, 2, 4 and 8 threads
+// 6.4, 6.4, 12.9 and 19.5 us a step of all of them, spread over the XCDs in larger tiles 7.4, 7.5,
+// 15.2 and 23.9; in four processes 6.4 to 7.1 us against 8.6 where each has a hardware queue.
 inline int xcd_chunk(int64_t tiles)
 {
     const int64_t cus = device_cus();

@@ -10,10 +10,11 @@
 // master weights and Adam moments in one flat vector, tap = 3(dy+1) + (dx+1)
 // reading in[y+dy][x+dx] with periodic wrap.
 //
-// Convolution as implicit GEMM: M = pixels, N = output channels, K = taps x cin.
-// Each wave owns MB x NB tiles of 16 x 16 outputs; per K-step of 32 a lane loads one
-// 16-byte chunk (8 channels of one tap) per A tile and per B tile straight from
-// global memory (L1/L2 resident) into the MFMA operand layout:
+// Convolution as implicit GEMM: M = pixels, N = output channels, K = taps x cin in steps of
+// 32, tiles of 16 x 16 outputs.  A block stages its padded input tile in LDS once for all
+// taps; training (conv_kernel) keeps the weights in registers, as the left operand, inference
+// (conv_tile_kernel, c12_kernel, c7_head_flux_kernel) fetches them as they are needed.
+// Operands, 16 bytes (8 channels of one tap) a lane:
 //   A: lane l holds A[l%16][8(l/16) .. +7];  B: B[8(l/16) .. +7][l%16];
 //   D: lane l holds D[4(l/16) + r][l%16], r = 0..3.
 #include <hip/hip_runtime.h>
@@ -88,7 +89,8 @@ __device__ __forceinline__ float hi_f(uint32_t w) { return __uint_as_float(w & 0
 // Order of a kernel's tiles: gfx950 dispatches block b to XCD b % 8, so each XCD takes a
 // contiguous run of the row-major tiles.  Halos then come from the XCD's own L2, and the
 // kernels of a network pass, whose runs cover the same rows at every level, find there what
-// the one before wrote: 256^2 inference 41.4 -> 38.9 us a step.  (All grids are multiples of 8 blocks: sides are multiples of 64.)
+// the one before wrote: 256^2 inference 41.4 -> 38.9 us a step.  (Grids that are not multiples of 8 blocks, those of the lowest level of a
+// single 64 x 64 sample, keep the plain order.)
 __device__ __forceinline__ int xcd_run()
 {
     const int n = gridDim.x;

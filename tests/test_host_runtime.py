@@ -294,8 +294,8 @@ print(json.dumps(rc))
 
 
 def test_strip_tests_run_in_strips(on_stub):
-    """Every grid of test_strips_equal_tiles and the finite check beside it takes strips on a device of 256
-    compute units, with room to the rule's line or not."""
+    """Every grid of test_strips_equal_tiles and of the finite check beside it takes strips on a device of
+    256 compute units."""
     import test_gpu_step_paths as paths
     (cases,) = [m.args[1] for m in paths.test_strips_equal_tiles.pytestmark if m.name == "parametrize"]
     out = on_stub(f"""
